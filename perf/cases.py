@@ -412,6 +412,7 @@ def run(s):
         rc = solver.lib.mpm_surrogate_gradient_noalloc(solver.h, s.pairs.data_ptr(), s.H.data_ptr(), case["rows"],
                                                        s.grad.data_ptr(), s.loss.data_ptr())
         _check(solver, rc, "mpm_surrogate_gradient_noalloc")
+        solver.synchronize()  # the gradient is ready for the caller's own stream from here on
         return dict(grad=s.grad, loss=s.loss)
     losses = solver.surrogate_train(s.pairs, s.H, epochs=1, batch=case["batch"], lr=1e-3, seed=5)
     return dict(losses=losses, weights=solver.surrogate_get_weights())
