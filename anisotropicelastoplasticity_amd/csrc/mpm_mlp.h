@@ -67,15 +67,13 @@ size_t mlp_forward_smem();
 size_t mlp_backward_smem();
 void mlp_set_smem_limits();
 void launch_mlp_forward(hipStream_t s, const uint16_t* wbf, const float* master, const float* in, float* out, int n,
-                        float* zsave, int grid);
-void launch_mlp_backward(hipStream_t s, const uint16_t* wbft, const float* in, const float* y, const float* target,
+                        float* zsave, int n_cu);
+void launch_mlp_backward(hipStream_t s, const uint16_t* wbft, const float* in, const float* y, const float* H,
                          const float* zsave, int n, float* grad_part, float* loss, int grid);
 void launch_mlp_reduce(hipStream_t s, const float* part, int nparts, float* grad, const float* loss_part,
-                       float* loss_acc);
-void launch_mlp_adam(hipStream_t s, float* master, float* m1, float* m2, const float* grad, uint16_t* wbf,
-                     uint16_t* wbft, float lr, int step);
+                       float* loss_acc, float* loss_mean, int n);
+void launch_mlp_reduce_adam(hipStream_t s, const float* part, int nparts, const float* loss_part, float* loss_acc,
+                            float* master, float* m1, float* m2, uint16_t* wbf, uint16_t* wbft, float lr, int step);
 void launch_mlp_to_bf16(hipStream_t s, const float* master, uint16_t* wbf, uint16_t* wbft);
-void launch_mlp_targets(hipStream_t s, const float* in, const float* H, int n, float* tgt);
-void launch_mlp_loss_mean(hipStream_t s, const float* loss_part, int nparts, int n, float* loss);
 
 }  // namespace mpm

@@ -75,23 +75,6 @@ static __device__ void stage_weights(MLPShared& s, const uint16_t* __restrict__ 
   for (int i = threadIdx.x; i < MLP_OUT_PAD; i += blockDim.x) s.b[4 * MLP_HIDDEN + i] = master[mlp_bias_offset(4) + i];
 }
 
-// acc[t] (16 rows x 16 cols of output tile t) += A (16 x 32*KS, row stride lda) * W^T where W is
-// [16*NT][32*KS] with row stride ldw: every operand is 8 contiguous bf16 per lane (backward pass).
-template <int NT, int KS>
-__device__ __forceinline__ void wave_gemm_nt(const uint16_t* A, int lda, const uint16_t* W, int ldw, f32x4* acc) {
-  const int lane = threadIdx.x & 63;
-  const int r = lane & 15, kq = (lane >> 4) * 8;
-#pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    const bf16x8 a = *reinterpret_cast<const bf16x8*>(A + r * lda + 32 * s + kq);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const bf16x8 b = *reinterpret_cast<const bf16x8*>(W + (16 * t + r) * ldw + 32 * s + kq);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
-    }
-  }
-}
-
 // One step of the layer pipeline over NT sample tiles (tiles T0 .. T0 + NT - 1 of the wave). Unit u
 // of a layer is its output feature tiles 2u and 2u + 1 (the next layer's K step u), accumulated over
 // the layer's KS K steps in ascending order into acc. The step issues those MFMAs and, between them,

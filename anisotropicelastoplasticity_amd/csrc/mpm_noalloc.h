@@ -10,10 +10,9 @@ namespace mpm {
 constexpr int NOALLOC_MAX_ROWS = 2048;
 // workgroups of its backward pass (64 rows each), each with a partial gradient
 constexpr int NOALLOC_GROUPS = (NOALLOC_MAX_ROWS + 63) / 64;
-// scratch (floats): normalised targets (3 per row), outputs (3 per row), pre-activations
-// (4 layers x 128 per row), partial gradients and losses of the backward workgroups
-constexpr size_t NOALLOC_TGT = 0;
-constexpr size_t NOALLOC_Y = NOALLOC_TGT + 3 * (size_t)NOALLOC_MAX_ROWS;
+// scratch (floats): outputs (3 per row), pre-activations (4 layers x 128 per row), partial gradients and
+// losses of the backward workgroups
+constexpr size_t NOALLOC_Y = 0;
 constexpr size_t NOALLOC_Z = NOALLOC_Y + 3 * (size_t)NOALLOC_MAX_ROWS;
 constexpr size_t NOALLOC_GPART = NOALLOC_Z + 4 * (size_t)MLP_HIDDEN * NOALLOC_MAX_ROWS;
 constexpr size_t NOALLOC_LPART = NOALLOC_GPART + (size_t)NOALLOC_GROUPS * MLP_NPARAM;

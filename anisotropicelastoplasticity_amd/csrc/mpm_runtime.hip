@@ -1924,19 +1924,6 @@ int mpm_surrogate_get_weights(mpm_ctx* ctx, float* w, int32_t nparam) {
   return MPM_OK;
 }
 
-// normalised targets y = (H - eps) / CORR_SCALE
-static void targets_of(const float* in, const float* H, int64_t n, std::vector<float>& y) {
-  y.resize((size_t)3 * n);
-  for (int64_t r = 0; r < n; ++r)
-    for (int c = 0; c < 3; ++c) y[3 * r + c] = (H[3 * r + c] - in[5 * r + c]) / MLP_CORR_SCALE;
-}
-
-// workgroups of the forward kernels: one per CU at most (each stages the weights once and its 8
-// waves take 64 rows at a time)
-static int forward_grid(const mpm_ctx* ctx, int64_t rows) {
-  return (int)std::max<int64_t>(1, std::min<int64_t>(ctx->n_cu, (rows + MLP_FWD_THREADS - 1) / MLP_FWD_THREADS));
-}
-
 int mpm_surrogate_predict(mpm_ctx* ctx, const float* in, float* H, int32_t n) {
   if (!ctx || !in || !H || n < 0) return MPM_ERR_INVALID;
   if (!ctx->mlp_ready) return fail(ctx, MPM_ERR_STATE, "surrogate weights not set");
@@ -1948,7 +1935,7 @@ int mpm_surrogate_predict(mpm_ctx* ctx, const float* in, float* H, int32_t n) {
   if (rc) { dfree(din); dfree(dout); return rc; }
   hipError_t e = hipMemcpyAsync(din, in, sizeof(float) * 5 * n, hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess) {
-    launch_mlp_forward(ctx->stream, ctx->mlp_wbf, ctx->mlp_master, din, dout, n, nullptr, forward_grid(ctx, n));
+    launch_mlp_forward(ctx->stream, ctx->mlp_wbf, ctx->mlp_master, din, dout, n, nullptr, ctx->n_cu);
     e = hipMemcpyAsync(H, dout, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, ctx->stream);
   }
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
@@ -1963,7 +1950,7 @@ int mpm_surrogate_predict(mpm_ctx* ctx, const float* in, float* H, int32_t n) {
 // one optimisation pass machinery: forward (saving pre-activations), backward, ordered reduction
 struct TrainBufs {
   float* in = nullptr;
-  float* tgt = nullptr;
+  float* H = nullptr;
   float* y = nullptr;
   float* z = nullptr;
   float* gpart = nullptr;
@@ -1972,7 +1959,7 @@ struct TrainBufs {
 };
 
 static void free_train(TrainBufs& b) {
-  dfree(b.in); dfree(b.tgt); dfree(b.y); dfree(b.z); dfree(b.gpart); dfree(b.lpart); dfree(b.lacc);
+  dfree(b.in); dfree(b.H); dfree(b.y); dfree(b.z); dfree(b.gpart); dfree(b.lpart); dfree(b.lacc);
 }
 
 // workgroups of the backward pass (each owns a partial-gradient slice of MLP_NPARAM floats)
@@ -1981,7 +1968,7 @@ static int backward_grid(int rows) { return std::min((rows + 63) / 64, 1024); }
 static int alloc_train(mpm_ctx* ctx, TrainBufs& b, int64_t n, int batch, int nacc) {
   const int groups = backward_grid(batch);
   int rc = dalloc(ctx, b.in, (size_t)5 * n);
-  if (!rc) rc = dalloc(ctx, b.tgt, (size_t)3 * n);
+  if (!rc) rc = dalloc(ctx, b.H, (size_t)3 * n);
   if (!rc) rc = dalloc(ctx, b.y, (size_t)3 * batch);
   if (!rc) rc = dalloc(ctx, b.z, (size_t)((batch + 15) / 16) * 4 * 16 * MLP_HIDDEN);
   if (!rc) rc = dalloc(ctx, b.gpart, (size_t)groups * MLP_NPARAM);
@@ -1990,11 +1977,12 @@ static int alloc_train(mpm_ctx* ctx, TrainBufs& b, int64_t n, int batch, int nac
   return rc;
 }
 
-static void train_batch(mpm_ctx* ctx, TrainBufs& b, int64_t r0, int nb, float* lacc) {
+// The partial gradients and losses of rows [r0, r0 + nb): one pair per workgroup; returns their number.
+static int batch_gradients(mpm_ctx* ctx, TrainBufs& b, int64_t r0, int nb) {
   const int groups = backward_grid(nb);
-  launch_mlp_forward(ctx->stream, ctx->mlp_wbf, ctx->mlp_master, b.in + 5 * r0, b.y, nb, b.z, forward_grid(ctx, nb));
-  launch_mlp_backward(ctx->stream, ctx->mlp_wbft, b.in + 5 * r0, b.y, b.tgt + 3 * r0, b.z, nb, b.gpart, b.lpart, groups);
-  launch_mlp_reduce(ctx->stream, b.gpart, groups, ctx->mlp_grad, b.lpart, lacc);
+  launch_mlp_forward(ctx->stream, ctx->mlp_wbf, ctx->mlp_master, b.in + 5 * r0, b.y, nb, b.z, ctx->n_cu);
+  launch_mlp_backward(ctx->stream, ctx->mlp_wbft, b.in + 5 * r0, b.y, b.H + 3 * r0, b.z, nb, b.gpart, b.lpart, groups);
+  return groups;
 }
 
 int mpm_surrogate_gradient(mpm_ctx* ctx, const float* in, const float* H, int32_t n, float* grad, float* loss) {
@@ -2004,13 +1992,12 @@ int mpm_surrogate_gradient(mpm_ctx* ctx, const float* in, const float* H, int32_
   TrainBufs b;
   int rc = alloc_train(ctx, b, n, n, 1);
   if (rc) { free_train(b); return rc; }
-  std::vector<float> y;
-  targets_of(in, H, n, y);
   hipError_t e = hipMemcpyAsync(b.in, in, sizeof(float) * 5 * n, hipMemcpyHostToDevice, ctx->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(b.tgt, y.data(), sizeof(float) * 3 * n, hipMemcpyHostToDevice, ctx->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(b.H, H, sizeof(float) * 3 * n, hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess) e = hipMemsetAsync(b.lacc, 0, sizeof(float), ctx->stream);
   if (e == hipSuccess) {
-    train_batch(ctx, b, 0, n, b.lacc);
+    const int groups = batch_gradients(ctx, b, 0, n);
+    launch_mlp_reduce(ctx->stream, b.gpart, groups, ctx->mlp_grad, b.lpart, b.lacc, nullptr, n);
     e = hipGetLastError();
   }
   float lsum = 0.0f;
@@ -2036,12 +2023,10 @@ int mpm_surrogate_gradient_noalloc(mpm_ctx* ctx, const float* in, const float* H
   // reads (rows < n, the first `groups` partials) is written earlier in the same call
   float* s = ctx->scratch;
   const int groups = backward_grid(n);
-  launch_mlp_targets(ctx->stream, in, H, n, s + NOALLOC_TGT);
-  launch_mlp_forward(ctx->stream, ctx->mlp_wbf, ctx->mlp_master, in, s + NOALLOC_Y, n, s + NOALLOC_Z, forward_grid(ctx, n));
-  launch_mlp_backward(ctx->stream, ctx->mlp_wbft, in, s + NOALLOC_Y, s + NOALLOC_TGT, s + NOALLOC_Z, n, s + NOALLOC_GPART,
+  launch_mlp_forward(ctx->stream, ctx->mlp_wbf, ctx->mlp_master, in, s + NOALLOC_Y, n, s + NOALLOC_Z, ctx->n_cu);
+  launch_mlp_backward(ctx->stream, ctx->mlp_wbft, in, s + NOALLOC_Y, H, s + NOALLOC_Z, n, s + NOALLOC_GPART,
                       s + NOALLOC_LPART, groups);
-  launch_mlp_reduce(ctx->stream, s + NOALLOC_GPART, groups, grad, s + NOALLOC_LPART, nullptr);
-  launch_mlp_loss_mean(ctx->stream, s + NOALLOC_LPART, groups, n, loss);
+  launch_mlp_reduce(ctx->stream, s + NOALLOC_GPART, groups, grad, s + NOALLOC_LPART, nullptr, loss, n);
   CK(hipGetLastError());
   return MPM_OK;
 }
@@ -2063,25 +2048,24 @@ int mpm_surrogate_train(mpm_ctx* ctx, const float* in, const float* H, int32_t n
     const int j = (int)(mix64(seed ^ (0xD1B54A32D192ED03ull * (uint64_t)(i + 1))) % (uint64_t)(i + 1));
     std::swap(order[i], order[j]);
   }
-  std::vector<float> ins((size_t)5 * n), hs((size_t)3 * n), y;
+  std::vector<float> ins((size_t)5 * n), hs((size_t)3 * n);
   for (int r = 0; r < n; ++r) {
     for (int c = 0; c < 5; ++c) ins[5 * (size_t)r + c] = in[5 * (size_t)order[r] + c];
     for (int c = 0; c < 3; ++c) hs[3 * (size_t)r + c] = H[3 * (size_t)order[r] + c];
   }
-  targets_of(ins.data(), hs.data(), n, y);
   if (batch > n) batch = n;
   TrainBufs b;
   rc = alloc_train(ctx, b, n, batch, epochs);
   if (rc) { free_train(b); return rc; }
   hipError_t e = hipMemcpyAsync(b.in, ins.data(), sizeof(float) * 5 * n, hipMemcpyHostToDevice, ctx->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(b.tgt, y.data(), sizeof(float) * 3 * n, hipMemcpyHostToDevice, ctx->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(b.H, hs.data(), sizeof(float) * 3 * n, hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess) e = hipMemsetAsync(b.lacc, 0, sizeof(float) * epochs, ctx->stream);
   for (int ep = 0; ep < epochs && e == hipSuccess; ++ep) {
     for (int64_t r0 = 0; r0 < n; r0 += batch) {
       const int nb = (int)std::min<int64_t>(batch, n - r0);
-      train_batch(ctx, b, r0, nb, b.lacc + ep);
-      launch_mlp_adam(ctx->stream, ctx->mlp_master, ctx->mlp_m1, ctx->mlp_m2, ctx->mlp_grad, ctx->mlp_wbf, ctx->mlp_wbft,
-                      lr, ++ctx->mlp_step);
+      const int groups = batch_gradients(ctx, b, r0, nb);
+      launch_mlp_reduce_adam(ctx->stream, b.gpart, groups, b.lpart, b.lacc + ep, ctx->mlp_master, ctx->mlp_m1,
+                             ctx->mlp_m2, ctx->mlp_wbf, ctx->mlp_wbft, lr, ++ctx->mlp_step);
     }
     e = hipGetLastError();
   }
