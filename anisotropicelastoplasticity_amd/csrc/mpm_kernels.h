@@ -174,7 +174,8 @@ struct P2GArgs {
   const int* counters;
   const int* active_tiles;
   float* partials;
-  const float4* gvel;  // node velocities (force pass)
+  const float4* gvel;  // node velocities (k_stress_predicted)
+  float* stress;       // 9 planes of `cap`: the predicted stress matrix at each sorted position (force pass)
   float dt;
   unsigned long long* fallback_svd;
   const Clock* clk;
@@ -317,6 +318,7 @@ void launch_count_nodes(hipStream_t s, const SceneTable& T, const float* gm, con
 void launch_fill_int(hipStream_t s, int* p, int64_t n, int v);
 void launch_copy(hipStream_t s, const float4* src, float4* dst, int64_t n4);
 // Dt from the max node speed (init: the first Dt, no frame bookkeeping), then the frame clamp.
+void launch_stress_predicted(hipStream_t s, const P2GArgs& a, int order, int nblocks);
 void launch_clock_update(hipStream_t s, Clock* c, int init);
 // End of a substep: count it, close a completed frame, stop the batch after a frame or the run.
 void launch_clock_end(hipStream_t s, Clock* c);

@@ -808,10 +808,10 @@ __device__ __forceinline__ P2GScene p2g_scene(const DevParams& P) {
 }
 
 // Particle data a staging lane needs, loaded one chunk ahead of its use (the loads of the next
-// chunk are in flight while the wave accumulates the current one). The force pass of the
-// predicted-stress mode loads inside p2g_stage instead.
+// chunk are in flight while the wave accumulates the current one). In the force pass of the
+// predicted-stress mode B holds the stress matrix that k_stress_predicted left at the sorted position.
 struct StageIn {
-  int pi, pid;  // pid: the particle's id when the scene has a cloth mesh (else -1)
+  int pid;  // the particle's id when the scene has a cloth mesh (else that of slot 0)
   float x[3], m, v[3], B[9], K[6];
 };
 
@@ -820,11 +820,10 @@ struct StageIn {
 __device__ __forceinline__ int p2g_slot(const P2GArgs& a, int idx) { return a.src[idx]; }
 
 template <int MODE>
-__device__ __forceinline__ void p2g_load_at(const P2GArgs& a, const P2GScene& S, int slot, StageIn& in) {
+__device__ __forceinline__ void p2g_load_at(const P2GArgs& a, const P2GScene& S, int slot, int idx, StageIn& in) {
   const int pi = clamp_index(slot, a.n);
   const float* st = a.state;
   const int64_t cap = a.cap;
-  in.pi = pi;
   // a scene without a mesh loads word 0 of the id plane in every lane (one cache line) instead of a
   // branch around the load: a branch here makes the wave wait for this chunk's loads before the
   // accumulation of the previous one
@@ -837,6 +836,9 @@ __device__ __forceinline__ void p2g_load_at(const P2GArgs& a, const P2GScene& S,
     for (int d = 0; d < 3; ++d) in.v[d] = st[(PV + d) * cap + pi];
 #pragma unroll
     for (int i = 0; i < 9; ++i) in.B[i] = st[(PB + i) * cap + pi];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 9; ++i) in.B[i] = a.stress[i * cap + idx];
   }
   if constexpr (MODE == P2G_MOM_STRESS) {
 #pragma unroll
@@ -846,12 +848,12 @@ __device__ __forceinline__ void p2g_load_at(const P2GArgs& a, const P2GScene& S,
 
 template <int MODE>
 __device__ __forceinline__ void p2g_load(const P2GArgs& a, const P2GScene& S, int idx, StageIn& in) {
-  p2g_load_at<MODE>(a, S, p2g_slot(a, idx), in);
+  p2g_load_at<MODE>(a, S, p2g_slot(a, idx), idx, in);
 }
 
 template <int ORDER, int MODE>
-__device__ __forceinline__ void p2g_stage(const P2GArgs& a, const P2GScene& S, const DevParams& P, int64_t noff,
-                                          float dt, const StageIn& in, int g0, int g1, int g2, float4* dst) {
+__device__ __forceinline__ void p2g_stage(const P2GArgs& a, const P2GScene& S, float dt, const StageIn& in, int g0, int g1,
+                                          int g2, float4* dst) {
   // No FMA contraction: the row and the layer pass inline this function into different kernels, and
   // the payload must have the same bits in both (contraction is decided per kernel otherwise).
 #pragma clang fp contract(off)
@@ -859,12 +861,9 @@ __device__ __forceinline__ void p2g_stage(const P2GArgs& a, const P2GScene& S, c
 #pragma unroll
   for (int i = 0; i < PAY; ++i) pay[i] = 0.0f;
   // kind of the point from its id (loaded with the rest of its data, used only here)
-  const int pi = in.pi;
   const int kind = (S.mesh_e1 <= S.mesh_v0 || in.pid < S.mesh_v0) ? KIND_PARTICLE
                                                                     : (in.pid < S.mesh_e0 ? KIND_VERTEX : KIND_ELEMENT);
   const int mid = in.pid - (kind == KIND_VERTEX ? S.mesh_v0 : S.mesh_e0);
-  const float* st = a.state;
-  const int64_t cap = a.cap;
   const int cc[3] = {g0, g1, g2};
   float f[3];
 #pragma unroll
@@ -929,49 +928,10 @@ __device__ __forceinline__ void p2g_stage(const P2GArgs& a, const P2GScene& S, c
 #pragma unroll
         for (int c = 0; c < 3; ++c) Sm[3 * r + c] = a.elem_stress[9 * mid + 3 * r + c] * S.inv_h[c];
     } else {
-      // stress matrix V P(F^) F^n^T at the predicted F^ = F + dt (sum_i v_i grad w_ip^T) F from the
-      // post-P2G grid velocity (HybridSolver.cpp:269-339)
-      float Fn[9];
-#pragma unroll
-      for (int i = 0; i < 9; ++i) Fn[i] = st[(PF + i) * cap + pi];
-      float G[9];
-#pragma unroll
-      for (int i = 0; i < 9; ++i) G[i] = 0.0f;
-      for (int oz = 0; oz < 4; ++oz) {
-        int n2 = g2 - 1 + oz;
-        if (n2 < 0 || n2 >= S.res[2]) continue;
-        for (int oy = 0; oy < 4; ++oy) {
-          int n1 = g1 - 1 + oy;
-          if (n1 < 0 || n1 >= S.res[1]) continue;
-          for (int ox = 0; ox < 4; ++ox) {
-            int n0 = g0 - 1 + ox;
-            if (n0 < 0 || n0 >= S.res[0]) continue;
-            float gw[3] = {dwx[ox] * wy[oy] * wz[oz] * S.inv_h[0], wx[ox] * dwy[oy] * wz[oz] * S.inv_h[1],
-                           wx[ox] * wy[oy] * dwz[oz] * S.inv_h[2]};
-            int64_t node = noff + ((int64_t)n2 * S.res[1] + n1) * S.res[0] + n0;
-            const float4 gv4 = a.gvel[2 * node];
-            const float vr[3] = {gv4.x, gv4.y, gv4.z};
-#pragma unroll
-            for (int r = 0; r < 3; ++r)
-#pragma unroll
-              for (int c = 0; c < 3; ++c) G[3 * r + c] += vr[r] * gw[c];
-          }
-        }
-      }
-      float GF[9], Fh[9];
-      mat_mul(G, Fn, GF);
-#pragma unroll
-      for (int i = 0; i < 9; ++i) Fh[i] = Fn[i] + dt * GF[i];
-      float Jp = st[PPL * cap + pi];
-      float vol = st[PVOL * cap + pi];
-      float Sp[9];
-      int fb = 0;
-      stress_matrix(P, Fh, Fn, Jp, vol, Sp, fb);
-      if (fb) atomicAdd(a.fallback_svd, (unsigned long long)fb);
 #pragma unroll
       for (int r = 0; r < 3; ++r)
 #pragma unroll
-        for (int c = 0; c < 3; ++c) Sm[3 * r + c] = Sp[3 * r + c] * S.inv_h[c];
+        for (int c = 0; c < 3; ++c) Sm[3 * r + c] = in.B[3 * r + c] * S.inv_h[c];
     }
   }
 #pragma unroll
@@ -986,6 +946,108 @@ __device__ __forceinline__ void p2g_stage(const P2GArgs& a, const P2GScene& S, c
     for (int r = 0; r < 3; ++r) pay[PY_G + 3 * ox + r] = (float)ox * wx[ox] * Q0[r] - dwx[ox] * S0[r];
 #pragma unroll
   for (int i = 0; i < PAY / 4; ++i) dst[i] = make_float4(pay[4 * i], pay[4 * i + 1], pay[4 * i + 2], pay[4 * i + 3]);
+}
+
+// Stress matrix V P(F^) F^n^T of every particle at the predicted F^ = F + dt (sum_i v_i grad w_ip^T) F from
+// the post-P2G grid velocity (HybridSolver.cpp:269-339), thread per sorted position j, written to
+// stress[9 planes][j] for the force pass of P2G. As G2P, the gather factors over the axes (row sums of v
+// with w and w' along x) and loads one z plane of nodes at a time.
+// The force pass used to do this inside its staging, where only the staging lanes of a wave (a quarter to a
+// half) gathered, node after node, and nothing overlapped the wait: 203 us for the force pass of 321k cubic
+// particles, now 33 us for this kernel and 35 us for the force pass (MI355X).
+template <int ORDER>
+__global__ __launch_bounds__(256) void k_stress_predicted(P2GArgs a) {
+  if (clock_skip(a.clk)) return;
+  const float dt = clock_dt(a.clk, a.dt);
+  const PBlock pb = particle_block(a.T);
+  const DevParams P = uniform_params(a.T.params[pb.s]);
+  const float4* gvel = a.gvel + 2 * a.T.node_off[pb.s];
+  const int j = pb.j;
+  int fb = 0;
+  if (j < pb.end) {
+    const float* st = a.state;
+    const int64_t cap = a.cap;
+    const int pi = clamp_index(a.src[j], a.n);
+    const int pid = reinterpret_cast<const int*>(st + (size_t)PID * cap)[P.mesh_e1 > P.mesh_v0 ? pi : 0];
+    float Fn[9], g[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) g[d] = (st[(PX + d) * cap + pi] - P.gmin[d]) * P.inv_h[d];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) Fn[i] = st[(PF + i) * cap + pi];
+    const float Jp = st[PPL * cap + pi], vol = st[PVOL * cap + pi];
+    int nid[3][ORDER + 1];
+    float w[3][4], dw[3][4];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const int base = stencil_base<ORDER>(g[d], P.res[d]);
+#pragma unroll
+      for (int o = 0; o < ORDER + 1; ++o) {
+        const int nn = base + o;
+        const bool in = nn >= 0 && nn < P.res[d];  // out-of-grid nodes: zero weight, clamped index
+        spline<ORDER>(g[d] - (float)nn, w[d][o], dw[d][o]);
+        w[d][o] = in ? w[d][o] : 0.0f;
+        dw[d][o] = in ? dw[d][o] * P.inv_h[d] : 0.0f;
+        nid[d][o] = nn < 0 ? 0 : (nn >= P.res[d] ? P.res[d] - 1 : nn);
+      }
+    }
+    const int64_t res0 = P.res[0], res01 = (int64_t)P.res[0] * P.res[1];
+    float G[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) G[i] = 0.0f;
+#pragma unroll 1
+    for (int oz = 0; oz < ORDER + 1; ++oz) {
+      float wz = w[2][0], dwz = dw[2][0];
+      int nz = nid[2][0];
+#pragma unroll
+      for (int o = 1; o < ORDER + 1; ++o) {
+        wz = oz == o ? w[2][o] : wz;
+        dwz = oz == o ? dw[2][o] : dwz;
+        nz = oz == o ? nid[2][o] : nz;
+      }
+      float4 q[ORDER + 1][ORDER + 1];
+#pragma unroll
+      for (int oy = 0; oy < ORDER + 1; ++oy) {
+        const float4* rp = gvel + 2 * (nz * res01 + nid[1][oy] * res0);
+#pragma unroll
+        for (int ox = 0; ox < ORDER + 1; ++ox) q[oy][ox] = rp[2 * nid[0][ox]];
+      }
+#pragma unroll
+      for (int oy = 0; oy < ORDER + 1; ++oy) {
+        float A[3] = {0.0f, 0.0f, 0.0f}, Ad[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int ox = 0; ox < ORDER + 1; ++ox) {
+          const float vi[3] = {q[oy][ox].x, q[oy][ox].y, q[oy][ox].z};
+#pragma unroll
+          for (int r = 0; r < 3; ++r) {
+            A[r] += w[0][ox] * vi[r];
+            Ad[r] += dw[0][ox] * vi[r];
+          }
+        }
+        const float wyz = w[1][oy] * wz, dyz = dw[1][oy] * wz, ydz = w[1][oy] * dwz;
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+          G[3 * r] += wyz * Ad[r];
+          G[3 * r + 1] += dyz * A[r];
+          G[3 * r + 2] += ydz * A[r];
+        }
+      }
+    }
+    if (particle_kind(P, pid) == KIND_PARTICLE) {
+      float GF[9], Fh[9], Sp[9];
+      mat_mul(G, Fn, GF);
+#pragma unroll
+      for (int i = 0; i < 9; ++i) Fh[i] = Fn[i] + dt * GF[i];
+      stress_matrix(P, Fh, Fn, Jp, vol, Sp, fb);
+#pragma unroll
+      for (int i = 0; i < 9; ++i) a.stress[i * cap + j] = Sp[i];
+    }
+  }
+  if (__ballot(fb != 0)) {  // one atomic per wave
+    unsigned long long c = (unsigned long long)fb;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off);
+    if (lane_id() == 0) atomicAdd(a.fallback_svd, c);
+  }
 }
 
 template <int ORDER, int MODE, int RANKS>
@@ -1079,8 +1141,8 @@ __global__ __launch_bounds__(64 * P2G_WAVES) void k_p2g(P2GArgs a) {
     int cr2 = cr, k2 = k;
     advance(cr2, k2);
     int pi2 = 0;
-    if (MODE != P2G_FORCE && cr < 2 && sr < P2G_RANKS && sr < rcnt_of(cr)) p2g_load<MODE>(a, S, rstart_of(cr) + sr, in);
-    if (MODE != P2G_FORCE && cr2 < 2 && sr < P2G_RANKS && P2G_RANKS * k2 + sr < rcnt_of(cr2))
+    if (cr < 2 && sr < P2G_RANKS && sr < rcnt_of(cr)) p2g_load<MODE>(a, S, rstart_of(cr) + sr, in);
+    if (cr2 < 2 && sr < P2G_RANKS && P2G_RANKS * k2 + sr < rcnt_of(cr2))
       pi2 = p2g_slot(a, rstart_of(cr2) + P2G_RANKS * k2 + sr);
     float acc[4][NQ];
 #pragma unroll
@@ -1095,8 +1157,7 @@ __global__ __launch_bounds__(64 * P2G_WAVES) void k_p2g(P2GArgs a) {
       if (sr < P2G_RANKS) {
         const int rank = P2G_RANKS * k + sr;
         if (rank < cnt) {
-          if constexpr (MODE == P2G_FORCE) p2g_load<MODE>(a, S, rstart + rank, in);
-          p2g_stage<ORDER, MODE>(a, S, P, noff, dt, in, g0, g1, g2, &s_pay[w][(cx * PAY_CELL + sr * PAY_STRIDE) / 4]);
+          p2g_stage<ORDER, MODE>(a, S, dt, in, g0, g1, g2, &s_pay[w][(cx * PAY_CELL + sr * PAY_STRIDE) / 4]);
         }
       }
       __builtin_amdgcn_wave_barrier();
@@ -1104,10 +1165,10 @@ __global__ __launch_bounds__(64 * P2G_WAVES) void k_p2g(P2GArgs a) {
       // ---- the next step: its particles' data (their slots arrived during this step), and the
       // slots of the step after it
       const int ncr = cr2, nk = k2;
-      if (MODE != P2G_FORCE && ncr < 2 && sr < P2G_RANKS && P2G_RANKS * nk + sr < rcnt_of(ncr))
-        p2g_load_at<MODE>(a, S, pi2, in);
+      if (ncr < 2 && sr < P2G_RANKS && P2G_RANKS * nk + sr < rcnt_of(ncr))
+        p2g_load_at<MODE>(a, S, pi2, rstart_of(ncr) + P2G_RANKS * nk + sr, in);
       advance(cr2, k2);
-      if (MODE != P2G_FORCE && cr2 < 2 && sr < P2G_RANKS && P2G_RANKS * k2 + sr < rcnt_of(cr2))
+      if (cr2 < 2 && sr < P2G_RANKS && P2G_RANKS * k2 + sr < rcnt_of(cr2))
         pi2 = p2g_slot(a, rstart_of(cr2) + P2G_RANKS * k2 + sr);
       // ---- accumulate this lane's cell, ascending rank
       const int nr = min(P2G_RANKS, cnt - P2G_RANKS * k);
@@ -1259,21 +1320,20 @@ __global__ __launch_bounds__(256) void k_p2g_layer(P2GArgs a) {
 #pragma unroll
           for (int q = 0; q < NQ; ++q) acc[i][j][q] = 0.0f;
       StageIn in;
-      if (MODE != P2G_FORCE && sr < RANKS && sr < cnt) p2g_load<MODE>(a, S, start + sr, in);
+      if (sr < RANKS && sr < cnt) p2g_load<MODE>(a, S, start + sr, in);
       int pi2 = 0;  // slot of this lane's particle in the chunk after the next
-      if (MODE != P2G_FORCE && sr < RANKS && RANKS + sr < cnt) pi2 = p2g_slot(a, start + RANKS + sr);
+      if (sr < RANKS && RANKS + sr < cnt) pi2 = p2g_slot(a, start + RANKS + sr);
       for (int k = 0; k * RANKS < cmax; ++k) {
         if (sr < RANKS) {
           const int rank = RANKS * k + sr;
           if (rank < cnt) {
-            if constexpr (MODE == P2G_FORCE) p2g_load<MODE>(a, S, start + rank, in);
-            p2g_stage<ORDER, MODE>(a, S, P, noff, dt, in, g0, g1, g2, &s_pay[w][(c * PAY_CELL + sr * PAY_STRIDE) / 4]);
+            p2g_stage<ORDER, MODE>(a, S, dt, in, g0, g1, g2, &s_pay[w][(c * PAY_CELL + sr * PAY_STRIDE) / 4]);
           }
         }
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        if (MODE != P2G_FORCE && sr < RANKS) {  // the next chunk's data and the slots of the one after
-          if (RANKS * (k + 1) + sr < cnt) p2g_load_at<MODE>(a, S, pi2, in);
+        if (sr < RANKS) {  // the next chunk's data and the slots of the one after
+          if (RANKS * (k + 1) + sr < cnt) p2g_load_at<MODE>(a, S, pi2, start + RANKS * (k + 1) + sr, in);
           if (RANKS * (k + 2) + sr < cnt) pi2 = p2g_slot(a, start + RANKS * (k + 2) + sr);
         }
         const int nr = min(RANKS, cnt - RANKS * k);
@@ -2572,6 +2632,12 @@ void launch_p2g(hipStream_t s, const P2GArgs& a, int order, int mode, int grid, 
     if (ranks == 4) launch_p2g_r<4>(s, a, order, mode, grid);
     else launch_p2g_r<8>(s, a, order, mode, grid);
   }
+}
+
+void launch_stress_predicted(hipStream_t s, const P2GArgs& a, int order, int nblocks) {
+  if (a.n <= 0) return;
+  if (order == 2) hipLaunchKernelGGL(k_stress_predicted<2>, dim3(nblocks), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL(k_stress_predicted<3>, dim3(nblocks), dim3(256), 0, s, a);
 }
 
 void launch_clock_update(hipStream_t s, Clock* c, int init) {

@@ -483,6 +483,8 @@ static P2GArgs p2g_args(mpm_ctx* ctx, float dt) {
   a.active_tiles = ctx->active_tiles;
   a.partials = ctx->partials;
   a.gvel = reinterpret_cast<const float4*>(ctx->grid + GRID_VEL * ctx->ng);
+  // scratch: the F planes of the buffer that this substep's G2P will write
+  a.stress = ctx->state[1 - ctx->cur] + (size_t)PF * ctx->cap;
   a.dt = dt;
   a.fallback_svd = ctx->fallbacks;
   a.clk = ctx->clk_active;
@@ -522,6 +524,7 @@ static int stage_p2g(mpm_ctx* ctx, float dt) {
   } else {
     launch_p2g(s, a, ctx->order, P2G_MOM, ctx->p2g_grid, ctx->p2g_ranks, ctx->p2g_pass);
     launch_grid(s, grid_args(ctx, dt), GRID_NORMALIZE, ctx->grid_grid);
+    launch_stress_predicted(s, a, ctx->order, ctx->nblocks_p);
     launch_p2g(s, a, ctx->order, P2G_FORCE, ctx->p2g_grid, ctx->p2g_ranks, ctx->p2g_pass);
   }
   return MPM_OK;
