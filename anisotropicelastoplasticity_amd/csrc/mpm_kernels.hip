@@ -36,6 +36,16 @@ __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }
 // produce wrong values, never an out-of-bounds access.
 __device__ __forceinline__ int clamp_index(int i, int n) { return i < 0 ? 0 : (i >= n ? n - 1 : i); }
 
+// Element i of a plane whose address is uniform, through a 32-bit byte offset: one vector register and no
+// 64-bit address arithmetic per access (a state plane holds fewer than 2^30 particles: 35 planes of as many
+// floats would not fit any device).
+__device__ __forceinline__ float plane_load(const float* plane, uint32_t i) {
+  return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(plane) + (size_t)(uint32_t)(4u * i));
+}
+__device__ __forceinline__ void plane_store(float* plane, uint32_t i, float v) {
+  *reinterpret_cast<float*>(reinterpret_cast<char*>(plane) + (size_t)(uint32_t)(4u * i)) = v;
+}
+
 // wave-uniform float held in a scalar register (the readfirstlane builtin works on 32-bit integers)
 __device__ __forceinline__ float uniform_f(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
@@ -821,28 +831,28 @@ __device__ __forceinline__ int p2g_slot(const P2GArgs& a, int idx) { return a.sr
 
 template <int MODE>
 __device__ __forceinline__ void p2g_load_at(const P2GArgs& a, const P2GScene& S, int slot, int idx, StageIn& in) {
-  const int pi = clamp_index(slot, a.n);
+  const uint32_t pi = (uint32_t)clamp_index(slot, a.n);
   const float* st = a.state;
   const int64_t cap = a.cap;
   // a scene without a mesh loads word 0 of the id plane in every lane (one cache line) instead of a
   // branch around the load: a branch here makes the wave wait for this chunk's loads before the
   // accumulation of the previous one
-  in.pid = reinterpret_cast<const int*>(st + (size_t)PID * cap)[S.mesh_e1 > S.mesh_v0 ? pi : 0];
+  in.pid = __float_as_int(plane_load(st + PID * cap, S.mesh_e1 > S.mesh_v0 ? pi : 0u));
 #pragma unroll
-  for (int d = 0; d < 3; ++d) in.x[d] = st[(PX + d) * cap + pi];
+  for (int d = 0; d < 3; ++d) in.x[d] = plane_load(st + (PX + d) * cap, pi);
   if constexpr (MODE != P2G_FORCE) {
-    in.m = st[PM * cap + pi];
+    in.m = plane_load(st + PM * cap, pi);
 #pragma unroll
-    for (int d = 0; d < 3; ++d) in.v[d] = st[(PV + d) * cap + pi];
+    for (int d = 0; d < 3; ++d) in.v[d] = plane_load(st + (PV + d) * cap, pi);
 #pragma unroll
-    for (int i = 0; i < 9; ++i) in.B[i] = st[(PB + i) * cap + pi];
+    for (int i = 0; i < 9; ++i) in.B[i] = plane_load(st + (PB + i) * cap, pi);
   } else {
 #pragma unroll
-    for (int i = 0; i < 9; ++i) in.B[i] = a.stress[i * cap + idx];
+    for (int i = 0; i < 9; ++i) in.B[i] = plane_load(a.stress + i * cap, (uint32_t)idx);
   }
   if constexpr (MODE == P2G_MOM_STRESS) {
 #pragma unroll
-    for (int i = 0; i < 6; ++i) in.K[i] = st[(PK + i) * cap + pi];
+    for (int i = 0; i < 6; ++i) in.K[i] = plane_load(st + (PK + i) * cap, pi);
   }
 }
 
@@ -880,6 +890,10 @@ __device__ __forceinline__ void p2g_stage(const P2GArgs& a, const P2GScene& S, f
     pay[PY_WZ + o] = wz[o];
     pay[PY_DWZ + o] = dwz[o];
   }
+  // the weights leave their registers before the rest is formed (the layer pass holds 64 sums meanwhile)
+#pragma unroll
+  for (int i = 0; i < PY_G / 4; ++i) dst[i] = make_float4(pay[4 * i], pay[4 * i + 1], pay[4 * i + 2], pay[4 * i + 3]);
+  __builtin_amdgcn_sched_barrier(0);
   float Q0[3] = {0.0f, 0.0f, 0.0f}, S0[3] = {0.0f, 0.0f, 0.0f};  // x columns of Q and of S
   if constexpr (MODE != P2G_FORCE) {
     // momentum w*(q0 + Q o): Q = m D^-1 B diag(h), q0 = m v - Q (1 + f)  (HybridSolver.cpp:134,169-170)
@@ -945,7 +959,7 @@ __device__ __forceinline__ void p2g_stage(const P2GArgs& a, const P2GScene& S, f
 #pragma unroll
     for (int r = 0; r < 3; ++r) pay[PY_G + 3 * ox + r] = (float)ox * wx[ox] * Q0[r] - dwx[ox] * S0[r];
 #pragma unroll
-  for (int i = 0; i < PAY / 4; ++i) dst[i] = make_float4(pay[4 * i], pay[4 * i + 1], pay[4 * i + 2], pay[4 * i + 3]);
+  for (int i = PY_G / 4; i < PAY / 4; ++i) dst[i] = make_float4(pay[4 * i], pay[4 * i + 1], pay[4 * i + 2], pay[4 * i + 3]);
 }
 
 // Stress matrix V P(F^) F^n^T of every particle at the predicted F^ = F + dt (sum_i v_i grad w_ip^T) F from
@@ -1263,7 +1277,46 @@ __global__ __launch_bounds__(64 * P2G_WAVES) void k_p2g(P2GArgs a) {
   }
 }
 
-// Layer pass (the alternative P2G schedule, chosen by the autotuner). One workgroup (4 waves) per
+// Constants of a tile's scene.
+struct TileScene {
+  P2GScene S;
+  int64_t noff;
+  int sc, toff, nt0, nt1;
+};
+__device__ __forceinline__ TileScene tile_scene(const P2GArgs& a, int sc) {
+  TileScene n;
+  n.sc = sc;
+  n.S = p2g_scene(a.T.params[sc]);
+  n.noff = a.T.node_off[sc];
+  n.toff = __builtin_amdgcn_readfirstlane(a.T.tile_off[sc]);
+  n.nt0 = __builtin_amdgcn_readfirstlane(a.T.params[sc].tiles[0]);
+  n.nt1 = __builtin_amdgcn_readfirstlane(a.T.params[sc].tiles[1]);
+  return n;
+}
+// The first cell of a wave's layer of a tile (uniform), and the lane's cell: occ, lo and hi as loaded (lo, hi
+// hold something else where occ is 0).
+struct TileCell {
+  int g0, g1, g2;
+  uint32_t occ;
+  int lo, hi;
+};
+__device__ __forceinline__ TileCell tile_cell(const P2GArgs& a, const TileScene& n, int gtile, int cx, int cy, int cz) {
+  TileCell b;
+  const int tile = gtile - n.toff;
+  const int t0 = tile % n.nt0, t1 = (tile / n.nt0) % n.nt1, t2 = tile / (n.nt0 * n.nt1);
+  b.g0 = 4 * t0;
+  b.g1 = 4 * t1;
+  b.g2 = 4 * t2 + cz;
+  const bool in = b.g0 + cx < n.S.res[0] && b.g1 + cy < n.S.res[1] && b.g2 < n.S.res[2];
+  const int64_t key = n.noff + (in ? (b.g2 * n.S.res[1] + b.g1 + cy) * n.S.res[0] + b.g0 + cx : 0);
+  b.occ = a.occ[key / SCAN_TILE];
+  b.lo = a.cell_start[key];
+  b.hi = a.cell_end[key];
+  if (!in) b.occ = 0u;
+  return b;
+}
+
+// Layer pass (the other P2G schedule). One workgroup (4 waves) per
 // active tile; wave w owns cell layer z = w and all 16 cells of it at once. Staging lane (c, r),
 // c = lane >> 2 (cell x = c & 3, y = c >> 2), r < RANKS, stages rank RANKS k + r of cell c; then
 // lane (c, zo) adds the chunk's particles of cell c, in ascending rank, to 16 x 4 register sums:
@@ -1272,123 +1325,137 @@ __global__ __launch_bounds__(64 * P2G_WAVES) void k_p2g(P2GArgs a) {
 // row halves with a slab each, the order in which a slab node receives the cell sums (rows
 // ascending, then ox ascending: phases oy = 3..0, ox = 0..3) and the order of the slab sums are
 // those of the row pass, so both passes give the same bits.
+//
+// Bound by vector instructions (two thirds of the VALU's cycles) and by what is exposed of each tile's chain
+// of loads (list entry, bins, slots, particles) before its first particle. So the next tile's bins are loaded
+// before this tile's chunks, its first slots after them, and its first particles before the slab sums are
+// stored; and a wave's slabs take the place of its payloads, which are done with by then: 52 KB a workgroup
+// instead of 71, three on a CU instead of two. P2G at 2^22 particles (7.5 per cell) 302 -> 272 us; 16 scenes
+// of 1.8 M in all 157 -> 148 us.
 template <int ORDER, int MODE, int RANKS>
-__global__ __launch_bounds__(256) void k_p2g_layer(P2GArgs a) {
+__global__ __launch_bounds__(256, 3) void k_p2g_layer(P2GArgs a) {
   if (clock_skip(a.clk)) return;
   const float dt = clock_dt(a.clk, a.dt);
-  constexpr int PAY_CELL = pay_cell<RANKS>();
-  __shared__ float4 s_pay[4][16 * PAY_CELL / 4];
-  __shared__ float s_slab[8][4][SLAB];  // [layer + 4 row half][quantity][node], as the row pass's waves
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int ntile = a.counters[CNT_TILES];
+  constexpr int PAY_CELL = RANKS * PAY_STRIDE;
   constexpr int NQ = (MODE == P2G_FORCE) ? 3 : 4;
+  constexpr int WAVE_FLOATS = 16 * PAY_CELL > 2 * NQ * SLAB ? 16 * PAY_CELL : 2 * NQ * SLAB;
+  __shared__ float4 s_wave[4][WAVE_FLOATS / 4];
+  static_assert(WAVE_FLOATS % 4 == 0 && (2 * NQ * SLAB) % 4 == 0, "float4 slots");
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int ntile = a.counters[CNT_TILES];
   const int c = lane >> 2, sr = lane & 3, zo = lane & 3;  // staging (c, sr); accumulation (c, zo)
   const int cx = c & 3, cy = c >> 2;
   const float fzo = (float)zo;
-  for (int i = tid; i < 8 * 4 * SLAB; i += 256) (&s_slab[0][0][0])[i] = 0.0f;
-  __syncthreads();
-  float* slab = &s_slab[w + 4 * (cy >> 1)][0][0];
+  float4* pay = &s_wave[w][0];
+  float* slab = reinterpret_cast<float*>(pay) + (cy >> 1) * NQ * SLAB;  // [row half][quantity][node]
   const XcdRange tr = xcd_range(ntile);
+  if (tr.first >= tr.end) return;  // uniform: no tile for this workgroup
+  auto scene_at = [&](int gtile) {
+    return a.T.nscenes == 1 ? 0 : __builtin_amdgcn_readfirstlane(scene_of(a.T.tile_off, a.T.nscenes, gtile));
+  };
+  const int last = tr.first + (tr.end - 1 - tr.first) / tr.stride * tr.stride;  // this workgroup's last list entry
+  int gtile = __builtin_amdgcn_readfirstlane(a.active_tiles[tr.first]);
+  int gtile_next = a.active_tiles[min(tr.first + tr.stride, last)];
+  TileScene n = tile_scene(a, scene_at(gtile));
+  TileCell cell = tile_cell(a, n, gtile, cx, cy, w);
+  int start = cell.lo, cnt = cell.occ ? cell.hi - cell.lo : 0;
+  StageIn in;
+  int pi2 = 0;  // slot of this lane's particle in the chunk after the next
+  if (sr < RANKS && sr < cnt) p2g_load<MODE>(a, n.S, start + sr, in);
+  if (sr < RANKS && RANKS + sr < cnt) pi2 = p2g_slot(a, start + RANKS + sr);
   for (int slot = tr.first; slot < tr.end; slot += tr.stride) {
-    const int gtile = a.active_tiles[slot];
-    const int sc = __builtin_amdgcn_readfirstlane(scene_of(a.T.tile_off, a.T.nscenes, gtile));
-    const DevParams& P = a.T.params[sc];
-    const P2GScene S = p2g_scene(P);
-    const int64_t noff = a.T.node_off[sc];
-    const int tile = gtile - a.T.tile_off[sc];
-    const int nt0 = __builtin_amdgcn_readfirstlane(P.tiles[0]), nt1 = __builtin_amdgcn_readfirstlane(P.tiles[1]);
-    const int t0 = tile % nt0, t1 = (tile / nt0) % nt1, t2 = tile / (nt0 * nt1);
-    const int g0 = 4 * t0 + cx, g1 = 4 * t1 + cy, g2 = 4 * t2 + w;
-    int start = 0, cnt = 0;
-    if (g0 < S.res[0] && g1 < S.res[1] && g2 < S.res[2]) {
-      const int64_t key = noff + (g2 * S.res[1] + g1) * S.res[0] + g0;
-      if (a.occ[key / SCAN_TILE]) {
-        start = a.cell_start[key];
-        cnt = a.cell_end[key] - start;
-      }
-    }
+    // the next tile's cells (the last tile's own again at the end: loaded, not used)
+    gtile = __builtin_amdgcn_readfirstlane(gtile_next);
+    gtile_next = a.active_tiles[min(slot + 2 * tr.stride, last)];
+    const P2GScene S = n.S;  // this tile's
+    const int sc_next = scene_at(gtile);
+    if (sc_next != n.sc) n = tile_scene(a, sc_next);
+    const TileCell next = tile_cell(a, n, gtile, cx, cy, w);
     int cmax = cnt;
 #pragma unroll
     for (int off = 4; off < 64; off <<= 1) cmax = max(cmax, __shfl_xor(cmax, off));
     cmax = __builtin_amdgcn_readfirstlane(cmax);
-    if (cmax > 0) {
-      float acc[4][4][NQ];  // [oy][ox][quantity]
+    float acc[4][4][NQ];  // [oy][ox][quantity]
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int q = 0; q < NQ; ++q) acc[i][j][q] = 0.0f;
-      StageIn in;
-      if (sr < RANKS && sr < cnt) p2g_load<MODE>(a, S, start + sr, in);
-      int pi2 = 0;  // slot of this lane's particle in the chunk after the next
-      if (sr < RANKS && RANKS + sr < cnt) pi2 = p2g_slot(a, start + RANKS + sr);
-      for (int k = 0; k * RANKS < cmax; ++k) {
-        if (sr < RANKS) {
-          const int rank = RANKS * k + sr;
-          if (rank < cnt) {
-            p2g_stage<ORDER, MODE>(a, S, dt, in, g0, g1, g2, &s_pay[w][(c * PAY_CELL + sr * PAY_STRIDE) / 4]);
-          }
-        }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        if (sr < RANKS) {  // the next chunk's data and the slots of the one after
-          if (RANKS * (k + 1) + sr < cnt) p2g_load_at<MODE>(a, S, pi2, start + RANKS * (k + 1) + sr, in);
-          if (RANKS * (k + 2) + sr < cnt) pi2 = p2g_slot(a, start + RANKS * (k + 2) + sr);
-        }
-        const int nr = min(RANKS, cnt - RANKS * k);
-        for (int r = 0; r < nr; ++r) {
-          const float4* src = &s_pay[w][(c * PAY_CELL + r * PAY_STRIDE) / 4];
-          const float* pf = reinterpret_cast<const float*>(src);
-          const float4 WX = src[PY_WX / 4], WY = src[PY_WY / 4], DWY = src[PY_DWY / 4];
-          const float wxs[4] = {WX.x, WX.y, WX.z, WX.w};
-          const float wys[4] = {WY.x, WY.y, WY.z, WY.w};
-          const float dwys[4] = {DWY.x, DWY.y, DWY.z, DWY.w};
-          const float wz = pf[PY_WZ + zo], dwz = pf[PY_DWZ + zo];
-          float g[12];
-#pragma unroll
-          for (int i = 0; i < 3; ++i) {
-            const float4 t = src[PY_G / 4 + i];
-            g[4 * i] = t.x; g[4 * i + 1] = t.y; g[4 * i + 2] = t.z; g[4 * i + 3] = t.w;
-          }
-          float qs[16];  // m, q0(3), Q12(6), S12(6)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float4 t = src[PY_M / 4 + i];
-            qs[4 * i] = t.x; qs[4 * i + 1] = t.y; qs[4 * i + 2] = t.z; qs[4 * i + 3] = t.w;
-          }
-#pragma unroll
-          for (int oy = 0; oy < 4; ++oy) {
-            const float wy = wys[oy], dwy = dwys[oy];
-            const float wyz = wy * wz, dyz = dwy * wz, ydz = wy * dwz;
-            float e[3];
-#pragma unroll
-            for (int rr = 0; rr < 3; ++rr) {
-              float qrow = qs[1 + rr];
-              if constexpr (MODE != P2G_FORCE)
-                qrow = __builtin_fmaf(qs[4 + 2 * rr + 1], fzo, __builtin_fmaf(qs[4 + 2 * rr], (float)oy, qrow));
-              e[rr] = wyz * qrow;
-              if constexpr (MODE != P2G_MOM)
-                e[rr] = __builtin_fmaf(-qs[10 + 2 * rr + 1], ydz, __builtin_fmaf(-qs[10 + 2 * rr], dyz, e[rr]));
-            }
-            const float mw = qs[0] * wyz;
-#pragma unroll
-            for (int ox = 0; ox < 4; ++ox) {
-              const float wx = wxs[ox];
-              constexpr int q1 = (MODE != P2G_FORCE) ? 1 : 0;
-              if constexpr (MODE != P2G_FORCE) acc[oy][ox][0] = __builtin_fmaf(wx, mw, acc[oy][ox][0]);
-#pragma unroll
-              for (int rr = 0; rr < 3; ++rr)
-                acc[oy][ox][q1 + rr] =
-                    __builtin_fmaf(wyz, g[3 * ox + rr], __builtin_fmaf(wx, e[rr], acc[oy][ox][q1 + rr]));
-            }
-          }
-        }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        for (int q = 0; q < NQ; ++q) acc[i][j][q] = 0.0f;
+    for (int k = 0; k * RANKS < cmax; ++k) {
+      if (sr < RANKS && RANKS * k + sr < cnt)
+        p2g_stage<ORDER, MODE>(a, S, dt, in, cell.g0 + cx, cell.g1 + cy, cell.g2, pay + (c * PAY_CELL + sr * PAY_STRIDE) / 4);
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      if (sr < RANKS) {  // the next chunk's data and the slots of the one after
+        if (RANKS * (k + 1) + sr < cnt) p2g_load_at<MODE>(a, S, pi2, start + RANKS * (k + 1) + sr, in);
+        if (RANKS * (k + 2) + sr < cnt) pi2 = p2g_slot(a, start + RANKS * (k + 2) + sr);
       }
-      // ---- the cells' sums into the slab of their row half: phase (oy descending, ox ascending),
-      // node (cx + ox, cy + oy, zo); a node receives its cells in ascending row, then ascending ox
+      const int nr = min(RANKS, cnt - RANKS * k);
+      for (int r = 0; r < nr; ++r) {
+        const float4* src = pay + (c * PAY_CELL + r * PAY_STRIDE) / 4;
+        const float* pf = reinterpret_cast<const float*>(src);
+        const float4 WX = src[PY_WX / 4], WY = src[PY_WY / 4], DWY = src[PY_DWY / 4];
+        const float wxs[4] = {WX.x, WX.y, WX.z, WX.w};
+        const float wys[4] = {WY.x, WY.y, WY.z, WY.w};
+        const float dwys[4] = {DWY.x, DWY.y, DWY.z, DWY.w};
+        const float wz = pf[PY_WZ + zo], dwz = pf[PY_DWZ + zo];
+        float g[12];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const float4 t = src[PY_G / 4 + i];
+          g[4 * i] = t.x; g[4 * i + 1] = t.y; g[4 * i + 2] = t.z; g[4 * i + 3] = t.w;
+        }
+        float qs[16];  // m, q0(3), Q12(6), S12(6)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float4 t = src[PY_M / 4 + i];
+          qs[4 * i] = t.x; qs[4 * i + 1] = t.y; qs[4 * i + 2] = t.z; qs[4 * i + 3] = t.w;
+        }
+#pragma unroll
+        for (int oy = 0; oy < 4; ++oy) {
+          const float wy = wys[oy], dwy = dwys[oy];
+          const float wyz = wy * wz, dyz = dwy * wz, ydz = wy * dwz;
+          float e[3];
+#pragma unroll
+          for (int rr = 0; rr < 3; ++rr) {
+            float qrow = qs[1 + rr];
+            if constexpr (MODE != P2G_FORCE)
+              qrow = __builtin_fmaf(qs[4 + 2 * rr + 1], fzo, __builtin_fmaf(qs[4 + 2 * rr], (float)oy, qrow));
+            e[rr] = wyz * qrow;
+            if constexpr (MODE != P2G_MOM)
+              e[rr] = __builtin_fmaf(-qs[10 + 2 * rr + 1], ydz, __builtin_fmaf(-qs[10 + 2 * rr], dyz, e[rr]));
+          }
+          const float mw = qs[0] * wyz;
+#pragma unroll
+          for (int ox = 0; ox < 4; ++ox) {
+            const float wx = wxs[ox];
+            constexpr int q1 = (MODE != P2G_FORCE) ? 1 : 0;
+            if constexpr (MODE != P2G_FORCE) acc[oy][ox][0] = __builtin_fmaf(wx, mw, acc[oy][ox][0]);
+#pragma unroll
+            for (int rr = 0; rr < 3; ++rr)
+              acc[oy][ox][q1 + rr] =
+                  __builtin_fmaf(wyz, g[3 * ox + rr], __builtin_fmaf(wx, e[rr], acc[oy][ox][q1 + rr]));
+          }
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    }
+    // the slots of the next tile's first two chunks
+    cell = next;
+    start = cell.lo;
+    cnt = cell.occ && slot + tr.stride < tr.end ? cell.hi - cell.lo : 0;
+    int pi1 = 0;
+    if (sr < RANKS && sr < cnt) pi1 = p2g_slot(a, start + sr);
+    if (sr < RANKS && RANKS + sr < cnt) pi2 = p2g_slot(a, start + RANKS + sr);
+    // ---- the payloads are done with: clear the wave's slabs, then the cells' sums into the slab of their
+    // row half: phase (oy descending, ox ascending), node (cx + ox, cy + oy, zo); a node receives its cells
+    // in ascending row, then ascending ox
+    for (int i = lane; i < 2 * NQ * SLAB / 4; i += 64) pay[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (cmax > 0) {
 #pragma unroll
       for (int oy = 3; oy >= 0; --oy)
 #pragma unroll
@@ -1400,8 +1467,9 @@ __global__ __launch_bounds__(256) void k_p2g_layer(P2GArgs a) {
           __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         }
     }
+    if (sr < RANKS && sr < cnt) p2g_load_at<MODE>(a, n.S, pi1, start + sr, in);  // the next tile's first chunk
     __syncthreads();
-    // ---- tile partial: as the row pass (layers l ascending, row halves in order); slabs cleared
+    // ---- tile partial: layers l ascending, row halves in order
     float* part = a.partials + (size_t)slot * PART_STRIDE + (MODE == P2G_FORCE ? 4 * FOOT3 : 0);
     for (int i = tid; i < FOOT3; i += 256) {
       const int X = i % FOOT, Y = (i / FOOT) % FOOT, Z = i / (FOOT * FOOT);
@@ -1410,15 +1478,11 @@ __global__ __launch_bounds__(256) void k_p2g_layer(P2GArgs a) {
       for (int q = 0; q < NQ; ++q) sum[q] = 0.0f;
 #pragma unroll
       for (int ww = 0; ww < 8; ++ww) {
-        const int l = ww >> 1, hh = ww & 1, wv = l + 4 * hh;
-        const int z = Z - l;
+        const int l = ww >> 1, hh = ww & 1, z = Z - l;
         if (z < 0 || z > 3) continue;
-        const int ln = X + FOOT * Y + FOOT * FOOT * z;
+        const float* p = reinterpret_cast<const float*>(&s_wave[l][0]) + hh * NQ * SLAB + X + FOOT * Y + FOOT * FOOT * z;
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-          sum[q] += s_slab[wv][q][ln];
-          s_slab[wv][q][ln] = 0.0f;
-        }
+        for (int q = 0; q < NQ; ++q) sum[q] += p[q * SLAB];
       }
       if constexpr (NQ == 4) {
         reinterpret_cast<float4*>(part)[i] = make_float4(sum[0], sum[1], sum[2], sum[3]);

@@ -133,8 +133,9 @@ struct mpm_ctx {
   float graph_dt[2] = {0.0f, 0.0f};
 
   int p2g_grid = 512;
-  int p2g_ranks = 8;  // P2G staging chunk (mpm_autotune / mpm_set_tuning)
-  int p2g_pass = P2G_ROWS;  // P2G schedule (mpm_autotune / mpm_set_tuning)
+  int p2g_ranks = 8;  // P2G staging chunk
+  int p2g_pass = P2G_ROWS;  // P2G schedule
+  bool p2g_tuned = false;   // set by mpm_autotune or mpm_set_tuning (else choose_p2g does)
   // adaptive time step (mpm_solve): the device clock, and the pointer the kernels get (null for
   // fixed-step runs)
   Clock* clock = nullptr;
@@ -508,6 +509,34 @@ static GridArgs grid_args(mpm_ctx* ctx, float dt) {
   g.clk = ctx->clk_active;
   g.vmax_out = nullptr;
   return g;
+}
+
+// The P2G launch shape of a context that nothing has tuned, before its substeps are captured: from the active
+// tiles of the last sort. A layer's wave works through its 16 cells in lockstep and a row's 8 waves share a
+// tile, so layers pay when the tiles outnumber the CUs and are not crowded. Measured (MI355X, quadratic, P2G
+// stage in us, rows of 8 ranks on 2 / 4 workgroups per CU against layers of 4 ranks on 3):
+//   particles  tiles  per tile     rows        layers
+//      64,000    216       296    19 /  19        20
+//     140,608    392       359    25 /  25        22
+//     262,144    343       764    42 /  40        38
+//     681,472  1,728       394    65 /  67        52
+//     681,472    729       935    57 /  63        67
+//   1,560,896  2,227       701   105 / 108       101
+//   1,560,896  1,579       989   118 / 114       139
+//   4,194,304  9,537       440   357 / 333       271
+// Cubic splines and predicted stress lie alike (681,472 particles, cubic: 77 / 80 against 60). A mesh crowds the
+// cells that it passes through, whatever the mean: 0.5 M sand particles on a 256 x 256-vertex cloth 89 / 89
+// against 99.
+static int choose_p2g(mpm_ctx* ctx) {
+  if (ctx->p2g_tuned) return MPM_OK;
+  int tiles = 0;
+  CK(hipMemcpyAsync(&tiles, ctx->counters + CNT_TILES, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+  CK(hipStreamSynchronize(ctx->stream));
+  const bool layers = ctx->mesh.ne == 0 && tiles > ctx->n_cu && ctx->n <= 640LL * tiles;
+  ctx->p2g_pass = layers ? P2G_LAYERS : P2G_ROWS;
+  ctx->p2g_ranks = layers ? 4 : 8;
+  ctx->p2g_grid = std::max(128, ctx->n_cu * (layers ? 3 : tiles > 4 * ctx->n_cu ? 4 : 2));
+  return MPM_OK;
 }
 
 static int stage_p2g(mpm_ctx* ctx, float dt) {
@@ -1377,6 +1406,8 @@ int mpm_run(mpm_ctx* ctx, float dt, int32_t nsteps) {
         (void)hipGraphExecDestroy(ctx->graph[c0]);
         ctx->graph[c0] = nullptr;
       }
+      rc = choose_p2g(ctx);
+      if (rc) return rc;
       hipGraph_t g = nullptr;
       const int64_t steps0 = ctx->substeps;
       const int sort0 = ctx->sort_buf;
@@ -1461,6 +1492,8 @@ int mpm_solve(mpm_ctx* ctx, double cfl, double maxt, mpm_frame_callback cb, void
     } else {
       const int c0 = ctx->cur;
       if (!ctx->graph_adapt[c0]) {
+        rc = choose_p2g(ctx);
+        if (rc) return rc;
         hipGraph_t gr = nullptr;
         const int64_t steps0 = ctx->substeps;
         const int sort0 = ctx->sort_buf;
@@ -1563,9 +1596,8 @@ int mpm_autotune(mpm_ctx* ctx, float dt, int32_t reps, mpm_tuning* chosen) {
   const P2GArgs a = p2g_args(ctx, dt);
   best.p2g_ms = 1e30f;
   struct P2GCand { int pass, ranks, mult; };
-  const P2GCand cands[] = {{P2G_ROWS, 4, 1}, {P2G_ROWS, 4, 2}, {P2G_ROWS, 4, 4}, {P2G_ROWS, 8, 1},
-                           {P2G_ROWS, 8, 2}, {P2G_ROWS, 8, 4}, {P2G_LAYERS, 2, 2}, {P2G_LAYERS, 2, 3},
-                           {P2G_LAYERS, 2, 6}, {P2G_LAYERS, 4, 2}, {P2G_LAYERS, 4, 4}};
+  const P2GCand cands[] = {{P2G_ROWS, 4, 2}, {P2G_ROWS, 8, 2}, {P2G_ROWS, 8, 4}, {P2G_LAYERS, 2, 6},
+                           {P2G_LAYERS, 4, 2}, {P2G_LAYERS, 4, 3}, {P2G_LAYERS, 4, 6}};
   for (const P2GCand& cd : cands) {
     const int blocks = std::max(64, cd.mult * ctx->n_cu);
     const float ms = time_launches(ctx, reps, [&] { launch_p2g(s, a, ctx->order, p2g_mode, blocks, cd.ranks, cd.pass); });
@@ -1595,6 +1627,7 @@ int mpm_autotune(mpm_ctx* ctx, float dt, int32_t reps, mpm_tuning* chosen) {
   ctx->p2g_ranks = best.p2g_ranks;
   ctx->p2g_grid = best.p2g_blocks;
   ctx->p2g_pass = best.p2g_pass;
+  ctx->p2g_tuned = true;
   ctx->grid_grid = best.grid_blocks;
   drop_graphs(ctx);
   if (chosen) *chosen = best;
@@ -1629,6 +1662,7 @@ int mpm_set_tuning(mpm_ctx* ctx, const mpm_tuning* t) {
   ctx->grid_grid = t->grid_blocks;
   ctx->sort_mode = t->sort_mode;
   ctx->p2g_pass = t->p2g_pass;
+  ctx->p2g_tuned = true;
   drop_graphs(ctx);
   return MPM_OK;
 }
