@@ -39,7 +39,9 @@ constexpr int FOOT3 = FOOT * FOOT * FOOT;
 // multiple of 4 floats so that every slot's float4 part is 16-byte aligned.
 constexpr int PART_STRIDE = 7 * FOOT3 + 3;
 
-enum Counter : int { CNT_TILES = 0, CNT_BLOCKS = 1, CNT_CAND = 2, CNT_APEX = 3, CNT_NUM = 4 };
+// The lengths of the active tile and node block lists of the last sort of state buffer b are counters
+// CNT_TILES + 2 b and CNT_BLOCKS + 2 b (the kernels get a pointer offset by 2 b).
+enum Counter : int { CNT_TILES = 0, CNT_BLOCKS = 1, CNT_CAND = 4, CNT_APEX = 5, CNT_NUM = 6 };
 enum P2GMode : int { P2G_MOM_STRESS = 0, P2G_MOM = 1, P2G_FORCE = 2 };
 enum GridMode : int { GRID_FUSED = 0, GRID_NORMALIZE = 1, GRID_FORCE_UPDATE = 2 };
 
@@ -125,16 +127,15 @@ struct Clock {
 __device__ __forceinline__ bool clock_skip(const Clock* c) { return c != nullptr && c->skip != 0; }
 __device__ __forceinline__ float clock_dt(const Clock* c, float dt) { return c != nullptr ? c->dt_f : dt; }
 
-struct ResetArgs {
-  uint32_t* zero_words;
-  int64_t n_zero;
-  const int* counters;
-  const int* active_tiles;
-  int* tile_slot;
-  const int* active_blocks;
-  int* block_slot;
-  int64_t max_tiles;
-  const Clock* clk;
+// The particles of the next sort's cells, counted by the kernel that moves them (k_g2p; k_cloth_elements
+// for a cloth's elements), so that the sort starts at the scan. cell_count is consumed and cleared by the
+// sort; the flags belong to the state buffer the particles are in: the sort of one buffer clears
+// the other's.
+struct BinCounts {
+  int* cell_count;     // [cells] zero between a sort and the next G2P
+  uint32_t* rank;      // [n] a particle's number among its cell's (in no particular order), by physical slot
+  uint8_t* scan_flag;  // [scan blocks] 1 where a cell of the block holds a particle
+  uint8_t* tile_flag;  // [tiles] 1 where a cell of the tile holds a particle
 };
 
 struct SortBufs {
@@ -143,21 +144,26 @@ struct SortBufs {
   uint32_t* hist;     // [4][256]
   uint32_t* tickets;  // [4] digit passes
   uint32_t* status;   // [passes][nblocks][256] digit-pass look-back words
-  uint32_t* scan_agg;   // [scan blocks] particles counted in each scan block's cells
-  int* cell_count;    // [cells] zero between substeps (the bin pass clears the occupied cells)
+  int64_t radix_words;  // words of hist, tickets and status together (zeroed before the digit passes)
+  BinCounts bins;     // this buffer's counts
+  uint8_t* scan_flag_clear;  // the other buffer's flags, cleared
+  uint8_t* tile_flag_clear;
+  uint32_t* scan_sum;  // [scan blocks] particles in each scan block's cells
   int* cell_start;    // [cells + 1] exclusive prefix of the counts; cell c holds [start[c], start[c+1])
-                      // (written for the scan blocks with particles, see occ)
-  uint32_t* occ;        // [scan blocks] 1 where a cell of the block holds a particle (set by the count)
-  uint32_t* occ_clear;  // [scan blocks] the other substep's flags, cleared by the count
-  int64_t ncells;
-  SceneTable T;       // the counting sort also writes src and flags the occupied tiles
-  int* tile_slot;
+                      // (written for the scan blocks with particles, see scan_flag)
+  int64_t ncells, ntiles;
+  SceneTable T;
+  int* tile_slot;     // per tile: slot in the active list, or -1
+  int* active_tiles;
+  int* block_slot;
+  int* active_blocks;
   const int* pid;     // caller id at each physical slot (the state's id plane)
   int* tslot;         // [n] scratch: the physical slot of each binned caller id
   int* pos;           // caller id -> physical slot: written by the radix mode's key conversion
-  int* src;
-  int* counters;      // zeroed by the cell scan (after the counting kernel has read them)
-  ResetArgs reset;    // the counting sort's reset work, done by its counting kernel
+  int* src;           // sorted position -> physical slot
+  int* counters;      // this buffer's list lengths (zero)
+  int* counters_clear;  // the other buffer's, zeroed
+  int* counters_misc;   // CNT_CAND and CNT_APEX, zeroed
   const Clock* clk;
 };
 
@@ -170,7 +176,7 @@ struct P2GArgs {
   const int* src;   // sorted position -> physical index in `state`
   const int* cell_start;
   const int* cell_end;
-  const uint32_t* occ;  // per scan block of cells: 1 if it holds particles (else its cells are empty)
+  const uint8_t* occ;   // per scan block of cells: 1 if it holds particles (else its cells are empty)
   const int* counters;
   const int* active_tiles;
   float* partials;
@@ -213,6 +219,7 @@ struct G2PArgs {
   int write_stress;    // store V tau of the new state (stress at F^n)
   const float* thr;
   uint32_t* keys;      // next cell key, indexed by physical slot in sout
+  BinCounts bins;      // the next sort's counts
   int* status;
   unsigned long long* fallback_svd;
   unsigned long long* fallback_apex;
@@ -283,20 +290,19 @@ void launch_keys(hipStream_t s, const SceneTable& T, int nblocks, const float* s
                  const float* thr, uint32_t* keys, int* status);
 void launch_stress_init(hipStream_t s, const SceneTable& T, int nblocks, float* st, int64_t cap, int n,
                         unsigned long long* fallback);
-void launch_reset(hipStream_t s, const ResetArgs& r);
+// The counts of particles whose keys no G2P has counted (set by the caller, or sorted before): clears the
+// flags and counters (and, if dirty, cell_count), then counts.
+void launch_count(hipStream_t s, const SceneTable& T, const BinCounts& b, const uint32_t* keys, int n, int64_t ncells,
+                  int64_t ntiles, int* counters, bool dirty);
 // cell_start of the scan blocks without particles (only the getter of the bins needs them).
 void launch_fill_bins(hipStream_t s, const uint32_t* ks, int n, int64_t ncells, int* cell_start);
-// Stable sort of the cell keys by caller id. Both modes count the particles of every cell and scan
-// the counts into cell_start. SORT_COUNTING then places each caller id at its stable rank inside
-// its cell; SORT_RADIX runs `passes` 8-bit LSD digit passes (1..4). Both give the same order. The
-// result is in k1/v1 for an odd `passes`, k2/v2 for an even one.
+// Stable sort of the cell keys by caller id, from the counts of every cell. Both modes scan the counts into
+// cell_start and make the active tile and node block lists. SORT_COUNTING then places each
+// caller id at its stable rank inside its cell; SORT_RADIX runs `passes` 8-bit LSD digit passes (1..4). Both
+// give the same order, src[j] = the physical slot of the particle at sorted position j, and cleared cell
+// counts. The sorted keys and ids are in k1/v1 for an odd `passes`, k2/v2 for an even one.
 enum SortMode : int { SORT_COUNTING = 0, SORT_RADIX = 1 };
-void launch_sort(hipStream_t s, const SortBufs& b, const uint32_t* keys_in, int n, int passes, int mode);
-// Active tiles and node blocks from the sorted keys; clears the counts of the occupied cells and
-// writes src[j] = pos[perm[j]]: the physical index of the particle at sorted position j.
-void launch_bounds(hipStream_t s, const SceneTable& T, int nblocks, const uint32_t* ks, int n, int64_t ntiles,
-                   int* cell_count, int* tile_slot, int* active_tiles, int* block_slot, int* active_blocks,
-                   int* counters, const int* perm, const int* pos, int* src, const Clock* clk, int mode);
+void launch_sort(hipStream_t s, const SortBufs& b, const uint32_t* keys_in, int n, int nblocks, int passes, int mode);
 // order: B-spline order of every scene (2 or 3); ranks: particles per cell staged per chunk (4 or 8)
 // pass P2G_ROWS (8-wave workgroups, ranks 4 or 8) or P2G_LAYERS (4-wave workgroups, ranks 2 or 4):
 // two schedules of the same sums in the same order, so every choice gives the same bits.
@@ -341,6 +347,7 @@ struct ClothArgs {
   int nfixed;
   float4* gvel;
   uint32_t* keys;
+  BinCounts bins;
   const float* thr;
   int* status;
   unsigned long long* fallback;

@@ -105,13 +105,19 @@ __device__ __forceinline__ DevParams uniform_params(const DevParams& G) {
 // Exact cell index along one axis: the number of thresholds thr[c] <= x, where thr[c] is the
 // smallest float f with (double(f) - min)/h >= c. This equals static_cast<int>((x - min)/h) of the
 // reference evaluated in double (HybridSolver.cpp:33-36) for x >= min, using FP32 compares only.
+// The FP32 quotient t is within inv_h (2^-24 |gmin| + 2^-24 |x - gmin|) + 2^-24 |t| (rounded bounds, difference,
+// spacing and product), less than 2^-22 (|gmin| inv_h + |t|), of the exact one: where t is farther than that
+// from a whole number, floor(t) is the cell, and the thresholds of the cell itself are not read.
 __device__ __forceinline__ int axis_cell(const float* thr, int res, float x, float gmin, float inv_h, int& oob) {
   if (!(x >= thr[0])) { oob = 1; return 0; }
   if (x >= thr[res]) { oob = 1; return res - 1; }
-  int c = (int)floorf((x - gmin) * inv_h);
+  const float t = (x - gmin) * inv_h, tf = floorf(t), near = 0x1p-22f * (fabsf(gmin) * inv_h + fabsf(t));
+  int c = (int)tf;
   c = c < 0 ? 0 : (c > res - 1 ? res - 1 : c);
-  while (c > 0 && x < thr[c]) --c;
-  while (c < res - 1 && x >= thr[c + 1]) ++c;
+  if (t - tf <= near || t - tf >= 1.0f - near) {
+    while (c > 0 && x < thr[c]) --c;
+    while (c < res - 1 && x >= thr[c + 1]) ++c;
+  }
   return c;
 }
 
@@ -127,11 +133,47 @@ __device__ __forceinline__ int stencil_base(float g, int res) {
   return (int)b;
 }
 
-__device__ __forceinline__ uint32_t cell_key(const DevParams& P, const float* thr, float x0, float x1, float x2, int& oob) {
-  int c0 = axis_cell(thr, P.res[0], x0, P.gmin[0], P.inv_h[0], oob);
-  int c1 = axis_cell(thr + (P.res[0] + 1), P.res[1], x1, P.gmin[1], P.inv_h[1], oob);
-  int c2 = axis_cell(thr + (P.res[0] + 1) + (P.res[1] + 1), P.res[2], x2, P.gmin[2], P.inv_h[2], oob);
-  return (uint32_t)(c2 * P.res[0] * P.res[1] + c1 * P.res[0] + c0);
+__device__ __forceinline__ uint32_t cell_key(const DevParams& P, const float* thr, float x0, float x1, float x2, int& oob,
+                                             int (&c)[3]) {
+  c[0] = axis_cell(thr, P.res[0], x0, P.gmin[0], P.inv_h[0], oob);
+  c[1] = axis_cell(thr + (P.res[0] + 1), P.res[1], x1, P.gmin[1], P.inv_h[1], oob);
+  c[2] = axis_cell(thr + (P.res[0] + 1) + (P.res[1] + 1), P.res[2], x2, P.gmin[2], P.inv_h[2], oob);
+  return (uint32_t)(c[2] * P.res[0] * P.res[1] + c[1] * P.res[0] + c[0]);
+}
+
+// Tile (within the scene) of cell (c0, c1, c2).
+__device__ __forceinline__ int tile_of(const DevParams& P, int c0, int c1, int c2) {
+  return ((c2 >> 2) * P.tiles[1] + (c1 >> 2)) * P.tiles[0] + (c0 >> 2);
+}
+
+// Adds the wave's particles (active lanes with valid set) to the next sort's counts; `tile` is the key's tile
+// over all scenes. Called with the wave's first lanes active. The lanes hold particles in the order of the cells
+// they come from, and few change their cell in a substep, so runs of one key in consecutive lanes are taken
+// together: a run's first lane adds its length with one atomic, all of them in the same instruction, and the
+// wave does not wait for the round trip before the ticket is used. (Grouping all lanes of a key, not only
+// consecutive ones, takes a loop over the keys: k_g2p 383 instead of 371 us at 2^22 particles. The scan blocks' totals are
+// not counted here: one more atomic per wave, on words that few cells share, took k_g2p from 74 to 153 us at
+// 2^20 particles.)
+struct CountTicket {
+  int base, head;
+};
+__device__ __forceinline__ CountTicket count_wave(const BinCounts& b, bool valid, uint32_t key, int tile) {
+  const int lane = (int)lane_id();
+  const uint32_t k = valid ? key : 0xFFFFFFFFu;  // no cell's key
+  const uint32_t prev = (uint32_t)__shfl_up((int)k, 1);
+  const uint64_t heads = __ballot(lane == 0 || k != prev), ends = heads | ~__ballot(true);
+  const uint64_t upto = heads & (~0ull >> (63 - lane)), above = ends & ~(~0ull >> (63 - lane));
+  CountTicket t{0, 63 - __clzll((long long)upto)};
+  if (valid && t.head == lane) {
+    t.base = atomicAdd(&b.cell_count[key], (above ? __ffsll((long long)above) - 1 : 64) - lane);
+    b.tile_flag[tile] = 1;
+    b.scan_flag[key / SCAN_TILE] = 1;
+  }
+  return t;
+}
+// The lane's number in its cell.
+__device__ __forceinline__ uint32_t count_rank(const CountTicket& t) {
+  return (uint32_t)(__shfl(t.base, t.head) + (int)lane_id() - t.head);
 }
 
 // ================================================================== keys of the caller order
@@ -144,9 +186,10 @@ __global__ __launch_bounds__(256) void k_keys(SceneTable T, const float* __restr
   const DevParams& P = T.params[b.s];
   const int j = b.j;
   int oob = 0;
+  int c[3];
   if (j < b.end)
     keys[j] = (uint32_t)T.node_off[b.s] +
-              cell_key(P, thr + T.thr_off[b.s], st[PX * cap + j], st[(PX + 1) * cap + j], st[(PX + 2) * cap + j], oob);
+              cell_key(P, thr + T.thr_off[b.s], st[PX * cap + j], st[(PX + 1) * cap + j], st[(PX + 2) * cap + j], oob, c);
   if (__ballot(oob) && lane_id() == 0) atomicOr(status, MPM_STATUS_OUT_OF_DOMAIN);
 }
 
@@ -176,17 +219,10 @@ __global__ __launch_bounds__(256) void k_stress_init(SceneTable T, float* __rest
 // preceding blocks (blocks take tickets in start order, so a block only waits on running blocks).
 constexpr uint32_t FLAG_AGG = 1u << 30, FLAG_PREFIX = 2u << 30, VALUE_MASK = (1u << 30) - 1u;
 
-__global__ __launch_bounds__(256) void k_reset(uint32_t* __restrict__ zero_words, int64_t n_zero,
-                                               const int* __restrict__ counters, const int* __restrict__ active_tiles,
-                                               int* __restrict__ tile_slot, const int* __restrict__ active_blocks,
-                                               int* __restrict__ block_slot, const Clock* clk) {
+__global__ __launch_bounds__(256) void k_reset(uint32_t* __restrict__ zero_words, int64_t n_zero, const Clock* clk) {
   if (clock_skip(clk)) return;
-  int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  for (int64_t i = t0; i < n_zero; i += stride) zero_words[i] = 0u;
-  int nt = counters[CNT_TILES], nb = counters[CNT_BLOCKS];
-  for (int64_t j = t0; j < nt; j += stride) tile_slot[active_tiles[j]] = -1;
-  for (int64_t j = t0; j < nb; j += stride) block_slot[active_blocks[j]] = -1;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_zero; i += stride) zero_words[i] = 0u;
 }
 
 // Lanes of a wave that share a digit are grouped with 8 ballots; one lane per group adds the count.
@@ -365,78 +401,52 @@ __global__ __launch_bounds__(256) void k_sort_pass(const uint32_t* __restrict__ 
 }
 
 // ------------------------------------------------------------------ one-digit counting sort
-// The cell key itself is the single digit: count the particles of every cell (atomic ranks, in
-// no particular order), scan the counts into cell offsets, scatter the caller ids into their
-// cells, then order each cell by caller id (the rank of id i in its cell is the number of smaller
-// ids there). The result equals the LSD passes' stable sort bit for bit. The count and the scatter
-// run over physical slots, where the previous sort left the particles in cell order: the keys are
-// read in order, lanes of a wave share few distinct keys, and the scatter's writes land close to
-// where they are read; the scatter keeps each id's slot beside it, so that the rank pass finds the
-// particle's key and slot without gathering by caller id.
-//
-// Counting: the lanes of a wave that share a key are grouped first (leader = the lowest such lane);
-// then every leader adds its group's size with one atomic, all leaders in the same instruction, so
-// a wave waits for one atomic round trip.
-//
-// With `reset` set (the counting sort, which has no k_reset launch) the kernel also does k_reset's
-// work: it returns the previous substep's active tiles and node blocks to -1. The counters those
-// lists are read with are zeroed by k_cell_scan.
-__global__ __launch_bounds__(256) void k_cell_count(const uint32_t* __restrict__ keys, int n, int* __restrict__ cnt,
-                                                    uint32_t* __restrict__ rank, ResetArgs r, int reset,
-                                                    uint32_t* __restrict__ occ, uint32_t* __restrict__ occ_clear,
-                                                    int nocc, const Clock* clk) {
-  if (clock_skip(clk)) return;
-  // the key is loaded first, so that its round trip overlaps the reset's
+// The cell key itself is the single digit: the particles of every cell are counted where they are moved
+// (count_wave: atomic ranks, in no particular order), the counts are scanned into cell offsets, the caller
+// ids are scattered into their cells, and each cell is ordered by caller id (the rank of id i in its cell is
+// the number of smaller ids there). The result equals the LSD passes' stable sort bit for bit. The count and
+// the scatter run over physical slots, where the previous sort left the particles in cell order: lanes of a
+// wave share few distinct keys, and the scatter's writes land close to where they are read; the scatter keeps
+// each id's slot beside it, so that the rank pass finds the particle's key and slot without gathering by
+// caller id.
+__global__ __launch_bounds__(256) void k_clear_counts(BinCounts b, int64_t nscan, int64_t ntiles, int64_t ncells,
+                                                      int* __restrict__ counters) {
+  const int64_t stride = (int64_t)gridDim.x * 256, t0 = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  for (int64_t q = t0; q < nscan; q += stride) b.scan_flag[q] = 0;
+  for (int64_t q = t0; q < ntiles; q += stride) b.tile_flag[q] = 0;
+  for (int64_t q = t0; q < ncells; q += stride) b.cell_count[q] = 0;
+  if (t0 < 2) counters[t0] = 0;
+}
+
+// The counts of particles by their keys (those that no G2P has counted).
+__global__ __launch_bounds__(256) void k_cell_count(SceneTable T, BinCounts b, const uint32_t* __restrict__ keys, int n) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   const bool valid = i < n;
   const uint32_t key = valid ? keys[i] : 0u;
-  // the previous substep's block flags (its P2G has run) start clean for the next one
-  for (int q = i; q < nocc; q += gridDim.x * 256) occ_clear[q] = 0u;
-  if (reset) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    for (int64_t q = t0; q < r.n_zero; q += stride) r.zero_words[q] = 0u;
-    const int nt = r.counters[CNT_TILES], nb = r.counters[CNT_BLOCKS];
-    for (int64_t q = t0; q < nt; q += stride) r.tile_slot[r.active_tiles[q]] = -1;
-    for (int64_t q = t0; q < nb; q += stride) r.block_slot[r.active_blocks[q]] = -1;
-  }
-  const int lane = (int)lane_id();
-  const uint64_t lt = (1ull << lane) - 1ull;
-  uint64_t todo = __ballot(valid);
-  int leader = lane, group = 0, within = 0;
-  while (todo) {
-    const int first = __ffsll((long long)todo) - 1;
-    const uint32_t k0 = (uint32_t)__shfl((int)key, first);
-    const uint64_t peers = __ballot(valid && key == k0);
-    if (valid && key == k0) {
-      leader = first;
-      group = __popcll(peers);
-      within = __popcll(peers & lt);
-    }
-    todo &= ~peers;
-  }
-  int base = 0;
-  if (valid && leader == lane) {
-    base = atomicAdd(&cnt[key], group);
-    occ[key / SCAN_TILE] = 1u;
-  }
-  base = __shfl(base, leader);
-  if (valid) rank[i] = (uint32_t)(base + within);
+  const int sc = scene_of(T.node_off, T.nscenes, (int64_t)key);
+  const DevParams& P = T.params[sc];
+  const uint32_t lk = key - (uint32_t)T.node_off[sc];
+  const int r01 = P.res[0] * P.res[1];
+  const int c2 = (int)(lk / (uint32_t)r01), rem = (int)(lk % (uint32_t)r01);
+  const int c1 = rem / P.res[0], c0 = rem % P.res[0];
+  const CountTicket t = count_wave(b, valid, key, T.tile_off[sc] + tile_of(P, c0, c1, c2));
+  const uint32_t r = count_rank(t);
+  if (valid) b.rank[i] = r;
 }
 
-// Total of each scan block's SCAN_TILE cell counts (the blocks are independent).
-__global__ __launch_bounds__(256) void k_scan_sums(const int* __restrict__ cnt, int64_t ncells, uint32_t* __restrict__ agg,
-                                                   const uint32_t* __restrict__ occ, const Clock* clk) {
-  if (clock_skip(clk)) return;
+// Total of a scan block's SCAN_TILE cell counts (the blocks are independent).
+__device__ __forceinline__ void sum_block(const SortBufs& a, int b) {
   __shared__ uint32_t s_wsum[4];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  if (!occ[blockIdx.x]) {  // no particle in the block's cells: nothing to read
-    if (tid == 0) agg[blockIdx.x] = 0u;
+  if (tid == 0) a.scan_flag_clear[b] = 0;
+  if (!a.bins.scan_flag[b]) {  // no particle in the block's cells: nothing to read
+    if (tid == 0) a.scan_sum[b] = 0u;
     return;
   }
-  const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)tid * SCAN_IPT;
+  const int* cnt = a.bins.cell_count;
+  const int64_t base = (int64_t)b * SCAN_TILE + (int64_t)tid * SCAN_IPT;
   uint32_t t = 0;
-  if (base + SCAN_IPT <= ncells) {
+  if (base + SCAN_IPT <= a.ncells) {
     const int4* p4 = reinterpret_cast<const int4*>(cnt + base);
 #pragma unroll
     for (int q = 0; q < SCAN_IPT / 4; ++q) {
@@ -445,35 +455,110 @@ __global__ __launch_bounds__(256) void k_scan_sums(const int* __restrict__ cnt, 
     }
   } else {
     for (int q = 0; q < SCAN_IPT; ++q)
-      if (base + q < ncells) t += (uint32_t)cnt[base + q];
+      if (base + q < a.ncells) t += (uint32_t)cnt[base + q];
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off);
   if (lane == 0) s_wsum[w] = t;
   __syncthreads();
-  if (tid == 0) agg[blockIdx.x] = s_wsum[0] + s_wsum[1] + s_wsum[2] + s_wsum[3];
+  if (tid == 0) a.scan_sum[b] = s_wsum[0] + s_wsum[1] + s_wsum[2] + s_wsum[3];
+}
+
+// Thread per tile t (tiles and node blocks share one index space). A flagged tile receives the
+// next slot of the active tile list. Node block t is active when any of its 27 neighbour tiles is
+// (the 7x7x7-node P2G footprint of those tiles covers it) and receives the next slot of the active
+// block list. A workgroup takes one atomic per list. Slot numbers depend on the order in which waves
+// run; no result depends on them. The other buffer's flags are cleared.
+__device__ __forceinline__ void claim_block(const SortBufs& a, int b) {
+  __shared__ int s_cnt[2][4];
+  __shared__ int s_base[2];
+  const int64_t t = (int64_t)b * 256 + threadIdx.x;
+  bool tile_on = false, block_on = false;
+  if (t < a.ntiles) {
+    const int sc = scene_of(a.T.tile_off, a.T.nscenes, (int)t);
+    const int* tl = a.T.params[sc].tiles;
+    const int off = a.T.tile_off[sc], lt = (int)t - off;
+    const int t0 = lt % tl[0], t1 = (lt / tl[0]) % tl[1], t2 = lt / (tl[0] * tl[1]);
+    uint8_t v[27];
+#pragma unroll
+    for (int q = 0; q < 27; ++q) {  // all 27 loads issued together
+      const int b0 = t0 + q % 3 - 1, b1 = t1 + (q / 3) % 3 - 1, b2 = t2 + q / 9 - 1;
+      const bool in = b0 >= 0 && b1 >= 0 && b2 >= 0 && b0 < tl[0] && b1 < tl[1] && b2 < tl[2];
+      v[q] = in ? a.bins.tile_flag[off + (b2 * tl[1] + b1) * tl[0] + b0] : 0;
+    }
+    tile_on = v[13] != 0;
+#pragma unroll
+    for (int q = 0; q < 27; ++q) block_on |= v[q] != 0;
+  }
+  const uint64_t mt = __ballot(tile_on), mb = __ballot(block_on);
+  const int lane = (int)lane_id(), w = (int)threadIdx.x >> 6;
+  if (lane == 0) {
+    s_cnt[0][w] = __popcll(mt);
+    s_cnt[1][w] = __popcll(mb);
+  }
+  __syncthreads();
+  // one atomic per list and workgroup (a single counter takes many device-scope atomics slowly across XCDs)
+  if (threadIdx.x < 2) {
+    const int k = (int)threadIdx.x;
+    const int total = s_cnt[k][0] + s_cnt[k][1] + s_cnt[k][2] + s_cnt[k][3];
+    s_base[k] = total ? atomicAdd(&a.counters[k == 0 ? CNT_TILES : CNT_BLOCKS], total) : 0;
+  }
+  __syncthreads();
+  const uint64_t below = (1ull << lane) - 1ull;
+  int slot_t = -1, slot_b = -1;
+  if (tile_on) {
+    int base = s_base[0];
+    for (int k = 0; k < w; ++k) base += s_cnt[0][k];
+    slot_t = base + __popcll(mt & below);
+    a.active_tiles[slot_t] = (int)t;
+  }
+  if (block_on) {
+    int base = s_base[1];
+    for (int k = 0; k < w; ++k) base += s_cnt[1][k];
+    slot_b = base + __popcll(mb & below);
+    a.active_blocks[slot_b] = (int)t;
+  }
+  if (t < a.ntiles) {
+    a.tile_slot[t] = slot_t;
+    a.block_slot[t] = slot_b;
+    a.tile_flag_clear[t] = 0;
+  }
+}
+
+// The scan blocks' totals (workgroups below nscan) and the tile lists (the others): independent of each other,
+// so one launch hides one's latency behind the other's. With the counts made by G2P a substep sorts in four
+// launches (this one, scan, scatter, rank) where a separate count, totals and claim took six: sort 117 -> 83 us and
+// G2P 356 -> 386 at 2^22 particles, sort 30 -> 22 us and G2P unchanged at 2^15.
+__global__ __launch_bounds__(256) void k_sums_claim(SortBufs a, int nscan) {
+  if (clock_skip(a.clk)) return;
+  const int b = (int)blockIdx.x;
+  if (b < nscan) {
+    if (b == 0 && threadIdx.x < 2) {
+      a.counters_clear[threadIdx.x] = 0;
+      a.counters_misc[threadIdx.x] = 0;
+    }
+    sum_block(a, b);
+  } else {
+    claim_block(a, b - nscan);
+  }
 }
 
 // Exclusive scan of the cell counts into cell_start[0 .. ncells]: block b starts at the sum of the
-// totals of the blocks before it (read and summed by the block itself) and scans its SCAN_TILE
-// cells; the blocks are independent. A block without particles writes nothing: its cells are
-// empty, which every reader learns from occ (the getter of the bins fills them, k_fill_bins). A
+// totals of the blocks before it (read and summed by the block itself) and scans its SCAN_TILE cells; the blocks are independent. A block without particles writes nothing: its cells are
+// empty, which every reader learns from scan_flag (the getter of the bins fills them, k_fill_bins). A
 // block with particles also writes the start of the next block's first cell (its own end), which
 // the next block, if it has particles, writes with the same value. The last block writes
 // cell_start[ncells].
-// Block 0 also zeroes the substep's counters (active tiles and node blocks, candidates, apex
-// projections), which k_cell_count has read.
 __global__ __launch_bounds__(256) void k_cell_scan(const int* __restrict__ cnt, int64_t ncells, int* __restrict__ cell_start,
-                                                   const uint32_t* __restrict__ agg, const uint32_t* __restrict__ occ,
-                                                   int* __restrict__ counters, const Clock* clk) {
+                                                   const uint32_t* __restrict__ agg, const uint8_t* __restrict__ flag,
+                                                   const Clock* clk) {
   if (clock_skip(clk)) return;
-  if (blockIdx.x == 0 && threadIdx.x < CNT_NUM) counters[threadIdx.x] = 0;
   __shared__ uint32_t s_wsum[4];
   __shared__ uint32_t s_boff[4];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   const int b = blockIdx.x;
   const bool last = (int64_t)(b + 1) * SCAN_TILE >= ncells;
-  if (!occ[b] && !last) return;
+  if (!flag[b] && !last) return;
   {
     uint32_t p = 0;
     for (int q = tid; q < b; q += 256) p += agg[q];
@@ -583,16 +668,16 @@ __global__ __launch_bounds__(256) void k_cell_scatter(const uint32_t* __restrict
 // Thread per sorted position: the caller id placed there by the scatter moves to its stable rank
 // within the cell (a cell of c particles costs c comparisons per particle). It also does the bin
 // pass's work (k_bounds) for its new position: src = the particle's physical slot, and the cell's
-// first particle clears the cell's count and flags the cell's tile.
+// first particle clears the cell's count.
 // The workgroup first copies the ids of its 256 positions and RANK_HALO on either side into LDS (one
 // coalesced round trip): a cell of at most RANK_HALO particles around any of its positions lies in
 // that window, and its ids are compared there; a larger cell reads them from global memory.
 constexpr int RANK_HALO = 64;
-__global__ __launch_bounds__(256) void k_cell_rank(SceneTable T, const uint32_t* __restrict__ keys,
-                                                   const int* __restrict__ tmp, const int* __restrict__ tslot, int n,
+__global__ __launch_bounds__(256) void k_cell_rank(const uint32_t* __restrict__ keys, const int* __restrict__ tmp,
+                                                   const int* __restrict__ tslot, int n,
                                                    const int* __restrict__ cell_start, uint32_t* __restrict__ ks,
-                                                   int* __restrict__ vs, int* __restrict__ cnt,
-                                                   int* __restrict__ tile_slot, int* __restrict__ src, const Clock* clk) {
+                                                   int* __restrict__ vs, int* __restrict__ cnt, int* __restrict__ src,
+                                                   const Clock* clk) {
   if (clock_skip(clk)) return;
   constexpr int WIN = 256 + 2 * RANK_HALO;
   __shared__ int s_ids[WIN];
@@ -629,101 +714,22 @@ __global__ __launch_bounds__(256) void k_cell_rank(SceneTable T, const uint32_t*
   vs[d] = i;
   ks[d] = k;
   src[d] = pi;
-  if (r != 0) return;
-  cnt[k] = 0;
-  const int sc = scene_of(T.part_off, T.nscenes, i);
-  const DevParams& P = T.params[sc];
-  const uint32_t lk = k - (uint32_t)T.node_off[sc];
-  const int r01 = P.res[0] * P.res[1];
-  const int c2 = (int)(lk / (uint32_t)r01), rem = (int)(lk % (uint32_t)r01);
-  const int c1 = rem / P.res[0], c0 = rem % P.res[0];
-  tile_slot[T.tile_off[sc] + ((c2 >> 2) * P.tiles[1] + (c1 >> 2)) * P.tiles[0] + (c0 >> 2)] = -2;
+  if (r == 0) cnt[k] = 0;
 }
 
-// ================================================================== bins and tiles
-// Thread per sorted position: the first position of each run of equal keys clears the cell's count
-// for the next substep and flags the cell's tile (plain stores of one value).
+// ================================================================== bins
+// Thread per sorted position (the digit passes only): src = the particle's physical slot; the first position of
+// each run of equal keys clears the cell's count for the next substep.
 __global__ __launch_bounds__(256) void k_bounds(SceneTable T, const uint32_t* __restrict__ ks, int n,
-                                                int* __restrict__ cnt, int* __restrict__ tile_slot,
-                                                const int* __restrict__ perm, const int* __restrict__ pos,
-                                                int* __restrict__ src, const Clock* clk) {
+                                                int* __restrict__ cnt, const int* __restrict__ perm,
+                                                const int* __restrict__ pos, int* __restrict__ src, const Clock* clk) {
   if (clock_skip(clk)) return;
   const PBlock b = particle_block(T);  // sorted positions are scene-major as well
   const int j = b.j;
   if (j >= b.end) return;
-  const DevParams& P = T.params[b.s];
   src[j] = clamp_index(pos[clamp_index(perm[j], n)], n);
   const uint32_t k = ks[j];
-  if (j != 0 && ks[j - 1] == k) return;
-  cnt[k] = 0;
-  const uint32_t lk = k - (uint32_t)T.node_off[b.s];
-  const int r01 = P.res[0] * P.res[1];
-  const int c2 = (int)(lk / (uint32_t)r01), rem = (int)(lk % (uint32_t)r01);
-  const int c1 = rem / P.res[0], c0 = rem % P.res[0];
-  tile_slot[T.tile_off[b.s] + ((c2 >> 2) * P.tiles[1] + (c1 >> 2)) * P.tiles[0] + (c0 >> 2)] = -2;
-}
-
-// Thread per tile t (tiles and node blocks share one index space). A flagged tile (-2) receives the
-// next slot of the active tile list. Node block t is active when any of its 27 neighbour tiles is
-// (the 7x7x7-node P2G footprint of those tiles covers it) and receives the next slot of the active
-// block list. A workgroup takes one atomic per list. While one thread reads a neighbour's entry,
-// another workgroup may be turning its -2 into a slot: both values mean "active", so the result does
-// not depend on the timing. Slot numbers depend on the order in which waves run; no result depends
-// on them.
-__global__ __launch_bounds__(256) void k_claim(SceneTable T, int64_t count, int* __restrict__ tile_slot,
-                                               int* __restrict__ active_tiles, int* __restrict__ block_slot,
-                                               int* __restrict__ active_blocks, int* __restrict__ counters,
-                                               const Clock* clk) {
-  if (clock_skip(clk)) return;
-  __shared__ int s_cnt[2][4];
-  __shared__ int s_base[2];
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  bool tile_on = false, block_on = false;
-  if (t < count) {
-    const int sc = scene_of(T.tile_off, T.nscenes, (int)t);
-    const int* tl = T.params[sc].tiles;
-    const int off = T.tile_off[sc], lt = (int)t - off;
-    const int t0 = lt % tl[0], t1 = (lt / tl[0]) % tl[1], t2 = lt / (tl[0] * tl[1]);
-    int v[27];
-#pragma unroll
-    for (int q = 0; q < 27; ++q) {  // all 27 loads issued together
-      const int b0 = t0 + q % 3 - 1, b1 = t1 + (q / 3) % 3 - 1, b2 = t2 + q / 9 - 1;
-      const bool in = b0 >= 0 && b1 >= 0 && b2 >= 0 && b0 < tl[0] && b1 < tl[1] && b2 < tl[2];
-      v[q] = in ? tile_slot[off + (b2 * tl[1] + b1) * tl[0] + b0] : -1;
-    }
-    tile_on = v[13] == -2;  // only this thread writes tile t
-#pragma unroll
-    for (int q = 0; q < 27; ++q) block_on |= v[q] != -1;
-  }
-  const uint64_t mt = __ballot(tile_on), mb = __ballot(block_on);
-  const int lane = (int)lane_id(), w = (int)threadIdx.x >> 6;
-  if (lane == 0) {
-    s_cnt[0][w] = __popcll(mt);
-    s_cnt[1][w] = __popcll(mb);
-  }
-  __syncthreads();
-  // one atomic per list and workgroup (a single counter takes many device-scope atomics slowly across XCDs)
-  if (threadIdx.x < 2) {
-    const int k = (int)threadIdx.x;
-    const int total = s_cnt[k][0] + s_cnt[k][1] + s_cnt[k][2] + s_cnt[k][3];
-    s_base[k] = total ? atomicAdd(&counters[k == 0 ? CNT_TILES : CNT_BLOCKS], total) : 0;
-  }
-  __syncthreads();
-  const uint64_t below = (1ull << lane) - 1ull;
-  if (tile_on) {
-    int base = s_base[0];
-    for (int k = 0; k < w; ++k) base += s_cnt[0][k];
-    const int slot = base + __popcll(mt & below);
-    tile_slot[t] = slot;
-    active_tiles[slot] = (int)t;
-  }
-  if (block_on) {
-    int base = s_base[1];
-    for (int k = 0; k < w; ++k) base += s_cnt[1][k];
-    const int slot = base + __popcll(mb & below);
-    block_slot[t] = slot;
-    active_blocks[slot] = (int)t;
-  }
+  if (j == 0 || ks[j - 1] != k) cnt[k] = 0;
 }
 
 // ================================================================== P2G
@@ -1930,8 +1936,20 @@ __global__ __launch_bounds__(256) void k_g2p(G2PArgs a) {
         }
       }
     }
-    // cloth vertices and elements keep only the skew part of B (damping 1, HybridSolver.cpp:926-932)
+    float xn[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      xn[d] = xp[d] + dt * vb[d];
+      if (fabsf(xn[d] - xp[d]) > P.h[d]) cfl = 1;
+    }
+    // the next sort's key and counts (of a cloth element: k_cloth_elements, which moves it to its vertices);
+    // the atomics are in flight during the return map
     const int kind = particle_kind(P, pid);
+    int cell[3];
+    const uint32_t key = (uint32_t)noff + cell_key(P, a.thr + a.T.thr_off[pb.s], xn[0], xn[1], xn[2], oob, cell);
+    const CountTicket ticket =
+        count_wave(a.bins, kind != KIND_ELEMENT, key, a.T.tile_off[pb.s] + tile_of(P, cell[0], cell[1], cell[2]));
+    // cloth vertices and elements keep only the skew part of B (damping 1, HybridSolver.cpp:926-932)
     const float damping = kind == KIND_PARTICLE ? P.damping : 1.0f;
     if (damping != 0.0f) {
       float C[9];
@@ -1988,12 +2006,6 @@ __global__ __launch_bounds__(256) void k_g2p(G2PArgs a) {
         a.apex_usv[(CAND_V + k) * n + r] = io.V[k];
       }
     }
-    float xn[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      xn[d] = xp[d] + dt * vb[d];
-      if (fabsf(xn[d] - xp[d]) > P.h[d]) cfl = 1;
-    }
     float* so = a.sout;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -2015,7 +2027,9 @@ __global__ __launch_bounds__(256) void k_g2p(G2PArgs a) {
     so[PPHI * cap + j] = phi_p;
     reinterpret_cast<int*>(so + (size_t)PID * cap)[j] = pid;
     if (a.pos_out) a.pos_out[pid] = j;
-    a.keys[j] = (uint32_t)noff + cell_key(P, a.thr + a.T.thr_off[pb.s], xn[0], xn[1], xn[2], oob);
+    a.keys[j] = key;
+    const uint32_t rank = count_rank(ticket);
+    if (kind != KIND_ELEMENT) a.bins.rank[j] = rank;
     bad = !(isfinite(xn[0]) && isfinite(xn[1]) && isfinite(xn[2]) && isfinite(vp[0]) && isfinite(vp[1]) &&
             isfinite(vp[2]) && isfinite(Fh[0]) && isfinite(Fh[4]) && isfinite(Fh[8]) && isfinite(plastic));
   }
@@ -2459,7 +2473,11 @@ __global__ __launch_bounds__(256) void k_cloth_elements(ClothArgs a) {
     cloth_return_map(P, D, fb);
 #pragma unroll
     for (int i = 0; i < 9; ++i) a.st[(PF + i) * a.cap + pe] = D[i];
-    a.keys[pe] = cell_key(P, a.thr, xe[0], xe[1], xe[2], oob);
+    int cell[3];
+    const uint32_t key = cell_key(P, a.thr, xe[0], xe[1], xe[2], oob, cell);
+    const CountTicket ticket = count_wave(a.bins, true, key, tile_of(P, cell[0], cell[1], cell[2]));
+    a.keys[pe] = key;
+    a.bins.rank[pe] = count_rank(ticket);
   }
   if (fb) atomicAdd(a.fallback, (unsigned long long)fb);
   if (oob) atomicOr(a.status, MPM_STATUS_OUT_OF_DOMAIN);
@@ -2594,29 +2612,32 @@ void launch_stress_init(hipStream_t s, const SceneTable& T, int nblocks, float* 
   if (n > 0) hipLaunchKernelGGL(k_stress_init, dim3(nblocks), dim3(256), 0, s, T, st, cap, n, fallback);
 }
 
-void launch_sort(hipStream_t s, const SortBufs& b, const uint32_t* keys_in, int n, int passes, int mode) {
+void launch_count(hipStream_t s, const SceneTable& T, const BinCounts& b, const uint32_t* keys, int n, int64_t ncells,
+                  int64_t ntiles, int* counters, bool dirty) {
+  const int64_t nscan = blocks_for(ncells, SCAN_TILE), work = dirty ? ncells : std::max(nscan, ntiles);
+  hipLaunchKernelGGL(k_clear_counts, dim3(std::min(4096, blocks_for(work, 256))), dim3(256), 0, s, b, nscan, ntiles,
+                     dirty ? ncells : 0, counters);
+  if (n > 0) hipLaunchKernelGGL(k_cell_count, dim3(blocks_for(n, 256)), dim3(256), 0, s, T, b, keys, n);
+}
+
+void launch_sort(hipStream_t s, const SortBufs& b, const uint32_t* keys_in, int n, int nblocks, int passes, int mode) {
   if (n <= 0) return;
-  {
-    // bins: counts (the rank is used by the counting sort) and their scan, in both modes
-    uint32_t* rank = (passes & 1) ? b.k2 : b.k1;
-    const int nscan = blocks_for(b.ncells, SCAN_TILE);
-    hipLaunchKernelGGL(k_cell_count, dim3(blocks_for(n, 256)), dim3(256), 0, s, keys_in, n, b.cell_count, rank,
-                       b.reset, mode == SORT_COUNTING ? 1 : 0, b.occ, b.occ_clear, nscan, b.clk);
-    hipLaunchKernelGGL(k_scan_sums, dim3(nscan), dim3(256), 0, s, b.cell_count, b.ncells, b.scan_agg, b.occ, b.clk);
-    hipLaunchKernelGGL(k_cell_scan, dim3(nscan), dim3(256), 0, s, b.cell_count, b.ncells, b.cell_start, b.scan_agg,
-                       b.occ, b.counters, b.clk);
-  }
+  const int nscan = blocks_for(b.ncells, SCAN_TILE);
+  hipLaunchKernelGGL(k_sums_claim, dim3(nscan + blocks_for(b.ntiles, 256)), dim3(256), 0, s, b, nscan);
+  hipLaunchKernelGGL(k_cell_scan, dim3(nscan), dim3(256), 0, s, b.bins.cell_count, b.ncells, b.cell_start, b.scan_sum,
+                     b.bins.scan_flag, b.clk);
   if (mode == SORT_COUNTING) {
     uint32_t* kf = (passes & 1) ? b.k1 : b.k2;  // the result goes where the digit passes put it
     int* vf = (passes & 1) ? b.v1 : b.v2;
-    const uint32_t* rank = (passes & 1) ? b.k2 : b.k1;
     int* tmp = (passes & 1) ? b.v2 : b.v1;
-    hipLaunchKernelGGL(k_cell_scatter, dim3(blocks_for(n, 256)), dim3(256), 0, s, keys_in, rank, n, b.cell_start, b.pid,
-                       tmp, b.tslot, b.clk);
-    hipLaunchKernelGGL(k_cell_rank, dim3(blocks_for(n, 256)), dim3(256), 0, s, b.T, keys_in, tmp, b.tslot, n,
-                       b.cell_start, kf, vf, b.cell_count, b.tile_slot, b.src, b.clk);
+    hipLaunchKernelGGL(k_cell_scatter, dim3(blocks_for(n, 256)), dim3(256), 0, s, keys_in, b.bins.rank, n, b.cell_start,
+                       b.pid, tmp, b.tslot, b.clk);
+    hipLaunchKernelGGL(k_cell_rank, dim3(blocks_for(n, 256)), dim3(256), 0, s, keys_in, tmp, b.tslot, n, b.cell_start,
+                       kf, vf, b.bins.cell_count, b.src, b.clk);
     return;
   }
+  hipLaunchKernelGGL(k_reset, dim3(std::min(4096, blocks_for(b.radix_words, 256))), dim3(256), 0, s, b.hist,
+                     b.radix_words, b.clk);
   // the digit passes are stable in their input order, which must be the caller order: the keys
   // (by physical slot) go to caller order first, and the caller id -> slot map comes with them
   uint32_t* kc = reinterpret_cast<uint32_t*>(b.tslot);
@@ -2633,31 +2654,12 @@ void launch_sort(hipStream_t s, const SortBufs& b, const uint32_t* keys_in, int 
     kin = ko;
     vin = vo;
   }
+  hipLaunchKernelGGL(k_bounds, dim3(nblocks), dim3(256), 0, s, b.T, kin, n, b.bins.cell_count, vin, b.pos, b.src, b.clk);
 }
 
 void launch_fill_bins(hipStream_t s, const uint32_t* ks, int n, int64_t ncells, int* cell_start) {
   if (ncells <= 0) return;
   hipLaunchKernelGGL(k_fill_bins, dim3(blocks_for(ncells + 1, 256)), dim3(256), 0, s, ks, n, ncells, cell_start);
-}
-
-void launch_reset(hipStream_t s, const ResetArgs& r) {
-  int64_t work = r.n_zero;
-  if (work < r.max_tiles) work = r.max_tiles;
-  int grid = blocks_for(work, 256);
-  if (grid > 4096) grid = 4096;
-  if (grid < 1) grid = 1;
-  hipLaunchKernelGGL(k_reset, dim3(grid), dim3(256), 0, s, r.zero_words, r.n_zero, r.counters, r.active_tiles,
-                     r.tile_slot, r.active_blocks, r.block_slot, r.clk);
-}
-
-void launch_bounds(hipStream_t s, const SceneTable& T, int nblocks, const uint32_t* ks, int n, int64_t ntiles,
-                   int* cell_count, int* tile_slot, int* active_tiles, int* block_slot, int* active_blocks,
-                   int* counters, const int* perm, const int* pos, int* src, const Clock* clk, int mode) {
-  if (n <= 0) return;
-  if (mode != SORT_COUNTING)  // the counting sort's rank kernel has done this pass
-    hipLaunchKernelGGL(k_bounds, dim3(nblocks), dim3(256), 0, s, T, ks, n, cell_count, tile_slot, perm, pos, src, clk);
-  hipLaunchKernelGGL(k_claim, dim3(blocks_for(ntiles, 256)), dim3(256), 0, s, T, ntiles, tile_slot, active_tiles,
-                     block_slot, active_blocks, counters, clk);
 }
 
 template <int RANKS>

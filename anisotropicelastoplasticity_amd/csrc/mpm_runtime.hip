@@ -82,13 +82,15 @@ struct mpm_ctx {
   float* thr = nullptr;      // per-axis cell thresholds
   float* grid = nullptr;     // m, mom(3), v(3), vbf(3)
   int* cell_start = nullptr;
-  int* cell_count = nullptr;  // per-cell particle counts of the counting sort (zero between substeps)
+  int* cell_count = nullptr;  // per-cell particle counts of the next sort (zero from a sort to the next G2P)
   int* cell_end = nullptr;  // cell_start + 1 (not a separate allocation)
-  // per scan block of cells: 1 where a cell holds a particle; two sets, used by alternate substeps
-  // (each substep's count clears the other set, whose P2G has run)
-  uint32_t* occ[2] = {nullptr, nullptr};
-  int occ_par = 0;
-  const uint32_t* occ_last = nullptr;  // the set of the last sort
+  // by state buffer: the scan blocks of cells and the tiles that hold particles (BinCounts)
+  uint8_t* scan_flag[2] = {nullptr, nullptr};
+  uint8_t* tile_flag[2] = {nullptr, nullptr};
+  uint32_t* scan_sum = nullptr;  // particles per scan block
+  // the counts of the particles in state[cur] are complete and not yet used by a sort (G2P has made them)
+  bool counted = false;
+  bool counts_dirty = false;  // cell_count holds counts that no sort will use
   int* tile_slot = nullptr;
   int* active_tiles = nullptr;
   int* block_slot = nullptr;
@@ -371,10 +373,7 @@ static float threshold(double gmin, double h, int c) {
 
 // Sort workspace words: 4 x 256 digit histograms, 4 digit-pass tickets and 4 cell-scan tickets, the
 // cell-scan look-back words (64-bit, one per scan block), then the digit passes' look-back words.
-static constexpr int64_t SORTWS_TICKETS = 1024, SORTWS_SCAN = 1032;
-// [SORTWS_SCAN, radix status): the scan blocks' totals
-static int64_t scan_blocks(const mpm_ctx* ctx) { return (ctx->ng + SCAN_TILE - 1) / SCAN_TILE; }
-static int64_t sortws_radix_status(const mpm_ctx* ctx) { return SORTWS_SCAN + scan_blocks(ctx) + 1; }
+static constexpr int64_t SORTWS_TICKETS = 1024, SORTWS_STATUS = 1032;
 
 // ------------------------------------------------------------------ substep stages
 // Rebuild pos[cur] from the id plane of state[cur] if G2P did not maintain it.
@@ -385,59 +384,68 @@ static void ensure_pos(mpm_ctx* ctx) {
   ctx->pos_ok = true;
 }
 
+// The counts belonging to state[b]; the ranks are where the sort leaves no result.
+static BinCounts bin_counts(mpm_ctx* ctx, int b) {
+  return {ctx->cell_count, (ctx->sort_passes & 1) ? ctx->k2 : ctx->k1, ctx->scan_flag[b], ctx->tile_flag[b]};
+}
+
+// The particles of state[cur] counted into their cells. A substep's G2P does so for the next one; after a
+// change of the particles or a sort that no G2P followed, the keys are counted here.
+static void ensure_counts(mpm_ctx* ctx) {
+  if (ctx->counted) return;
+  if (!ctx->keys_valid)
+    launch_keys(ctx->stream, ctx->T, ctx->nblocks_p, ctx->state[ctx->cur], ctx->cap, ctx->n, ctx->thr, ctx->keys, ctx->status);
+  launch_count(ctx->stream, ctx->T, bin_counts(ctx, ctx->cur), ctx->keys, ctx->n, ctx->ng, ctx->ntiles,
+               ctx->counters + 2 * ctx->cur, ctx->counts_dirty);
+  ctx->counted = true;
+  ctx->counts_dirty = false;
+}
+
+// The particles or the grid changed: keys and counts are made anew.
+static void drop_keys(mpm_ctx* ctx) {
+  ctx->keys_valid = false;
+  ctx->counts_dirty = ctx->counts_dirty || ctx->counted;
+  ctx->counted = false;
+}
+
 static int stage_sort(mpm_ctx* ctx) {
   hipStream_t s = ctx->stream;
   float* st = ctx->state[ctx->cur];
   if (ctx->mesh.ne > 0 || ctx->mesh.nv > 0) ensure_pos(ctx);  // the cloth kernels address by caller id
-  if (!ctx->keys_valid) launch_keys(s, ctx->T, ctx->nblocks_p, st, ctx->cap, ctx->n, ctx->thr, ctx->keys, ctx->status);
-  ResetArgs r;
-  if (ctx->sort_mode == SORT_COUNTING) {  // nothing to zero: the scan totals are overwritten
-    r.zero_words = ctx->sortws + SORTWS_TICKETS;
-    r.n_zero = 0;
-  } else {
-    r.zero_words = ctx->sortws;
-    r.n_zero = ctx->sortws_words;
-  }
-  r.counters = ctx->counters;
-  r.active_tiles = ctx->active_tiles;
-  r.tile_slot = ctx->tile_slot;
-  r.active_blocks = ctx->active_blocks;
-  r.block_slot = ctx->block_slot;
-  r.max_tiles = ctx->ntiles;
-  r.clk = ctx->clk_active;
-  // the counting sort's first kernel does the reset work itself (one launch fewer)
-  if (ctx->sort_mode != SORT_COUNTING) launch_reset(s, r);
+  ensure_counts(ctx);
   SortBufs b;
-  b.reset = r;
   b.k1 = ctx->k1;
   b.k2 = ctx->k2;
   b.v1 = ctx->v1;
   b.v2 = ctx->v2;
   b.hist = ctx->sortws;
   b.tickets = ctx->sortws + SORTWS_TICKETS;
-  b.scan_agg = ctx->sortws + SORTWS_SCAN;
-  b.status = ctx->sortws + sortws_radix_status(ctx);
-  b.cell_count = ctx->cell_count;
+  b.status = ctx->sortws + SORTWS_STATUS;
+  b.radix_words = ctx->sortws_words;
+  b.bins = bin_counts(ctx, ctx->cur);
+  b.scan_sum = ctx->scan_sum;
+  b.scan_flag_clear = ctx->scan_flag[1 - ctx->cur];
+  b.tile_flag_clear = ctx->tile_flag[1 - ctx->cur];
   b.cell_start = ctx->cell_start;
   b.ncells = ctx->ng;
+  b.ntiles = ctx->ntiles;
   b.T = ctx->T;
   b.tile_slot = ctx->tile_slot;
+  b.active_tiles = ctx->active_tiles;
+  b.block_slot = ctx->block_slot;
+  b.active_blocks = ctx->active_blocks;
   b.pid = reinterpret_cast<const int*>(st + (size_t)PID * ctx->cap);
   b.tslot = ctx->tslot;
   b.pos = ctx->pos[ctx->cur];
   b.src = ctx->src;
-  b.counters = ctx->counters;
+  b.counters = ctx->counters + 2 * ctx->cur;
+  b.counters_clear = ctx->counters + 2 * (1 - ctx->cur);
+  b.counters_misc = ctx->counters + CNT_CAND;
   b.clk = ctx->clk_active;
-  b.occ = ctx->occ[ctx->occ_par];
-  b.occ_clear = ctx->occ[1 - ctx->occ_par];
-  ctx->occ_last = b.occ;
-  ctx->occ_par = 1 - ctx->occ_par;
-  launch_sort(s, b, ctx->keys, ctx->n, ctx->sort_passes, ctx->sort_mode);
+  launch_sort(s, b, ctx->keys, ctx->n, ctx->nblocks_p, ctx->sort_passes, ctx->sort_mode);
   if (ctx->sort_mode != SORT_COUNTING) ctx->pos_ok = true;  // the radix mode's key conversion wrote pos[cur]
-  launch_bounds(s, ctx->T, ctx->nblocks_p, ctx->ks_sorted, ctx->n, ctx->ntiles, ctx->cell_count,
-                ctx->tile_slot, ctx->active_tiles, ctx->block_slot, ctx->active_blocks, ctx->counters, ctx->vs_sorted,
-                ctx->pos[ctx->cur], ctx->src, ctx->clk_active, ctx->sort_mode);
   ctx->sort_buf = ctx->cur;
+  ctx->counted = false;
   return MPM_OK;
 }
 
@@ -463,6 +471,7 @@ static ClothArgs cloth_args(mpm_ctx* ctx, int b) {
   c.nfixed = m.nfixed;
   c.gvel = reinterpret_cast<float4*>(ctx->grid + GRID_VEL * ctx->ng);
   c.keys = ctx->keys;
+  c.bins = bin_counts(ctx, b);
   c.thr = ctx->thr;
   c.status = ctx->status;
   c.fallback = ctx->fallbacks;
@@ -479,8 +488,8 @@ static P2GArgs p2g_args(mpm_ctx* ctx, float dt) {
   a.src = ctx->src;
   a.cell_start = ctx->cell_start;
   a.cell_end = ctx->cell_end;
-  a.occ = ctx->occ_last;
-  a.counters = ctx->counters;
+  a.occ = ctx->scan_flag[ctx->sort_buf];
+  a.counters = ctx->counters + 2 * ctx->sort_buf;
   a.active_tiles = ctx->active_tiles;
   a.partials = ctx->partials;
   a.gvel = reinterpret_cast<const float4*>(ctx->grid + GRID_VEL * ctx->ng);
@@ -497,7 +506,7 @@ static P2GArgs p2g_args(mpm_ctx* ctx, float dt) {
 static GridArgs grid_args(mpm_ctx* ctx, float dt) {
   GridArgs g;
   g.T = ctx->T;
-  g.counters = ctx->counters;
+  g.counters = ctx->counters + 2 * ctx->sort_buf;
   g.active_blocks = ctx->active_blocks;
   g.tile_slot = ctx->tile_slot;
   g.partials = ctx->partials;
@@ -530,7 +539,7 @@ static GridArgs grid_args(mpm_ctx* ctx, float dt) {
 static int choose_p2g(mpm_ctx* ctx) {
   if (ctx->p2g_tuned) return MPM_OK;
   int tiles = 0;
-  CK(hipMemcpyAsync(&tiles, ctx->counters + CNT_TILES, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+  CK(hipMemcpyAsync(&tiles, ctx->counters + CNT_TILES + 2 * ctx->sort_buf, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   CK(hipStreamSynchronize(ctx->stream));
   const bool layers = ctx->mesh.ne == 0 && tiles > ctx->n_cu && ctx->n <= 640LL * tiles;
   ctx->p2g_pass = layers ? P2G_LAYERS : P2G_ROWS;
@@ -586,6 +595,7 @@ static int stage_g2p(mpm_ctx* ctx, float dt) {
   a.write_stress = ctx->predicted ? 0 : 1;
   a.thr = ctx->thr;
   a.keys = ctx->keys;
+  a.bins = bin_counts(ctx, 1 - ctx->cur);
   a.status = ctx->status;
   a.fallback_svd = ctx->fallbacks;
   a.fallback_apex = ctx->fallbacks + 1;
@@ -668,6 +678,7 @@ static int stage_g2p(mpm_ctx* ctx, float dt) {
   if (ctx->clk_active) launch_clock_end(ctx->stream, ctx->clk_active);
   ctx->cur = 1 - ctx->cur;
   ctx->keys_valid = true;
+  ctx->counted = true;
   ctx->stress_valid = !ctx->predicted;
   ctx->pos_ok = a.pos_out != nullptr;
   ctx->substeps += 1;
@@ -793,7 +804,7 @@ int mpm_destroy(mpm_ctx* ctx) {
   drop_graphs(ctx);
   dfree(ctx->table_buf);
   drop_mesh(ctx);
-  dfree(ctx->thr); dfree(ctx->grid); dfree(ctx->cell_start); dfree(ctx->cell_count); dfree(ctx->occ[0]); dfree(ctx->occ[1]);
+  dfree(ctx->thr); dfree(ctx->grid); dfree(ctx->cell_start); dfree(ctx->cell_count); dfree(ctx->scan_sum); dfree(ctx->scan_flag[0]); dfree(ctx->scan_flag[1]); dfree(ctx->tile_flag[0]); dfree(ctx->tile_flag[1]);
   ctx->cell_end = nullptr;
   dfree(ctx->tile_slot); dfree(ctx->active_tiles); dfree(ctx->block_slot); dfree(ctx->active_blocks);
   dfree(ctx->partials);
@@ -824,7 +835,7 @@ static int alloc_partials(mpm_ctx* ctx) {
 static int alloc_sortws(mpm_ctx* ctx) {
   if (ctx->n <= 0) return MPM_OK;
   ctx->nb_sort = (ctx->n + SORT_TILE - 1) / SORT_TILE;
-  const int64_t words = sortws_radix_status(ctx) + (int64_t)ctx->sort_passes * ctx->nb_sort * 256;
+  const int64_t words = SORTWS_STATUS + (int64_t)ctx->sort_passes * ctx->nb_sort * 256;
   if (words != ctx->sortws_words || !ctx->sortws) {
     int rc = dalloc(ctx, ctx->sortws, words);
     if (rc) return rc;
@@ -897,9 +908,12 @@ static int layout(mpm_ctx* ctx) {
   int rc = dalloc(ctx, ctx->grid, (size_t)GRID_FLOATS * ng);
   if (!rc) rc = dalloc(ctx, ctx->cell_start, ng + 1);
   const int64_t nscan = (ng + SCAN_TILE - 1) / SCAN_TILE;
-  if (!rc) rc = dalloc(ctx, ctx->occ[0], (size_t)nscan);
-  if (!rc) rc = dalloc(ctx, ctx->occ[1], (size_t)nscan);
+  for (int b = 0; b < 2; ++b) {
+    if (!rc) rc = dalloc(ctx, ctx->scan_flag[b], (size_t)nscan);
+    if (!rc) rc = dalloc(ctx, ctx->tile_flag[b], (size_t)nt);
+  }
   if (!rc) rc = dalloc(ctx, ctx->cell_count, ng);
+  if (!rc) rc = dalloc(ctx, ctx->scan_sum, (size_t)nscan);
   if (!rc) rc = dalloc(ctx, ctx->tile_slot, nt);
   if (!rc) rc = dalloc(ctx, ctx->active_tiles, nt);
   if (!rc) rc = dalloc(ctx, ctx->block_slot, nt);
@@ -909,9 +923,10 @@ static int layout(mpm_ctx* ctx) {
   CK(hipMemsetAsync(ctx->grid, 0, sizeof(float) * GRID_FLOATS * ng, ctx->stream));
   ctx->cell_end = ctx->cell_start + 1;  // cell c holds sorted positions [cell_start[c], cell_start[c + 1])
   CK(hipMemsetAsync(ctx->cell_start, 0, sizeof(int) * (ng + 1), ctx->stream));
-  CK(hipMemsetAsync(ctx->occ[0], 0, sizeof(uint32_t) * nscan, ctx->stream));
-  CK(hipMemsetAsync(ctx->occ[1], 0, sizeof(uint32_t) * nscan, ctx->stream));
-  ctx->occ_last = ctx->occ[0];
+  for (int b = 0; b < 2; ++b) {
+    CK(hipMemsetAsync(ctx->scan_flag[b], 0, (size_t)nscan, ctx->stream));
+    CK(hipMemsetAsync(ctx->tile_flag[b], 0, (size_t)nt, ctx->stream));
+  }
   CK(hipMemsetAsync(ctx->cell_count, 0, sizeof(int) * ng, ctx->stream));
   launch_fill_int(ctx->stream, ctx->tile_slot, nt, -1);
   launch_fill_int(ctx->stream, ctx->block_slot, nt, -1);
@@ -923,7 +938,8 @@ static int layout(mpm_ctx* ctx) {
       for (int c = 0; c <= sc.res[a]; ++c) thr.push_back(threshold(sc.gmin[a], sc.h[a], c));
   CK(hipMemcpyAsync(ctx->thr, thr.data(), thr.size() * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
   ctx->have_grid = true;
-  ctx->keys_valid = false;
+  drop_keys(ctx);
+  ctx->counts_dirty = false;
   ctx->partial_slots = 0;
   pick_sorted(ctx);
   if (ctx->k1) CK(hipMemsetAsync(ctx->k1, 0, sizeof(uint32_t) * ctx->cap, ctx->stream));
@@ -1044,8 +1060,7 @@ static int install_state(mpm_ctx* ctx, int n, const std::vector<float>& h) {
   CK(hipStreamSynchronize(ctx->stream));
   ctx->stress_valid = false;
   ctx->cur = 0;
-  ctx->sort_buf = 0;
-  ctx->keys_valid = false;
+  drop_keys(ctx);
   ctx->substeps = 0;
   ctx->next_stage = MPM_STAGE_SORT;
   return MPM_OK;
@@ -1408,6 +1423,7 @@ int mpm_run(mpm_ctx* ctx, float dt, int32_t nsteps) {
       }
       rc = choose_p2g(ctx);
       if (rc) return rc;
+      ensure_counts(ctx);  // a captured pair starts at the scan of what the G2P before it counted
       hipGraph_t g = nullptr;
       const int64_t steps0 = ctx->substeps;
       const int sort0 = ctx->sort_buf;
@@ -1419,6 +1435,7 @@ int mpm_run(mpm_ctx* ctx, float dt, int32_t nsteps) {
       ctx->substeps = steps0;
       ctx->cur = c0;
       ctx->sort_buf = sort0;
+      ctx->counted = true;
       if (r2 || ec != hipSuccess) {
         if (g) (void)hipGraphDestroy(g);
         if (r2) return r2;
@@ -1430,6 +1447,7 @@ int mpm_run(mpm_ctx* ctx, float dt, int32_t nsteps) {
       ctx->graph_dt[c0] = dt;
       ctx->cur = c0;  // capture did not execute anything
     }
+    ensure_counts(ctx);
     for (int i = 0; i < pairs; ++i) CK(hipGraphLaunch(ctx->graph[c0], ctx->stream));
     ctx->substeps += 2 * pairs;
     ctx->sort_buf = 1 - c0;
@@ -1494,6 +1512,7 @@ int mpm_solve(mpm_ctx* ctx, double cfl, double maxt, mpm_frame_callback cb, void
       if (!ctx->graph_adapt[c0]) {
         rc = choose_p2g(ctx);
         if (rc) return rc;
+        ensure_counts(ctx);
         hipGraph_t gr = nullptr;
         const int64_t steps0 = ctx->substeps;
         const int sort0 = ctx->sort_buf;
@@ -1504,6 +1523,7 @@ int mpm_solve(mpm_ctx* ctx, double cfl, double maxt, mpm_frame_callback cb, void
         ctx->substeps = steps0;
         ctx->cur = c0;  // capture did not execute anything
         ctx->sort_buf = sort0;
+        ctx->counted = true;
         if (r2 || ec != hipSuccess) {
           if (gr) (void)hipGraphDestroy(gr);
           if (r2) return r2;
@@ -1513,6 +1533,7 @@ int mpm_solve(mpm_ctx* ctx, double cfl, double maxt, mpm_frame_callback cb, void
         (void)hipGraphDestroy(gr);
         if (ei != hipSuccess) return fail(ctx, MPM_ERR_HIP, std::string("graph instantiate: ") + hipGetErrorString(ei));
       }
+      ensure_counts(ctx);
       CK(hipGraphLaunch(ctx->graph_adapt[c0], ctx->stream));
       executed = -1;  // read back below
     }
@@ -1727,13 +1748,13 @@ int mpm_get_stats(mpm_ctx* ctx, mpm_stats* s) {
   std::memset(s, 0, sizeof(*s));
   s->substeps = ctx->substeps;
   s->n_particles = ctx->n;
-  int cnt[CNT_NUM] = {0, 0};
+  int cnt[CNT_NUM] = {};
   int status = 0;
   unsigned long long fb[4] = {0, 0, 0, 0};
   unsigned long long sc[4] = {0, 0, 0, 0};
   if (ctx->have_grid && ctx->n > 0) {
     CK(hipMemsetAsync(ctx->fallbacks + 2, 0, sizeof(unsigned long long), ctx->stream));
-    launch_count_nodes(ctx->stream, ctx->T, ctx->grid, ctx->counters, ctx->active_blocks, ctx->fallbacks + 2, ctx->grid_grid);
+    launch_count_nodes(ctx->stream, ctx->T, ctx->grid, ctx->counters + 2 * ctx->sort_buf, ctx->active_blocks, ctx->fallbacks + 2, ctx->grid_grid);
   }
   CK(hipMemcpyAsync(cnt, ctx->counters, sizeof(cnt), hipMemcpyDeviceToHost, ctx->stream));
   CK(hipMemcpyAsync(&status, ctx->status, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
@@ -1741,8 +1762,8 @@ int mpm_get_stats(mpm_ctx* ctx, mpm_stats* s) {
   CK(hipMemcpyAsync(sc, ctx->sur_counts, sizeof(sc), hipMemcpyDeviceToHost, ctx->stream));
   CK(hipStreamSynchronize(ctx->stream));
   s->status = status;
-  s->n_active_tiles = cnt[CNT_TILES];
-  s->n_active_blocks = cnt[CNT_BLOCKS];
+  s->n_active_tiles = cnt[CNT_TILES + 2 * ctx->sort_buf];
+  s->n_active_blocks = cnt[CNT_BLOCKS + 2 * ctx->sort_buf];
   s->n_active_nodes = (int64_t)fb[2];
   s->fp64_svd_count = (int64_t)fb[0];
   s->fp64_apex_count = (int64_t)fb[1];

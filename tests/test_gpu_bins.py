@@ -1,0 +1,117 @@
+"""GPU checks of the sort's bins, which each substep's G2P counts for the next one (a cloth's elements by the kernel
+that moves them). Whatever comes between two substeps - another sort, the other sort mode, new particles, a
+frame's end - the sorted order stays the stable order of the keys, and the state's bits do not change.
+The keys themselves are compared with floor((x - min) / h) in double at the cells' boundaries and beside them.
+"""
+import numpy as np
+import pytest
+
+from anisotropicelastoplasticity_amd import Solver, _lib, scenes
+
+pytestmark = pytest.mark.gpu
+
+KEYS = ("x", "v", "B", "F", "plastic")
+
+
+def _scene(kind):
+    if kind == "cloth":
+        return scenes.config3_cloth_sand(n_side=17, edge=1.0 / 60.0, sand_cells=(7, 5, 6))
+    return scenes.small_scene(_lib.SAND, 2, 0, _lib.FRICTION_STICKY, seed=9, res=(29, 31, 27), cells=(9, 8, 7), dt=1e-4)
+
+
+def _load(sc, s):
+    sc, mesh = sc if isinstance(sc, tuple) else (sc, None)
+    sc.load_into(s)
+    if mesh:
+        s.set_mesh(mesh["x"], mesh["faces"], **{k: v for k, v in mesh.items() if k not in ("x", "faces")})
+    return sc
+
+
+def _between(s, what, sc):
+    if what == "autotune":
+        s.autotune(sc.dt, reps=1)
+    elif what == "radix":
+        t = s.tuning()
+        s.set_tuning(t["p2g_ranks"], t["p2g_blocks"], t["grid_blocks"], _lib.SORT_RADIX, t["p2g_pass"])
+    elif what == "eager":
+        s.time_substeps(sc.dt, 2)
+        s.substep(sc.dt)
+
+
+@pytest.mark.parametrize("kind", ["sand", "cloth"])
+@pytest.mark.parametrize("what", ["autotune", "radix", "eager"])
+def test_substeps_after(kind, what):
+    scene = _scene(kind)
+    outs = []
+    for interrupted in (False, True):
+        with Solver(0) as s:
+            sc = _load(scene, s)
+            s.run(sc.dt, 5)
+            if interrupted:
+                _between(s, what, sc)
+            elif what == "eager":
+                s.run(sc.dt, 3)
+            s.run(sc.dt, 6)
+            if kind == "sand":
+                keys, ids, bins = s.get_sorted()
+                assert np.array_equal(np.diff(bins), np.bincount(keys, minlength=len(bins) - 1))
+                order = np.lexsort((ids, keys))
+                assert np.array_equal(order, np.arange(s.n)) and np.array_equal(np.sort(ids), np.arange(s.n))
+            outs.append((s.get_particles(), s.stats()["n_active_tiles"], s.stats()["n_active_blocks"]))
+    print(kind, what, outs[0][1:], outs[1][1:], flush=True)
+    assert outs[0][1:] == outs[1][1:]
+    for k in KEYS:
+        assert np.array_equal(outs[0][0][k].view(np.uint32), outs[1][0][k].view(np.uint32)), k
+
+
+@pytest.mark.parametrize("steps", [1, 4, 7])
+def test_new_particles(steps):
+    # counts that no sort has used are dropped with the particles they belong to
+    sc, other = _scene("sand"), _scene("sand")
+    other.particles["x"] = (other.particles["x"] + 0.1).astype(np.float32)
+    outs = []
+    for first in (None, other):
+        with Solver(0) as s:
+            (first or sc).load_into(s)
+            if first:
+                s.run(sc.dt, steps)
+                p = sc.particles
+                s.set_particles(p["x"], p["mass"], v=p.get("v"), B=p.get("B"), F=p.get("F"), plastic=p.get("plastic"),
+                                volume=p.get("volume"), phi=p.get("phi"))
+            s.run(sc.dt, 5)
+            outs.append(s.get_particles())
+    for k in KEYS:
+        assert np.array_equal(outs[0][k].view(np.uint32), outs[1][k].view(np.uint32)), k
+
+
+@pytest.mark.parametrize("lo,size", [(0.0, 1.0), (0.37, 1.0), (-5.3, 7.7), (1000.1, 1.0), (-64.0, 128.0)])
+def test_keys_at_cell_boundaries(lo, size):
+    res = (37, 41, 23)
+    mn, mx = [lo, lo + 0.11, lo - 0.23], [lo + size, lo + 0.11 + size, lo - 0.23 + size]
+    axes, rng = [], np.random.default_rng(3)
+    for d in range(3):
+        h = (mx[d] - mn[d]) / res[d]
+        c = np.float32(mn[d] + h * np.arange(1, res[d]))
+        near = [c]
+        for _ in range(3):
+            near.append(np.nextafter(near[-1], np.float32(np.inf)))
+        near.append(np.nextafter(c, np.float32(-np.inf)))
+        near.append(np.nextafter(near[-1], np.float32(-np.inf)))
+        near.append(np.float32(mn[d] + h * rng.uniform(0.01, res[d] - 0.01, 500)))
+        axes.append(np.concatenate(near))
+    n = max(map(len, axes))
+    x = np.stack([rng.permutation(np.resize(a, n)) for a in axes]).astype(np.float32)
+    want = np.zeros(n, np.int64)
+    for d, mult in ((0, 1), (1, res[0]), (2, res[0] * res[1])):
+        h = (mx[d] - mn[d]) / res[d]
+        want += np.floor((x[d].astype(np.float64) - mn[d]) / h).astype(np.int64) * mult
+    with Solver(0) as s:
+        s.set_grid(mn, mx, res)
+        s.set_params(scenes.sand_params())
+        s.set_particles(x, np.ones(n, np.float32))
+        s.stage(_lib.STAGE_SORT, 1e-4)
+        keys, ids, _ = s.get_sorted()
+    got = np.empty(n, np.int64)
+    got[ids] = keys
+    print(lo, size, n, int((got != want).sum()), flush=True)
+    assert np.array_equal(got, want)
