@@ -107,7 +107,12 @@ __device__ __forceinline__ DevParams uniform_params(const DevParams& G) {
 // reference evaluated in double (HybridSolver.cpp:33-36) for x >= min, using FP32 compares only.
 // The FP32 quotient t is within inv_h (2^-24 |gmin| + 2^-24 |x - gmin|) + 2^-24 |t| (rounded bounds, difference,
 // spacing and product), less than 2^-22 (|gmin| inv_h + |t|), of the exact one: where t is farther than that
-// from a whole number, floor(t) is the cell, and the thresholds of the cell itself are not read.
+// from a whole number, floor(t) is the cell, and the thresholds of the cell itself are not gathered (k_g2p with
+// them 386 -> 365 us at 2^22 particles, 185 -> 177 us for 16 scenes of 1.8 M).
+// The FP32 quotient t is within inv_h (2^-24 |gmin| + 2^-24 |x - gmin|) + 2^-24 |t| (rounded bounds, difference,
+// spacing and product), less than 2^-22 (|gmin| inv_h + |t|), of the exact one: where t is farther than that
+// from a whole number, floor(t) is the cell, and the thresholds of the cell itself are not gathered (k_g2p with
+// them 386 -> 365 us at 2^22 particles, 185 -> 177 us for 16 scenes of 1.8 M).
 __device__ __forceinline__ int axis_cell(const float* thr, int res, float x, float gmin, float inv_h, int& oob) {
   if (!(x >= thr[0])) { oob = 1; return 0; }
   if (x >= thr[res]) { oob = 1; return res - 1; }
@@ -528,7 +533,7 @@ __device__ __forceinline__ void claim_block(const SortBufs& a, int b) {
 // The scan blocks' totals (workgroups below nscan) and the tile lists (the others): independent of each other,
 // so one launch hides one's latency behind the other's. With the counts made by G2P a substep sorts in four
 // launches (this one, scan, scatter, rank) where a separate count, totals and claim took six: sort 117 -> 83 us and
-// G2P 356 -> 386 at 2^22 particles, sort 30 -> 22 us and G2P unchanged at 2^15.
+// G2P 356 -> 365 at 2^22 particles, sort 30 -> 22 us and G2P unchanged at 2^15.
 __global__ __launch_bounds__(256) void k_sums_claim(SortBufs a, int nscan) {
   if (clock_skip(a.clk)) return;
   const int b = (int)blockIdx.x;
