@@ -109,10 +109,6 @@ __device__ __forceinline__ DevParams uniform_params(const DevParams& G) {
 // spacing and product), less than 2^-22 (|gmin| inv_h + |t|), of the exact one: where t is farther than that
 // from a whole number, floor(t) is the cell, and the thresholds of the cell itself are not gathered (k_g2p with
 // them 386 -> 365 us at 2^22 particles, 185 -> 177 us for 16 scenes of 1.8 M).
-// The FP32 quotient t is within inv_h (2^-24 |gmin| + 2^-24 |x - gmin|) + 2^-24 |t| (rounded bounds, difference,
-// spacing and product), less than 2^-22 (|gmin| inv_h + |t|), of the exact one: where t is farther than that
-// from a whole number, floor(t) is the cell, and the thresholds of the cell itself are not gathered (k_g2p with
-// them 386 -> 365 us at 2^22 particles, 185 -> 177 us for 16 scenes of 1.8 M).
 __device__ __forceinline__ int axis_cell(const float* thr, int res, float x, float gmin, float inv_h, int& oob) {
   if (!(x >= thr[0])) { oob = 1; return 0; }
   if (x >= thr[res]) { oob = 1; return res - 1; }
@@ -538,10 +534,8 @@ __global__ __launch_bounds__(256) void k_sums_claim(SortBufs a, int nscan) {
   if (clock_skip(a.clk)) return;
   const int b = (int)blockIdx.x;
   if (b < nscan) {
-    if (b == 0 && threadIdx.x < 2) {
-      a.counters_clear[threadIdx.x] = 0;
-      a.counters_misc[threadIdx.x] = 0;
-    }
+    if (b == 0 && threadIdx.x < 2) a.counters_clear[threadIdx.x] = 0;
+    if (b == 0 && threadIdx.x == 2) *a.cand_count = 0;
     sum_block(a, b);
   } else {
     claim_block(a, b - nscan);
@@ -2070,15 +2064,44 @@ __global__ __launch_bounds__(256) void k_g2p(G2PArgs a) {
 // k_g2p stored and the particle's q, phi and V, the FP64 projection and F_E and V tau (the same
 // function return_map calls, on the same operands), stored over the trial F^ left in the output
 // buffer. The result equals computing it inside k_g2p.
+//
+// A workgroup takes the masks of `gw` G2P waves at a time (4, a G2P workgroup's, where that gives few groups;
+// else 16, which gathers fuller waves), lists their flagged positions in LDS and works the list off. Bound by
+// the launch and one round trip of the masks where few particles are flagged. (With a list over all waves, made by
+// two launches before this one, G2P to here took 95 us instead of 92 at 2^20 particles, 177 instead of 171 for 16 scenes.)
 __global__ __launch_bounds__(256) void k_apex_finish(ApexArgs a) {
   if (clock_skip(a.clk)) return;
-  const int count = min(*a.apex_count, a.n);
+  __shared__ int s_slot[64 * APEX_GROUP], s_idx[64 * APEX_GROUP];
+  const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
   int fb_apex = 0;
-  for (int c0 = blockIdx.x * 256; c0 < count; c0 += gridDim.x * 256) {
-    const int c = c0 + (int)threadIdx.x;
-    if (c < count) {
-      const int j = clamp_index(a.apex_slot[c], a.n);
-      const int r = clamp_index(a.apex_idx[c], a.n);
+  for (int w0 = (int)blockIdx.x * a.gw; w0 < a.nwaves; w0 += (int)gridDim.x * a.gw) {
+    const int nw = min(a.gw, a.nwaves - w0);
+    // wave wv lists the masks wv, wv + 4, ...; every wave forms the offsets (lane l: mask l) by itself
+    const uint64_t ml = lane < nw ? a.mask[w0 + lane] : 0ull;
+    int off = __popcll(ml);
+    const int own = off;
+#pragma unroll
+    for (int d = 1; d < APEX_GROUP; d <<= 1) {
+      const int y = __shfl_up(off, d);
+      if (lane >= d) off += y;
+    }
+    const int count = __builtin_amdgcn_readlane(off, APEX_GROUP - 1);
+    if (count == 0) continue;  // uniform over the workgroup
+    off -= own;
+    for (int q = wv; q < nw; q += 4) {
+      const uint64_t m = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(ml >> 32), q) << 32) |
+                         (uint32_t)__builtin_amdgcn_readlane((int)ml, q);
+      const int o = __builtin_amdgcn_readlane(off, q), p = a.wave_pos[w0 + q];
+      if ((m >> lane) & 1ull) {
+        const int rank = __popcll(m & ((1ull << lane) - 1ull));
+        s_slot[o + rank] = p + lane;
+        s_idx[o + rank] = p + rank;
+      }
+    }
+    __syncthreads();
+    for (int c = (int)threadIdx.x; c < count; c += 256) {
+      const int j = clamp_index(s_slot[c], a.n);
+      const int r = clamp_index(s_idx[c], a.n);
       const int sc = scene_of(a.T.part_off, a.T.nscenes, j);
       const DevParams& P = a.T.params[sc];
       float* st = a.st;
@@ -2116,6 +2139,7 @@ __global__ __launch_bounds__(256) void k_apex_finish(ApexArgs a) {
         for (int e = 0; e < 6; ++e) st[(PK + e) * cap + j] = K[e];
       }
     }
+    __syncthreads();
   }
   // one atomic per wave
   unsigned long long c = (unsigned long long)fb_apex;
@@ -2124,46 +2148,41 @@ __global__ __launch_bounds__(256) void k_apex_finish(ApexArgs a) {
   if ((threadIdx.x & 63) == 0 && c) atomicAdd(a.fallback_apex, c);
 }
 
-// ================================================================== position lists
-// Lists of the sorted positions that G2P flagged, in ascending order and without atomics: the
-// deferred FP64 apex projections and the surrogate's candidates (two lists, one set of launches).
-// Every G2P wave w stores the ballots of its flagged lanes (mask[l][w]) and the position of its
+// ================================================================== position list
+// List of the sorted positions that G2P flagged as the surrogate's candidates, in ascending order and without
+// atomics. Every G2P wave w stores the ballot of its flagged lanes (mask[w]) and the position of its
 // lane 0 (wpos[w]). Waves form groups of 64: k_list_sums totals each group; k_list_write (one
 // workgroup per group) adds up the totals of the groups before its own, places each wave's
 // positions after that offset and the waves before it in the group, and the last group's
-// workgroup writes the list lengths.
+// workgroup writes the list's length.
 __global__ __launch_bounds__(256) void k_list_sums(ListArgs a) {
   const int ng = (a.nwaves + 63) / 64;
   const int g = blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (g >= ng) return;
   const int w = g * 64 + lane;
-  for (int l = 0; l < a.nlists; ++l) {
-    int c = w < a.nwaves ? __popcll(a.mask[l][w]) : 0;
+  int c = w < a.nwaves ? __popcll(a.mask[w]) : 0;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off);
-    if (lane == 0) a.gsum[l * ng + g] = c;
-  }
+  for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off);
+  if (lane == 0) a.gsum[g] = c;
 }
 
 __global__ __launch_bounds__(256) void k_list_write(ListArgs a) {
-  __shared__ uint64_t s_m[2][64];
-  __shared__ int s_off[2][64], s_p[64], s_red[2][4];
+  __shared__ uint64_t s_m[64];
+  __shared__ int s_off[64], s_p[64], s_red[4];
   const int ng = (a.nwaves + 63) / 64;
   const int g = blockIdx.x, t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int w = g * 64 + lane;
-  // each list's offset of this group: the totals of the groups before it, summed by the workgroup
+  // the offset of this group: the totals of the groups before it, summed by the workgroup
   // itself (integer sums, so the order does not matter)
-  for (int l = 0; l < a.nlists; ++l) {
-    int sum = 0;
-    for (int i = t; i < g; i += 256) sum += a.gsum[l * ng + i];
+  int sum = 0;
+  for (int i = t; i < g; i += 256) sum += a.gsum[i];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-    if (lane == 0) s_red[l][wv] = sum;
-  }
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+  if (lane == 0) s_red[wv] = sum;
   __syncthreads();
-  if (wv < a.nlists) {  // wave l: the offsets of list l's 64 masks of the group
-    const int pre = s_red[wv][0] + s_red[wv][1] + s_red[wv][2] + s_red[wv][3];
-    const uint64_t m = w < a.nwaves ? a.mask[wv][w] : 0ull;
+  if (wv == 0) {  // the offsets of the group's 64 masks
+    const int pre = s_red[0] + s_red[1] + s_red[2] + s_red[3];
+    const uint64_t m = w < a.nwaves ? a.mask[w] : 0ull;
     const int c = __popcll(m);
     int x = c;
 #pragma unroll
@@ -2171,24 +2190,23 @@ __global__ __launch_bounds__(256) void k_list_write(ListArgs a) {
       const int y = __shfl_up(x, off);
       if (lane >= off) x += y;
     }
-    s_m[wv][lane] = m;
-    s_off[wv][lane] = pre + x - c;
+    s_m[lane] = m;
+    s_off[lane] = pre + x - c;
     // the last group's workgroup writes the list's length
-    if (g == ng - 1 && lane == 63) *a.count[wv] = pre + x;
+    if (g == ng - 1 && lane == 63) *a.count = pre + x;
   } else if (wv == 3) {
     s_p[lane] = w < a.nwaves ? a.wpos[w] : 0;
   }
   __syncthreads();
-  // wave wv writes the positions of masks 16 wv .. 16 wv + 15 of each list, one mask at a time
-  for (int l = 0; l < a.nlists; ++l)
-    for (int i = 16 * wv; i < 16 * wv + 16; ++i) {
-      const uint64_t mi = s_m[l][i];
-      if ((mi >> lane) & 1ull) {
-        const int rank = __popcll(mi & ((1ull << lane) - 1ull));
-        a.list[l][s_off[l][i] + rank] = s_p[i] + lane;
-        a.idx[l][s_off[l][i] + rank] = s_p[i] + rank;
-      }
+  // wave wv writes the positions of masks 16 wv .. 16 wv + 15, one mask at a time
+  for (int i = 16 * wv; i < 16 * wv + 16; ++i) {
+    const uint64_t mi = s_m[i];
+    if ((mi >> lane) & 1ull) {
+      const int rank = __popcll(mi & ((1ull << lane) - 1ull));
+      a.list[s_off[i] + rank] = s_p[i] + lane;
+      a.idx[s_off[i] + rank] = s_p[i] + rank;
     }
+  }
 }
 
 // ================================================================== surrogate return map
@@ -2776,8 +2794,8 @@ void surrogate_set_smem_limit() {
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)surrogate_smem());
 }
 
-void launch_position_lists(hipStream_t s, const ListArgs& a) {
-  if (a.nwaves <= 0 || a.nlists <= 0) return;
+void launch_position_list(hipStream_t s, const ListArgs& a) {
+  if (a.nwaves <= 0) return;
   const int ng = (a.nwaves + 63) / 64;
   hipLaunchKernelGGL(k_list_sums, dim3((ng + 3) / 4), dim3(256), 0, s, a);
   hipLaunchKernelGGL(k_list_write, dim3(ng), dim3(256), 0, s, a);
@@ -2791,8 +2809,11 @@ void launch_surrogate(hipStream_t s, const SurrogateArgs& a, int n_cu, hipEvent_
   hipLaunchKernelGGL(k_surrogate, dim3(n_cu), dim3(MLP_FWD_THREADS), surrogate_smem(), s, a);
 }
 
-void launch_apex_finish(hipStream_t s, const ApexArgs& a, int grid) {
-  hipLaunchKernelGGL(k_apex_finish, dim3(grid), dim3(256), 0, s, a);
+void launch_apex_finish(hipStream_t s, ApexArgs a, int n_cu) {
+  const int small = blocks_for(a.nwaves, 4);
+  a.gw = small <= 8 * n_cu ? 4 : APEX_GROUP;
+  hipLaunchKernelGGL(k_apex_finish, dim3(a.gw == 4 ? small : std::min(8 * n_cu, blocks_for(a.nwaves, APEX_GROUP))),
+                     dim3(256), 0, s, a);
 }
 
 void launch_fill_int(hipStream_t s, int* p, int64_t n, int v) {

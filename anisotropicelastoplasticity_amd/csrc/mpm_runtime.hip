@@ -159,11 +159,11 @@ struct mpm_ctx {
   float* pair_log = nullptr;
   int64_t pair_cap = 0;
   // per G2P wave (4 per particle block): sorted position of lane 0, and the lanes that deferred to
-  // the surrogate or to the FP64 apex pass; the lists are built from them without atomics
+  // the surrogate or to the FP64 apex pass
   int* wave_pos = nullptr;
   uint64_t* cand_mask = nullptr;
   uint64_t* apex_mask = nullptr;
-  int* list_gsum = nullptr;  // per list and group of 64 waves: count, then offset
+  int* list_gsum = nullptr;  // candidates per group of 64 waves
   int64_t wave_cap = 0;
   float* dec_log = nullptr;  // per-candidate gate records of the last surrogate substep
   int64_t dec_cap = 0;
@@ -176,9 +176,7 @@ struct mpm_ctx {
   // set by mpm_time_kernels: the start and end of a stage's main kernel (taken by its launch)
   hipEvent_t ev_main[2] = {nullptr, nullptr};
   hipEvent_t ev_sur[2] = {nullptr, nullptr};  // the surrogate kernel's start and stop (timing only)
-  int* apex_slot = nullptr;  // sorted slots of the deferred FP64 apex projections (n)
-  int* apex_idx = nullptr;    // their record indices in apex_usv (n)
-  float* apex_usv = nullptr;  // their trial SVD (CAND_SVD_PLANES x n)
+  float* apex_usv = nullptr;  // the trial SVDs of the deferred FP64 apex projections (CAND_SVD_PLANES x n)
 };
 
 static void drop_mesh(mpm_ctx* ctx);
@@ -440,7 +438,7 @@ static int stage_sort(mpm_ctx* ctx) {
   b.src = ctx->src;
   b.counters = ctx->counters + 2 * ctx->cur;
   b.counters_clear = ctx->counters + 2 * (1 - ctx->cur);
-  b.counters_misc = ctx->counters + CNT_CAND;
+  b.cand_count = ctx->counters + CNT_CAND;
   b.clk = ctx->clk_active;
   launch_sort(s, b, ctx->keys, ctx->n, ctx->nblocks_p, ctx->sort_passes, ctx->sort_mode);
   if (ctx->sort_mode != SORT_COUNTING) ctx->pos_ok = true;  // the radix mode's key conversion wrote pos[cur]
@@ -613,35 +611,16 @@ static int stage_g2p(mpm_ctx* ctx, float dt) {
   a.apex_usv = ctx->apex_usv;
   a.clk = ctx->clk_active;
   launch_g2p(ctx->stream, a, ctx->order, ctx->nblocks_p, ctx->ev_main[0], ctx->ev_main[1]);
-  {
-    ListArgs la{};
-    la.wpos = ctx->wave_pos;
-    la.gsum = ctx->list_gsum;
-    la.nwaves = 4 * ctx->nblocks_p;
-    if (a.apex_mask) {
-      la.mask[la.nlists] = ctx->apex_mask;
-      la.list[la.nlists] = ctx->apex_slot;
-      la.idx[la.nlists] = ctx->apex_idx;
-      la.count[la.nlists++] = ctx->counters + CNT_APEX;
-    }
-    if (surrogate) {
-      la.mask[la.nlists] = ctx->cand_mask;
-      la.list[la.nlists] = ctx->cand_slot;
-      la.idx[la.nlists] = ctx->cand_idx;
-      la.count[la.nlists++] = ctx->counters + CNT_CAND;
-    }
-    launch_position_lists(ctx->stream, la);
-  }
   if (a.apex_mask) {
     ApexArgs x;
     x.T = ctx->T;
     x.st = ctx->state[1 - ctx->cur];
     x.cap = ctx->cap;
     x.n = ctx->n;
-    x.apex_slot = ctx->apex_slot;
-    x.apex_idx = ctx->apex_idx;
+    x.mask = ctx->apex_mask;
+    x.wave_pos = ctx->wave_pos;
+    x.nwaves = 4 * ctx->nblocks_p;
     x.apex_usv = ctx->apex_usv;
-    x.apex_count = ctx->counters + CNT_APEX;
     x.write_stress = a.write_stress;
     x.log_pairs = a.sur_mode == 1;
     x.pair_log = ctx->pair_log;
@@ -650,9 +629,18 @@ static int stage_g2p(mpm_ctx* ctx, float dt) {
     x.fallback_svd = ctx->fallbacks;
     x.fallback_apex = ctx->fallbacks + 1;
     x.clk = ctx->clk_active;
-    launch_apex_finish(ctx->stream, x, 2 * ctx->n_cu);
+    launch_apex_finish(ctx->stream, x, ctx->n_cu);
   }
   if (surrogate) {
+    ListArgs la;
+    la.mask = ctx->cand_mask;
+    la.list = ctx->cand_slot;
+    la.idx = ctx->cand_idx;
+    la.count = ctx->counters + CNT_CAND;
+    la.gsum = ctx->list_gsum;
+    la.wpos = ctx->wave_pos;
+    la.nwaves = 4 * ctx->nblocks_p;
+    launch_position_list(ctx->stream, la);
     SurrogateArgs sa;
     sa.T = ctx->T;
     sa.wbf = ctx->mlp_wbf;
@@ -809,7 +797,7 @@ int mpm_destroy(mpm_ctx* ctx) {
   dfree(ctx->tile_slot); dfree(ctx->active_tiles); dfree(ctx->block_slot); dfree(ctx->active_blocks);
   dfree(ctx->partials);
   dfree(ctx->state[0]); dfree(ctx->state[1]); dfree(ctx->keys); dfree(ctx->pos[0]); dfree(ctx->pos[1]); dfree(ctx->tslot);
-  dfree(ctx->k1); dfree(ctx->k2); dfree(ctx->v1); dfree(ctx->v2); dfree(ctx->src); dfree(ctx->sortws); dfree(ctx->apex_slot); dfree(ctx->apex_idx); dfree(ctx->apex_usv);
+  dfree(ctx->k1); dfree(ctx->k2); dfree(ctx->v1); dfree(ctx->v2); dfree(ctx->src); dfree(ctx->sortws); dfree(ctx->apex_usv);
   dfree(ctx->counters); dfree(ctx->status); dfree(ctx->fallbacks);
   dfree(ctx->clock);
   dfree(ctx->mlp_master); dfree(ctx->mlp_m1); dfree(ctx->mlp_m2); dfree(ctx->mlp_grad); dfree(ctx->mlp_wbf);
@@ -1007,7 +995,7 @@ static int alloc_wave_tables(mpm_ctx* ctx) {
   int rc = dalloc(ctx, ctx->wave_pos, (size_t)nw);
   if (!rc) rc = dalloc(ctx, ctx->cand_mask, (size_t)nw);
   if (!rc) rc = dalloc(ctx, ctx->apex_mask, (size_t)nw);
-  if (!rc) rc = dalloc(ctx, ctx->list_gsum, (size_t)(2 * ((nw + 63) / 64)));
+  if (!rc) rc = dalloc(ctx, ctx->list_gsum, (size_t)((nw + 63) / 64));
   ctx->wave_cap = rc ? 0 : nw;
   return rc;
 }
@@ -1029,8 +1017,6 @@ static int install_state(mpm_ctx* ctx, int n, const std::vector<float>& h) {
     if (!rc) rc = dalloc(ctx, ctx->v1, n);
     if (!rc) rc = dalloc(ctx, ctx->v2, n);
     if (!rc) rc = dalloc(ctx, ctx->src, n);
-    if (!rc) rc = dalloc(ctx, ctx->apex_slot, n);
-    if (!rc) rc = dalloc(ctx, ctx->apex_idx, n);
     if (!rc) rc = dalloc(ctx, ctx->apex_usv, (size_t)CAND_SVD_PLANES * n);
     if (!rc && (ctx->sur_enabled || ctx->cand)) rc = dalloc(ctx, ctx->cand, (size_t)CAND_SVD_PLANES * n);
     if (!rc && (ctx->sur_enabled || ctx->cand_slot)) rc = dalloc(ctx, ctx->cand_slot, (size_t)n);
