@@ -109,9 +109,11 @@ __device__ __forceinline__ DevParams uniform_params(const DevParams& G) {
 // spacing and product), less than 2^-22 (|gmin| inv_h + |t|), of the exact one: where t is farther than that
 // from a whole number, floor(t) is the cell, and the thresholds of the cell itself are not gathered (k_g2p with
 // them 386 -> 365 us at 2^22 particles, 185 -> 177 us for 16 scenes of 1.8 M).
-__device__ __forceinline__ int axis_cell(const float* thr, int res, float x, float gmin, float inv_h, int& oob) {
-  if (!(x >= thr[0])) { oob = 1; return 0; }
-  if (x >= thr[res]) { oob = 1; return res - 1; }
+// lo, hi: thr[0] and thr[res].
+__device__ __forceinline__ int axis_cell(const float* thr, float lo, float hi, int res, float x, float gmin, float inv_h,
+                                         int& oob) {
+  if (!(x >= lo)) { oob = 1; return 0; }
+  if (x >= hi) { oob = 1; return res - 1; }
   const float t = (x - gmin) * inv_h, tf = floorf(t), near = 0x1p-22f * (fabsf(gmin) * inv_h + fabsf(t));
   int c = (int)tf;
   c = c < 0 ? 0 : (c > res - 1 ? res - 1 : c);
@@ -134,11 +136,30 @@ __device__ __forceinline__ int stencil_base(float g, int res) {
   return (int)b;
 }
 
-__device__ __forceinline__ uint32_t cell_key(const DevParams& P, const float* thr, float x0, float x1, float x2, int& oob,
+// A scene's thresholds and its grid's bounds among them. Formed at a kernel's start, where the compiler reads
+// uniform data through the scalar cache; after a kernel's first stores it would read each bound as a vector and
+// wait for it: six round trips one after another in every G2P wave (k_g2p 362 -> 328 us at 2^22 particles, 172 ->
+// 157 for 16 scenes, 90 -> 86 at 2^20).
+struct CellThr {
+  const float* thr[3];
+  float lo[3], hi[3];
+};
+__device__ __forceinline__ CellThr cell_thr(const float* thr, const int* res) {
+  CellThr t;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    t.thr[d] = thr;
+    t.lo[d] = thr[0];
+    t.hi[d] = thr[res[d]];
+    thr += res[d] + 1;
+  }
+  return t;
+}
+__device__ __forceinline__ uint32_t cell_key(const DevParams& P, const CellThr& t, float x0, float x1, float x2, int& oob,
                                              int (&c)[3]) {
-  c[0] = axis_cell(thr, P.res[0], x0, P.gmin[0], P.inv_h[0], oob);
-  c[1] = axis_cell(thr + (P.res[0] + 1), P.res[1], x1, P.gmin[1], P.inv_h[1], oob);
-  c[2] = axis_cell(thr + (P.res[0] + 1) + (P.res[1] + 1), P.res[2], x2, P.gmin[2], P.inv_h[2], oob);
+  c[0] = axis_cell(t.thr[0], t.lo[0], t.hi[0], P.res[0], x0, P.gmin[0], P.inv_h[0], oob);
+  c[1] = axis_cell(t.thr[1], t.lo[1], t.hi[1], P.res[1], x1, P.gmin[1], P.inv_h[1], oob);
+  c[2] = axis_cell(t.thr[2], t.lo[2], t.hi[2], P.res[2], x2, P.gmin[2], P.inv_h[2], oob);
   return (uint32_t)(c[2] * P.res[0] * P.res[1] + c[1] * P.res[0] + c[0]);
 }
 
@@ -187,10 +208,11 @@ __global__ __launch_bounds__(256) void k_keys(SceneTable T, const float* __restr
   const DevParams& P = T.params[b.s];
   const int j = b.j;
   int oob = 0;
+  const CellThr t = cell_thr(thr + T.thr_off[b.s], P.res);
   int c[3];
   if (j < b.end)
     keys[j] = (uint32_t)T.node_off[b.s] +
-              cell_key(P, thr + T.thr_off[b.s], st[PX * cap + j], st[(PX + 1) * cap + j], st[(PX + 2) * cap + j], oob, c);
+              cell_key(P, t, st[PX * cap + j], st[(PX + 1) * cap + j], st[(PX + 2) * cap + j], oob, c);
   if (__ballot(oob) && lane_id() == 0) atomicOr(status, MPM_STATUS_OUT_OF_DOMAIN);
 }
 
@@ -529,7 +551,7 @@ __device__ __forceinline__ void claim_block(const SortBufs& a, int b) {
 // The scan blocks' totals (workgroups below nscan) and the tile lists (the others): independent of each other,
 // so one launch hides one's latency behind the other's. With the counts made by G2P a substep sorts in four
 // launches (this one, scan, scatter, rank) where a separate count, totals and claim took six: sort 117 -> 83 us and
-// G2P 356 -> 365 at 2^22 particles, sort 30 -> 22 us and G2P unchanged at 2^15.
+// G2P 356 -> 328 at 2^22 particles (of which 55 us less by the cell_key changes), sort 30 -> 22 us at 2^15.
 __global__ __launch_bounds__(256) void k_sums_claim(SortBufs a, int nscan) {
   if (clock_skip(a.clk)) return;
   const int b = (int)blockIdx.x;
@@ -1707,6 +1729,8 @@ __global__ __launch_bounds__(256) void k_g2p(G2PArgs a) {
   const int64_t noff = a.T.node_off[pb.s];
   const float4* gvel = a.gvel + 2 * noff;
   const int j = pb.j;
+  const CellThr thr = cell_thr(a.thr + a.T.thr_off[pb.s], P.res);
+  const int toff = a.T.tile_off[pb.s];
   int oob = 0, bad = 0, cfl = 0, fb_svd = 0, fb_apex = 0;
   bool cand = false, apex = false;
   const int wv = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
@@ -1945,9 +1969,9 @@ __global__ __launch_bounds__(256) void k_g2p(G2PArgs a) {
     // the atomics are in flight during the return map
     const int kind = particle_kind(P, pid);
     int cell[3];
-    const uint32_t key = (uint32_t)noff + cell_key(P, a.thr + a.T.thr_off[pb.s], xn[0], xn[1], xn[2], oob, cell);
+    const uint32_t key = (uint32_t)noff + cell_key(P, thr, xn[0], xn[1], xn[2], oob, cell);
     const CountTicket ticket =
-        count_wave(a.bins, kind != KIND_ELEMENT, key, a.T.tile_off[pb.s] + tile_of(P, cell[0], cell[1], cell[2]));
+        count_wave(a.bins, kind != KIND_ELEMENT, key, toff + tile_of(P, cell[0], cell[1], cell[2]));
     // cloth vertices and elements keep only the skew part of B (damping 1, HybridSolver.cpp:926-932)
     const float damping = kind == KIND_PARTICLE ? P.damping : 1.0f;
     if (damping != 0.0f) {
@@ -2465,8 +2489,9 @@ __global__ __launch_bounds__(256) void k_cloth_elements(ClothArgs a) {
   if (clock_skip(a.clk)) return;
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   int fb = 0, oob = 0;
+  const DevParams& P = a.P;
+  const CellThr thr = cell_thr(a.thr, P.res);
   if (e < a.ne) {
-    const DevParams& P = a.P;
     const int id = P.mesh_e0 + e;
     // the element's and its vertices' slots, then all of their data in one round of loads
     const int pe = clamp_index(a.pos[id], a.n);
@@ -2497,7 +2522,7 @@ __global__ __launch_bounds__(256) void k_cloth_elements(ClothArgs a) {
 #pragma unroll
     for (int i = 0; i < 9; ++i) a.st[(PF + i) * a.cap + pe] = D[i];
     int cell[3];
-    const uint32_t key = cell_key(P, a.thr, xe[0], xe[1], xe[2], oob, cell);
+    const uint32_t key = cell_key(P, thr, xe[0], xe[1], xe[2], oob, cell);
     const CountTicket ticket = count_wave(a.bins, true, key, tile_of(P, cell[0], cell[1], cell[2]));
     a.keys[pe] = key;
     a.bins.rank[pe] = count_rank(ticket);
