@@ -116,7 +116,6 @@ struct Clock {
   float dt_f;        // Dt as the kernels use it
   unsigned int vmax_bits;  // max |v| over nodes after the velocity update (float bits, atomicMax)
   int frame;         // frames completed
-  int frame_now;     // the current substep completes a frame
   int frame_done;    // a frame completed since the host last cleared it
   int done;          // t > maxt
   int skip;          // the rest of the replayed batch does nothing
@@ -325,10 +324,10 @@ void launch_count_nodes(hipStream_t s, const SceneTable& T, const float* gm, con
                         unsigned long long* out, int grid);
 void launch_fill_int(hipStream_t s, int* p, int64_t n, int v);
 void launch_copy(hipStream_t s, const float4* src, float4* dst, int64_t n4);
-// Dt from the max node speed (init: the first Dt, no frame bookkeeping), then the frame clamp.
 void launch_stress_predicted(hipStream_t s, const P2GArgs& a, int order, int nblocks);
-void launch_clock_update(hipStream_t s, Clock* c, int init);
-// End of a substep: count it, close a completed frame, stop the batch after a frame or the run.
+// The first Dt from the max node speed.
+void launch_clock_init(hipStream_t s, Clock* c);
+// End of a substep: the new Dt from the max node speed and the frame clamp; count it, close a completed frame, stop the batch after a frame or the run.
 void launch_clock_end(hipStream_t s, Clock* c);
 // Cloth (mesh vertices and elements among the particles of scene 0; caller ids from the DevParams).
 struct ClothArgs {

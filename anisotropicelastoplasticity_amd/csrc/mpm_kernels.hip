@@ -1632,7 +1632,10 @@ __global__ __launch_bounds__(64) void k_grid(GridArgs a) {
   if (a.vmax_out != nullptr) {
     // max over the wave, one atomic per wave (non-negative floats order as their bit patterns)
     for (int off = 32; off > 0; off >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, off));
-    if (threadIdx.x == 0 && vmax > 0.0f) atomicMax(a.vmax_out, __float_as_uint(vmax));
+    // (only a new maximum, as far as this wave can see: the waves' atomics on one word run one after another)
+    if (threadIdx.x == 0 && vmax > 0.0f &&
+        __hip_atomic_load(a.vmax_out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < __float_as_uint(vmax))
+      atomicMax(a.vmax_out, __float_as_uint(vmax));
   }
 }
 
@@ -1641,37 +1644,49 @@ __global__ __launch_bounds__(64) void k_grid(GridArgs a) {
 // RegularGrid.h:60), evaluated in double as in the reference from the max node speed after the
 // velocity update; then the frame clamp to 1/60 s (:880-892): a substep that reaches the frame end
 // is shortened to it, t advances by 1/60 and the frame time restarts.
-__global__ void k_clock_update(Clock* c, int init) {
-  if (threadIdx.x != 0 || blockIdx.x != 0 || c->skip) return;
+// The new Dt from the velocities after the grid update, and whether it ends the frame: G2P forms it for itself,
+// k_clock_end stores it.
+struct ClockStep {
+  double dt;
+  bool frame;
+};
+__device__ __forceinline__ ClockStep clock_step(const Clock* c, bool init) {
   const double vmax = (double)__uint_as_float(c->vmax_bits);
-  c->vmax_bits = 0u;
   const double rate = vmax / c->hmin;
-  double Dt = c->cfl / (rate > 300.0 ? rate : 300.0);
-  if (!init) {
-    if (c->inner + Dt >= 1.0 / 60.0) {
-      Dt = 1.0 / 60.0 - c->inner;
-      c->t += 1.0 / 60.0;
-      c->inner = 0.0;
-      c->frame_now = 1;
-    } else {
-      c->inner += Dt;
-    }
+  ClockStep s{c->cfl / (rate > 300.0 ? rate : 300.0), false};
+  if (!init && c->inner + s.dt >= 1.0 / 60.0) {
+    s.dt = 1.0 / 60.0 - c->inner;
+    s.frame = true;
   }
-  c->dt = Dt;
-  c->dt_f = (float)Dt;
+  return s;
 }
 
-// End of a substep: the reference closes a frame after the substep that completed it (output at
-// HybridSolver.cpp:990-1029) and leaves its loop when t > maxt (:867).
+// The first Dt, before any substep.
+__global__ void k_clock_init(Clock* c) {
+  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  c->dt = clock_step(c, true).dt;
+  c->dt_f = (float)c->dt;
+  c->vmax_bits = 0u;
+}
+
+// End of a substep: the clock advances by the Dt that its G2P took; the reference closes a frame after the
+// substep that completed it (output at HybridSolver.cpp:990-1029) and leaves its loop when t > maxt (:867).
 __global__ void k_clock_end(Clock* c) {
   if (threadIdx.x != 0 || blockIdx.x != 0 || c->skip) return;
+  const ClockStep s = clock_step(c, false);
+  c->dt = s.dt;
+  c->dt_f = (float)s.dt;
+  c->vmax_bits = 0u;
   c->executed += 1;
   c->substeps += 1;
-  if (c->frame_now) {
-    c->frame_now = 0;
+  if (s.frame) {
+    c->t += 1.0 / 60.0;
+    c->inner = 0.0;
     c->frame += 1;
     c->frame_done = 1;
     c->skip = 1;
+  } else {
+    c->inner += s.dt;
   }
   if (c->t > c->maxt) {
     c->done = 1;
@@ -1722,7 +1737,7 @@ __device__ __forceinline__ int floor_div(int a, uint32_t m, int l) {
 template <int ORDER>
 __global__ __launch_bounds__(256) void k_g2p(G2PArgs a) {
   if (clock_skip(a.clk)) return;
-  const float dt = clock_dt(a.clk, a.dt);
+  const float dt = a.clk != nullptr ? (float)clock_step(a.clk, false).dt : a.dt;
   const int pblk = (int)blockIdx.x;
   const PBlock pb = particle_block(a.T, pblk);
   const DevParams P = uniform_params(a.T.params[pb.s]);
@@ -2754,9 +2769,7 @@ void launch_stress_predicted(hipStream_t s, const P2GArgs& a, int order, int nbl
   else hipLaunchKernelGGL(k_stress_predicted<3>, dim3(nblocks), dim3(256), 0, s, a);
 }
 
-void launch_clock_update(hipStream_t s, Clock* c, int init) {
-  hipLaunchKernelGGL(k_clock_update, dim3(1), dim3(64), 0, s, c, init);
-}
+void launch_clock_init(hipStream_t s, Clock* c) { hipLaunchKernelGGL(k_clock_init, dim3(1), dim3(64), 0, s, c); }
 
 void launch_clock_end(hipStream_t s, Clock* c) { hipLaunchKernelGGL(k_clock_end, dim3(1), dim3(64), 0, s, c); }
 
