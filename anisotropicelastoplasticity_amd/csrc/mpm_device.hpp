@@ -652,11 +652,12 @@ __device__ __forceinline__ void cloth_return_map(const DevParams& P, float* D, i
 }
 
 // ------------------------------------------------------------------ level sets (LevelSet.cpp:8-42)
-__device__ __forceinline__ void levelset(const DevParams& P, const float* x, float& phi, float* n) {
+template <class PP>  // DevParams, in any address space
+__device__ __forceinline__ void levelset(PP& P, const float* x, float& phi, float* n) {
   phi = 3.0e38f;
   n[0] = n[1] = n[2] = 0.0f;
   for (int k = 0; k < P.nls; ++k) {
-    const mpm_levelset& pr = P.ls[k];
+    auto& pr = P.ls[k];
     float p, nn[3] = {0.0f, 0.0f, 0.0f};
     if (pr.type == MPM_LS_PLANE) {
       float len = sqrtf(pr.a[0] * pr.a[0] + pr.a[1] * pr.a[1] + pr.a[2] * pr.a[2]);
@@ -689,7 +690,8 @@ __device__ __forceinline__ void levelset(const DevParams& P, const float* x, flo
 }
 
 // Grid collision of one node (HybridSolver.cpp:478-507); v in/out, vbf = velocity before friction.
-__device__ __forceinline__ void collide(const DevParams& P, const float* xnode, float* v, float* vbf) {
+template <class PP>
+__device__ __forceinline__ void collide(PP& P, const float* xnode, float* v, float* vbf) {
   vbf[0] = v[0]; vbf[1] = v[1]; vbf[2] = v[2];
   if (P.nls == 0) return;
   float phi, n[3];

@@ -60,9 +60,19 @@ struct SceneTable {
   const int* thr_off;        // [S] per-axis cell thresholds of the scene
 };
 
-// Largest s in [0, S) with off[s] <= x (off ascending).
+// Data that no thread writes during the kernel, at a uniform address: read through the scalar cache also after
+// the kernel's first stores, where the compiler by itself would issue a vector load and wait for it. (The lists and
+// scene tables of P2G and k_grid: 16 scenes P2G 149 -> 143 us and grid 31 -> 27, 2^22 particles grid 43 -> 42.)
 template <class T>
-__device__ __forceinline__ int scene_of(const T* off, int S, T x) {
+using const_ptr = const __attribute__((address_space(4))) T*;
+template <class T>
+__device__ __forceinline__ const_ptr<T> as_const(const T* p) {
+  return (const_ptr<T>)(uintptr_t)p;
+}
+
+// Largest s in [0, S) with off[s] <= x (off ascending).
+template <class P, class T>
+__device__ __forceinline__ int scene_of(P off, int S, T x) {
   int lo = 0, hi = S - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;

@@ -828,7 +828,8 @@ struct P2GScene {
 };
 
 
-__device__ __forceinline__ P2GScene p2g_scene(const DevParams& P) {
+template <class PP>
+__device__ __forceinline__ P2GScene p2g_scene(PP& P) {
   P2GScene S;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
@@ -1091,6 +1092,51 @@ __global__ __launch_bounds__(256) void k_stress_predicted(P2GArgs a) {
   }
 }
 
+// Constants of a tile's scene.
+struct TileScene {
+  P2GScene S;
+  int64_t noff;
+  int sc, toff, nt0, nt1;
+};
+__device__ __forceinline__ TileScene tile_scene(const P2GArgs& a, int sc) {
+  TileScene n;
+  const auto P = as_const(a.T.params) + sc;
+  n.sc = sc;
+  n.S = p2g_scene(*P);
+  n.noff = as_const(a.T.node_off)[sc];
+  n.toff = as_const(a.T.tile_off)[sc];
+  n.nt0 = P->tiles[0];
+  n.nt1 = P->tiles[1];
+  return n;
+}
+// A tile's first cell (uniform) and, of a wave's two rows, the lane's cells as loaded (lo, hi hold something else
+// where occ is 0).
+struct TileRows {
+  int t0, t1, t2;
+  uint32_t occ[2];
+  int lo[2], hi[2];
+};
+__device__ __forceinline__ TileRows tile_rows(const P2GArgs& a, const TileScene& n, int gtile, int cx, int layer, int half) {
+  TileRows b;
+  const int tile = gtile - n.toff;
+  b.t0 = tile % n.nt0;
+  b.t1 = (tile / n.nt0) % n.nt1;
+  b.t2 = tile / (n.nt0 * n.nt1);
+  const int g0 = 4 * b.t0 + cx, g2 = 4 * b.t2 + layer;
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int g1 = 4 * b.t1 + 2 * half + r;
+    const bool in = g0 < n.S.res[0] && g1 < n.S.res[1] && g2 < n.S.res[2];
+    const int64_t key = n.noff + (in ? (g2 * n.S.res[1] + g1) * n.S.res[0] + g0 : 0);
+    b.occ[r] = a.occ[key / SCAN_TILE];
+    b.lo[r] = a.cell_start[key];
+    b.hi[r] = a.cell_end[key];
+    if (!in) b.occ[r] = 0u;
+  }
+  return b;
+}
+
+
 template <int ORDER, int MODE, int RANKS>
 __global__ __launch_bounds__(64 * P2G_WAVES) void k_p2g(P2GArgs a) {
   if (clock_skip(a.clk)) return;
@@ -1101,7 +1147,7 @@ __global__ __launch_bounds__(64 * P2G_WAVES) void k_p2g(P2GArgs a) {
   __shared__ float s_slab[P2G_WAVES][4][SLAB];  // [wave][quantity][node]
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   const int layer = w & 3, half = w >> 2;  // wave w owns cell layer z = w & 3, rows 2 (w >> 2) and 2 (w >> 2) + 1
-  const int ntile = a.counters[CNT_TILES];
+  const int ntile = as_const(a.counters)[CNT_TILES];
   constexpr int NQ = (MODE == P2G_FORCE) ? 3 : 4;
   // staging role: lane (cx, sr), sr < RANKS; accumulation role: lane (cx, zo, oy)
   const int cx = lane >> 4, sr = lane & 15;
@@ -1109,59 +1155,41 @@ __global__ __launch_bounds__(64 * P2G_WAVES) void k_p2g(P2GArgs a) {
   const float foy = (float)oy, fzo = (float)zo;
   float* slab = &s_slab[w][0][0];
   for (int i = lane; i < 4 * SLAB; i += 64) slab[i] = 0.0f;
-  // a context with one scene reads its constants once; the next tile's index is loaded a tile ahead
-  const bool one_scene = a.T.nscenes == 1;
-  P2GScene S1{};
-  int64_t noff1 = 0;
-  int toff1 = 0, nt0_1 = 1, nt1_1 = 1;
-  if (one_scene) {
-    S1 = p2g_scene(a.T.params[0]);
-    noff1 = a.T.node_off[0];
-    toff1 = a.T.tile_off[0];
-    nt0_1 = __builtin_amdgcn_readfirstlane(a.T.params[0].tiles[0]);
-    nt1_1 = __builtin_amdgcn_readfirstlane(a.T.params[0].tiles[1]);
-  }
   // the tiles of one XCD are a contiguous range of the (ascending) active tiles
   const XcdRange tr = xcd_range(ntile);
-  int gtile_next = tr.first < tr.end ? a.active_tiles[tr.first] : 0;
+  if (tr.first >= tr.end) return;  // uniform: no tile for this workgroup
+  const auto tiles = as_const(a.active_tiles);
+  auto scene_at = [&](int gtile) {
+    return a.T.nscenes == 1 ? 0 : __builtin_amdgcn_readfirstlane(scene_of(as_const(a.T.tile_off), a.T.nscenes, gtile));
+  };
+  const int last = tr.first + (tr.end - 1 - tr.first) / tr.stride * tr.stride;  // this workgroup's last list entry
+  int gtile = tiles[tr.first];
+  int gtile_next = tiles[min(tr.first + tr.stride, last)];
+  TileScene n = tile_scene(a, scene_at(gtile));
+  TileRows rows = tile_rows(a, n, gtile, cx, layer, half);
+  // the lane's cell of each of the wave's two rows, and each row's largest count (uniform)
+  int rstart0, rcnt0, rstart1, rcnt1, rmax0, rmax1;
+  auto take_rows = [&]() {
+    rstart0 = rows.lo[0];
+    rcnt0 = rows.occ[0] ? rows.hi[0] - rows.lo[0] : 0;
+    rstart1 = rows.lo[1];
+    rcnt1 = rows.occ[1] ? rows.hi[1] - rows.lo[1] : 0;
+    rmax0 = max(max(__builtin_amdgcn_readlane(rcnt0, 0), __builtin_amdgcn_readlane(rcnt0, 16)),
+                max(__builtin_amdgcn_readlane(rcnt0, 32), __builtin_amdgcn_readlane(rcnt0, 48)));
+    rmax1 = max(max(__builtin_amdgcn_readlane(rcnt1, 0), __builtin_amdgcn_readlane(rcnt1, 16)),
+                max(__builtin_amdgcn_readlane(rcnt1, 32), __builtin_amdgcn_readlane(rcnt1, 48)));
+  };
   for (int slot = tr.first; slot < tr.end; slot += tr.stride) {
-    const int gtile = __builtin_amdgcn_readfirstlane(gtile_next);
-    if (slot + tr.stride < tr.end) gtile_next = a.active_tiles[slot + tr.stride];
-    const int sc = one_scene ? 0 : __builtin_amdgcn_readfirstlane(scene_of(a.T.tile_off, a.T.nscenes, gtile));
-    const DevParams& P = a.T.params[sc];
-    const P2GScene S = one_scene ? S1 : p2g_scene(P);
-    const int64_t noff = one_scene ? noff1 : a.T.node_off[sc];
-    const int tile = gtile - (one_scene ? toff1 : a.T.tile_off[sc]);
-    const int nt0 = one_scene ? nt0_1 : __builtin_amdgcn_readfirstlane(P.tiles[0]);
-    const int nt1 = one_scene ? nt1_1 : __builtin_amdgcn_readfirstlane(P.tiles[1]);
-    const int t0 = tile % nt0, t1 = (tile / nt0) % nt1, t2 = tile / (nt0 * nt1);
-    const int g2 = 4 * t2 + layer;
-    const int g0 = 4 * t0 + cx;  // this lane's cell of each row (both roles)
-    // the bins of this lane's cell in the wave's two rows, and each row's largest count (uniform)
-    int rstart0 = 0, rcnt0 = 0, rstart1 = 0, rcnt1 = 0;
-    {
-      const int g1a = 4 * t1 + 2 * half, g1b = g1a + 1;
-      if (g0 < S.res[0] && g2 < S.res[2]) {
-        if (g1a < S.res[1]) {
-          const int64_t key = noff + (g2 * S.res[1] + g1a) * S.res[0] + g0;
-          if (a.occ[key / SCAN_TILE]) {
-            rstart0 = a.cell_start[key];
-            rcnt0 = a.cell_end[key] - rstart0;
-          }
-        }
-        if (g1b < S.res[1]) {
-          const int64_t key = noff + (g2 * S.res[1] + g1b) * S.res[0] + g0;
-          if (a.occ[key / SCAN_TILE]) {
-            rstart1 = a.cell_start[key];
-            rcnt1 = a.cell_end[key] - rstart1;
-          }
-        }
-      }
+    const int g0 = 4 * rows.t0 + cx, t1 = rows.t1, g2 = 4 * rows.t2 + layer;  // this lane's cell of each row (both roles)
+    const P2GScene S = n.S;  // this tile's
+    take_rows();
+    if (slot + tr.stride < tr.end) {  // the next tile's cells
+      gtile = gtile_next;
+      gtile_next = tiles[min(slot + 2 * tr.stride, last)];
+      const int sc_next = scene_at(gtile);
+      if (sc_next != n.sc) n = tile_scene(a, sc_next);
+      rows = tile_rows(a, n, gtile, cx, layer, half);
     }
-    const int rmax0 = max(max(__builtin_amdgcn_readlane(rcnt0, 0), __builtin_amdgcn_readlane(rcnt0, 16)),
-                          max(__builtin_amdgcn_readlane(rcnt0, 32), __builtin_amdgcn_readlane(rcnt0, 48)));
-    const int rmax1 = max(max(__builtin_amdgcn_readlane(rcnt1, 0), __builtin_amdgcn_readlane(rcnt1, 16)),
-                          max(__builtin_amdgcn_readlane(rcnt1, 32), __builtin_amdgcn_readlane(rcnt1, 48)));
     auto rmax_of = [&](int r) { return r == 0 ? rmax0 : rmax1; };
     auto rcnt_of = [&](int r) { return r == 0 ? rcnt0 : rcnt1; };
     auto rstart_of = [&](int r) { return r == 0 ? rstart0 : rstart1; };
@@ -1304,22 +1332,6 @@ __global__ __launch_bounds__(64 * P2G_WAVES) void k_p2g(P2GArgs a) {
   }
 }
 
-// Constants of a tile's scene.
-struct TileScene {
-  P2GScene S;
-  int64_t noff;
-  int sc, toff, nt0, nt1;
-};
-__device__ __forceinline__ TileScene tile_scene(const P2GArgs& a, int sc) {
-  TileScene n;
-  n.sc = sc;
-  n.S = p2g_scene(a.T.params[sc]);
-  n.noff = a.T.node_off[sc];
-  n.toff = __builtin_amdgcn_readfirstlane(a.T.tile_off[sc]);
-  n.nt0 = __builtin_amdgcn_readfirstlane(a.T.params[sc].tiles[0]);
-  n.nt1 = __builtin_amdgcn_readfirstlane(a.T.params[sc].tiles[1]);
-  return n;
-}
 // The first cell of a wave's layer of a tile (uniform), and the lane's cell: occ, lo and hi as loaded (lo, hi
 // hold something else where occ is 0).
 struct TileCell {
@@ -1369,7 +1381,7 @@ __global__ __launch_bounds__(256, 3) void k_p2g_layer(P2GArgs a) {
   __shared__ float4 s_wave[4][WAVE_FLOATS / 4];
   static_assert(WAVE_FLOATS % 4 == 0 && (2 * NQ * SLAB) % 4 == 0, "float4 slots");
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int ntile = a.counters[CNT_TILES];
+  const int ntile = as_const(a.counters)[CNT_TILES];
   const int c = lane >> 2, sr = lane & 3, zo = lane & 3;  // staging (c, sr); accumulation (c, zo)
   const int cx = c & 3, cy = c >> 2;
   const float fzo = (float)zo;
@@ -1378,11 +1390,12 @@ __global__ __launch_bounds__(256, 3) void k_p2g_layer(P2GArgs a) {
   const XcdRange tr = xcd_range(ntile);
   if (tr.first >= tr.end) return;  // uniform: no tile for this workgroup
   auto scene_at = [&](int gtile) {
-    return a.T.nscenes == 1 ? 0 : __builtin_amdgcn_readfirstlane(scene_of(a.T.tile_off, a.T.nscenes, gtile));
+    return a.T.nscenes == 1 ? 0 : __builtin_amdgcn_readfirstlane(scene_of(as_const(a.T.tile_off), a.T.nscenes, gtile));
   };
   const int last = tr.first + (tr.end - 1 - tr.first) / tr.stride * tr.stride;  // this workgroup's last list entry
-  int gtile = __builtin_amdgcn_readfirstlane(a.active_tiles[tr.first]);
-  int gtile_next = a.active_tiles[min(tr.first + tr.stride, last)];
+  const auto tiles = as_const(a.active_tiles);
+  int gtile = tiles[tr.first];
+  int gtile_next = tiles[min(tr.first + tr.stride, last)];
   TileScene n = tile_scene(a, scene_at(gtile));
   TileCell cell = tile_cell(a, n, gtile, cx, cy, w);
   int start = cell.lo, cnt = cell.occ ? cell.hi - cell.lo : 0;
@@ -1392,8 +1405,8 @@ __global__ __launch_bounds__(256, 3) void k_p2g_layer(P2GArgs a) {
   if (sr < RANKS && RANKS + sr < cnt) pi2 = p2g_slot(a, start + RANKS + sr);
   for (int slot = tr.first; slot < tr.end; slot += tr.stride) {
     // the next tile's cells (the last tile's own again at the end: loaded, not used)
-    gtile = __builtin_amdgcn_readfirstlane(gtile_next);
-    gtile_next = a.active_tiles[min(slot + 2 * tr.stride, last)];
+    gtile = gtile_next;
+    gtile_next = tiles[min(slot + 2 * tr.stride, last)];
     const P2GScene S = n.S;  // this tile's
     const int sc_next = scene_at(gtile);
     if (sc_next != n.sc) n = tile_scene(a, sc_next);
@@ -1530,18 +1543,17 @@ template <int MODE>
 __global__ __launch_bounds__(64) void k_grid(GridArgs a) {
   if (clock_skip(a.clk)) return;
   const float dt = clock_dt(a.clk, a.dt);
-  const int nblk = a.counters[CNT_BLOCKS];
+  const int nblk = as_const(a.counters)[CNT_BLOCKS];
   float vmax = 0.0f;  // max |v| over this lane's nodes after the velocity update
   const int lx = threadIdx.x & 3, ly = (threadIdx.x >> 2) & 3, lz = threadIdx.x >> 4;
   const XcdRange br = xcd_range(nblk);
   for (int s = br.first; s < br.end; s += br.stride) {
-    const int gblk = a.active_blocks[s];
-    const int sc = __builtin_amdgcn_readfirstlane(scene_of(a.T.tile_off, a.T.nscenes, gblk));
-    const DevParams& P = a.T.params[sc];
-    const int toff = a.T.tile_off[sc];
+    const int gblk = as_const(a.active_blocks)[s];
+    const int sc = __builtin_amdgcn_readfirstlane(scene_of(as_const(a.T.tile_off), a.T.nscenes, gblk));
+    const auto& P = as_const(a.T.params)[sc];
+    const int toff = as_const(a.T.tile_off)[sc];
     const int blk = gblk - toff;
-    const int nt0 = __builtin_amdgcn_readfirstlane(P.tiles[0]), nt1 = __builtin_amdgcn_readfirstlane(P.tiles[1]),
-              nt2 = __builtin_amdgcn_readfirstlane(P.tiles[2]);
+    const int nt0 = P.tiles[0], nt1 = P.tiles[1], nt2 = P.tiles[2];
     const int b0 = blk % nt0, b1 = (blk / nt0) % nt1, b2 = blk / (nt0 * nt1);
     // the slots of the 27 tiles around the block (b - 1 .. b + 1 per axis), one lane each; every
     // node of the block is covered by tiles among them
@@ -1552,11 +1564,10 @@ __global__ __launch_bounds__(64) void k_grid(GridArgs a) {
       if (q < 27 && u0 >= 0 && u1 >= 0 && u2 >= 0 && u0 < nt0 && u1 < nt1 && u2 < nt2)
         slot27 = a.tile_slot[toff + (u2 * nt1 + u1) * nt0 + u0];
     }
-    const int r0 = __builtin_amdgcn_readfirstlane(P.res[0]), r1 = __builtin_amdgcn_readfirstlane(P.res[1]),
-              r2 = __builtin_amdgcn_readfirstlane(P.res[2]);
+    const int r0 = P.res[0], r1 = P.res[1], r2 = P.res[2];
     const int n0 = 4 * b0 + lx, n1 = 4 * b1 + ly, n2 = 4 * b2 + lz;
     const bool in_grid = n0 < r0 && n1 < r1 && n2 < r2;
-    const int64_t node = a.T.node_off[sc] + ((int64_t)n2 * r1 + n1) * r0 + n0;
+    const int64_t node = as_const(a.T.node_off)[sc] + ((int64_t)n2 * r1 + n1) * r0 + n0;
     const int nn[3] = {n0, n1, n2}, ntl[3] = {nt0, nt1, nt2};
     // covering tiles of this node along each axis: tlo and tlo + 1 (if <= thi), both in b - 1 .. b + 1
     int tlo[3], thi[3];
