@@ -315,9 +315,10 @@ void launch_fill_bins(hipStream_t s, const uint32_t* ks, int n, int64_t ncells, 
 enum SortMode : int { SORT_COUNTING = 0, SORT_RADIX = 1 };
 void launch_sort(hipStream_t s, const SortBufs& b, const uint32_t* keys_in, int n, int nblocks, int passes, int mode);
 // order: B-spline order of every scene (2 or 3); ranks: particles per cell staged per chunk (4 or 8)
-// pass P2G_ROWS (8-wave workgroups, ranks 4 or 8) or P2G_LAYERS (4-wave workgroups, ranks 2 or 4):
-// two schedules of the same sums in the same order, so every choice gives the same bits.
-enum P2GPass : int { P2G_ROWS = 0, P2G_LAYERS = 1 };
+// pass P2G_ROWS (8-wave workgroups, ranks 4 or 8), P2G_WIDE_ROWS (16-wave workgroups, 8 ranks; not a tuning) or
+// P2G_LAYERS (4-wave workgroups, ranks 2 or 4): schedules of the same sums in the same order, so every choice
+// gives the same bits.
+enum P2GPass : int { P2G_ROWS = 0, P2G_LAYERS = 1, P2G_WIDE_ROWS = 2 };
 void launch_p2g(hipStream_t s, const P2GArgs& a, int order, int mode, int grid, int ranks, int pass);
 void launch_grid(hipStream_t s, const GridArgs& a, int mode, int grid);
 // With ev_start set, the launch records the kernel's own start and end into ev_start / ev_stop.

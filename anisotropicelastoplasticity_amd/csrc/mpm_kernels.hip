@@ -799,7 +799,7 @@ constexpr int PAY_STRIDE = 52;
 template <int RANKS>
 constexpr int pay_cell() { return RANKS * PAY_STRIDE + 4; }
 constexpr int SLAB = FOOT * FOOT * 4;   // nodes of a wave's slab
-constexpr int P2G_WAVES = 8;            // waves per P2G workgroup: 4 cell layers x 2 row halves
+constexpr int P2G_SLABS = 8;            // slabs of a tile: 4 cell layers x 2 row halves
 // payload layout (floats): the x weights of window nodes c-1 .. c+2, the y and z weights and
 // derivatives (per cell width), the x-column terms g[ox][r] = ox wx[ox] Q[r][0] - dwx[ox] S[r][0]
 // that every lane of the cell adds with weight wy wz, the mass, q0 (a cloth vertex's force in the
@@ -1122,14 +1122,16 @@ __device__ __forceinline__ TileScene tile_scene(const P2GArgs& a, int sc) {
   n.nt1 = P->tiles[1];
   return n;
 }
-// A tile's first cell (uniform) and, of a wave's two rows, the lane's cells as loaded (lo, hi hold something else
-// where occ is 0).
+
+// A tile's first cell (uniform) and, of a wave's ROWS rows from row0, the lane's cells as loaded (lo, hi hold
+// something else where occ is 0), in one round trip.
 struct TileRows {
   int t0, t1, t2;
   uint32_t occ[2];
   int lo[2], hi[2];
 };
-__device__ __forceinline__ TileRows tile_rows(const P2GArgs& a, const TileScene& n, int gtile, int cx, int layer, int half) {
+template <int ROWS>
+__device__ __forceinline__ TileRows tile_rows(const P2GArgs& a, const TileScene& n, int gtile, int cx, int layer, int row0) {
   TileRows b;
   const int tile = gtile - n.toff;
   b.t0 = tile % n.nt0;
@@ -1137,8 +1139,8 @@ __device__ __forceinline__ TileRows tile_rows(const P2GArgs& a, const TileScene&
   b.t2 = tile / (n.nt0 * n.nt1);
   const int g0 = 4 * b.t0 + cx, g2 = 4 * b.t2 + layer;
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const int g1 = 4 * b.t1 + 2 * half + r;
+  for (int r = 0; r < ROWS; ++r) {
+    const int g1 = 4 * b.t1 + row0 + r;
     const bool in = g0 < n.S.res[0] && g1 < n.S.res[1] && g2 < n.S.res[2];
     const int64_t key = n.noff + (in ? (g2 * n.S.res[1] + g1) * n.S.res[0] + g0 : 0);
     b.occ[r] = a.occ[key / SCAN_TILE];
@@ -1150,24 +1152,27 @@ __device__ __forceinline__ TileRows tile_rows(const P2GArgs& a, const TileScene&
 }
 
 
-template <int ORDER, int MODE, int RANKS>
-__global__ __launch_bounds__(64 * P2G_WAVES) void k_p2g(P2GArgs a) {
+template <int ORDER, int MODE, int RANKS, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void k_p2g(P2GArgs a) {
   if (clock_skip(a.clk)) return;
   const float dt = clock_dt(a.clk, a.dt);
   constexpr int P2G_RANKS = RANKS;
   constexpr int PAY_CELL = pay_cell<RANKS>();
-  __shared__ float4 s_pay[P2G_WAVES][4 * PAY_CELL / 4];
-  __shared__ float s_slab[P2G_WAVES][4][SLAB];  // [wave][quantity][node]
+  constexpr int ROWS = 16 / WAVES;  // rows per wave
+  __shared__ float4 s_pay[WAVES][4 * PAY_CELL / 4];
+  __shared__ float s_slab[P2G_SLABS][4][SLAB];  // [layer + 4 row half][quantity][node]
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int layer = w & 3, half = w >> 2;  // wave w owns cell layer z = w & 3, rows 2 (w >> 2) and 2 (w >> 2) + 1
+  // wave w owns cell layer z = w & 3 and ROWS rows from row0
+  const int layer = w & 3, row0 = __builtin_amdgcn_readfirstlane(ROWS * (w >> 2));
   const int ntile = as_const(a.counters)[CNT_TILES];
   constexpr int NQ = (MODE == P2G_FORCE) ? 3 : 4;
   // staging role: lane (cx, sr), sr < RANKS; accumulation role: lane (cx, zo, oy)
   const int cx = lane >> 4, sr = lane & 15;
   const int zo = (lane >> 2) & 3, oy = lane & 3;
   const float foy = (float)oy, fzo = (float)zo;
-  float* slab = &s_slab[w][0][0];
-  for (int i = lane; i < 4 * SLAB; i += 64) slab[i] = 0.0f;
+  float* slab = &s_slab[layer + 4 * (row0 >> 1)][0][0];
+  for (int i = tid; i < P2G_SLABS * 4 * SLAB; i += 64 * WAVES) (&s_slab[0][0][0])[i] = 0.0f;
+  __syncthreads();
   // the tiles of one XCD are a contiguous range of the (ascending) active tiles
   const XcdRange tr = xcd_range(ntile);
   if (tr.first >= tr.end) return;  // uniform: no tile for this workgroup
@@ -1179,14 +1184,14 @@ __global__ __launch_bounds__(64 * P2G_WAVES) void k_p2g(P2GArgs a) {
   int gtile = tiles[tr.first];
   int gtile_next = tiles[min(tr.first + tr.stride, last)];
   TileScene n = tile_scene(a, scene_at(gtile));
-  TileRows rows = tile_rows(a, n, gtile, cx, layer, half);
-  // the lane's cell of each of the wave's two rows, and each row's largest count (uniform)
+  TileRows rows = tile_rows<ROWS>(a, n, gtile, cx, layer, row0);
+  // the lane's cell of each of the wave's rows, and each row's largest count (uniform)
   int rstart0, rcnt0, rstart1, rcnt1, rmax0, rmax1;
   auto take_rows = [&]() {
     rstart0 = rows.lo[0];
     rcnt0 = rows.occ[0] ? rows.hi[0] - rows.lo[0] : 0;
-    rstart1 = rows.lo[1];
-    rcnt1 = rows.occ[1] ? rows.hi[1] - rows.lo[1] : 0;
+    rstart1 = ROWS == 2 ? rows.lo[1] : 0;
+    rcnt1 = ROWS == 2 && rows.occ[1] ? rows.hi[1] - rows.lo[1] : 0;
     rmax0 = max(max(__builtin_amdgcn_readlane(rcnt0, 0), __builtin_amdgcn_readlane(rcnt0, 16)),
                 max(__builtin_amdgcn_readlane(rcnt0, 32), __builtin_amdgcn_readlane(rcnt0, 48)));
     rmax1 = max(max(__builtin_amdgcn_readlane(rcnt1, 0), __builtin_amdgcn_readlane(rcnt1, 16)),
@@ -1201,7 +1206,7 @@ __global__ __launch_bounds__(64 * P2G_WAVES) void k_p2g(P2GArgs a) {
       gtile_next = tiles[min(slot + 2 * tr.stride, last)];
       const int sc_next = scene_at(gtile);
       if (sc_next != n.sc) n = tile_scene(a, sc_next);
-      rows = tile_rows(a, n, gtile, cx, layer, half);
+      rows = tile_rows<ROWS>(a, n, gtile, cx, layer, row0);
     }
     auto rmax_of = [&](int r) { return r == 0 ? rmax0 : rmax1; };
     auto rcnt_of = [&](int r) { return r == 0 ? rcnt0 : rcnt1; };
@@ -1231,8 +1236,22 @@ __global__ __launch_bounds__(64 * P2G_WAVES) void k_p2g(P2GArgs a) {
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int q = 0; q < NQ; ++q) acc[i][q] = 0.0f;
+    // row sums into the slab: phase ox, node (cx + ox, cy + oy, zo)
+    auto add_row = [&](int cy) {
+#pragma unroll
+      for (int ox = 0; ox < 4; ++ox) {
+        const int ln = (cx + ox) + FOOT * (cy + oy) + FOOT * FOOT * zo;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {  // no other wave's at this time, and a different node per lane: no atomics
+          slab[q * SLAB + ln] += acc[ox][q];
+          acc[ox][q] = 0.0f;
+        }
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      }
+    };
     while (cr < 2) {
-      const int cy = 2 * half + cr;
+      const int cy = row0 + cr;
       const int g1 = 4 * t1 + cy;
       const int cnt = rcnt_of(cr), rstart = rstart_of(cr);
       // ---- stage ranks RANKS k .. RANKS k + RANKS - 1 of each cell of the row
@@ -1296,34 +1315,26 @@ __global__ __launch_bounds__(64 * P2G_WAVES) void k_p2g(P2GArgs a) {
       }
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      if (ncr != cr) {
-        // ---- row sums into the wave's slab: phase ox, node (cx + ox, cy + oy, zo)
-#pragma unroll
-        for (int ox = 0; ox < 4; ++ox) {
-          const int ln = (cx + ox) + FOOT * (cy + oy) + FOOT * FOOT * zo;
-#pragma unroll
-          for (int q = 0; q < NQ; ++q) {  // the wave's own slab, a different node per lane: no atomics
-            slab[q * SLAB + ln] += acc[ox][q];
-            acc[ox][q] = 0.0f;
-          }
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        }
-      }
+      if (ROWS == 2 && ncr != cr) add_row(cy);
       cr = ncr;
       k = nk;
+    }
+    if constexpr (ROWS == 1) {  // the two waves of a slab one after the other, in row order
+      if (row0 % 2 == 0 && rmax0 > 0) add_row(row0);
+      __syncthreads();
+      if (row0 % 2 == 1 && rmax0 > 0) add_row(row0);
     }
     __syncthreads();
     // ---- tile partial: node (X, Y, Z) = sum over layers l, 0 <= Z - l <= 3, ascending, and within a
     // layer over the row halves in order; slabs cleared
     float* part = a.partials + (size_t)slot * PART_STRIDE + (MODE == P2G_FORCE ? 4 * FOOT3 : 0);
-    for (int i = tid; i < FOOT3; i += 64 * P2G_WAVES) {
+    for (int i = tid; i < FOOT3; i += 64 * WAVES) {
       const int X = i % FOOT, Y = (i / FOOT) % FOOT, Z = i / (FOOT * FOOT);
       float s[NQ];
 #pragma unroll
       for (int q = 0; q < NQ; ++q) s[q] = 0.0f;
 #pragma unroll
-      for (int ww = 0; ww < P2G_WAVES; ++ww) {
+      for (int ww = 0; ww < P2G_SLABS; ++ww) {
         const int l = ww >> 1, hh = ww & 1, wv = l + 4 * hh;
         const int z = Z - l;
         if (z < 0 || z > 3) continue;
@@ -2749,17 +2760,17 @@ void launch_fill_bins(hipStream_t s, const uint32_t* ks, int n, int64_t ncells, 
   hipLaunchKernelGGL(k_fill_bins, dim3(blocks_for(ncells + 1, 256)), dim3(256), 0, s, ks, n, ncells, cell_start);
 }
 
-template <int RANKS>
+template <int RANKS, int WAVES>
 static void launch_p2g_r(hipStream_t s, const P2GArgs& a, int order, int mode, int grid) {
   if (mode == P2G_MOM_STRESS) {
-    if (order == 2) hipLaunchKernelGGL((k_p2g<2, P2G_MOM_STRESS, RANKS>), dim3(grid), dim3(64 * P2G_WAVES), 0, s, a);
-    else hipLaunchKernelGGL((k_p2g<3, P2G_MOM_STRESS, RANKS>), dim3(grid), dim3(64 * P2G_WAVES), 0, s, a);
+    if (order == 2) hipLaunchKernelGGL((k_p2g<2, P2G_MOM_STRESS, RANKS, WAVES>), dim3(grid), dim3(64 * WAVES), 0, s, a);
+    else hipLaunchKernelGGL((k_p2g<3, P2G_MOM_STRESS, RANKS, WAVES>), dim3(grid), dim3(64 * WAVES), 0, s, a);
   } else if (mode == P2G_MOM) {
-    if (order == 2) hipLaunchKernelGGL((k_p2g<2, P2G_MOM, RANKS>), dim3(grid), dim3(64 * P2G_WAVES), 0, s, a);
-    else hipLaunchKernelGGL((k_p2g<3, P2G_MOM, RANKS>), dim3(grid), dim3(64 * P2G_WAVES), 0, s, a);
+    if (order == 2) hipLaunchKernelGGL((k_p2g<2, P2G_MOM, RANKS, WAVES>), dim3(grid), dim3(64 * WAVES), 0, s, a);
+    else hipLaunchKernelGGL((k_p2g<3, P2G_MOM, RANKS, WAVES>), dim3(grid), dim3(64 * WAVES), 0, s, a);
   } else {
-    if (order == 2) hipLaunchKernelGGL((k_p2g<2, P2G_FORCE, RANKS>), dim3(grid), dim3(64 * P2G_WAVES), 0, s, a);
-    else hipLaunchKernelGGL((k_p2g<3, P2G_FORCE, RANKS>), dim3(grid), dim3(64 * P2G_WAVES), 0, s, a);
+    if (order == 2) hipLaunchKernelGGL((k_p2g<2, P2G_FORCE, RANKS, WAVES>), dim3(grid), dim3(64 * WAVES), 0, s, a);
+    else hipLaunchKernelGGL((k_p2g<3, P2G_FORCE, RANKS, WAVES>), dim3(grid), dim3(64 * WAVES), 0, s, a);
   }
 }
 
@@ -2781,9 +2792,11 @@ void launch_p2g(hipStream_t s, const P2GArgs& a, int order, int mode, int grid, 
   if (pass == P2G_LAYERS) {
     if (ranks == 2) launch_p2g_l<2>(s, a, order, mode, grid);
     else launch_p2g_l<4>(s, a, order, mode, grid);
+  } else if (pass == P2G_WIDE_ROWS) {
+    launch_p2g_r<8, 16>(s, a, order, mode, grid);
   } else {
-    if (ranks == 4) launch_p2g_r<4>(s, a, order, mode, grid);
-    else launch_p2g_r<8>(s, a, order, mode, grid);
+    if (ranks == 4) launch_p2g_r<4, 8>(s, a, order, mode, grid);
+    else launch_p2g_r<8, 8>(s, a, order, mode, grid);
   }
 }
 

@@ -137,6 +137,7 @@ struct mpm_ctx {
   int p2g_grid = 512;
   int p2g_ranks = 8;  // P2G staging chunk
   int p2g_pass = P2G_ROWS;  // P2G schedule
+  bool p2g_wide = false;    // rows by 16 waves (choose_p2g only)
   bool p2g_tuned = false;   // set by mpm_autotune or mpm_set_tuning (else choose_p2g does)
   // adaptive time step (mpm_solve): the device clock, and the pointer the kernels get (null for
   // fixed-step runs)
@@ -533,7 +534,10 @@ static GridArgs grid_args(mpm_ctx* ctx, float dt) {
 //   4,194,304  9,537       440   357 / 333       271
 // Cubic splines and predicted stress lie alike (681,472 particles, cubic: 77 / 80 against 60). A mesh crowds the
 // cells that it passes through, whatever the mean: 0.5 M sand particles on a 256 x 256-vertex cloth 89 / 89
-// against 99.
+// against 99. Where every tile has a CU to itself, 16 waves take its rows one each instead of two: 145 tiles of 2^15
+// particles 18.1 -> 16.7 us, 8 tiles (cubic, predicted stress: both passes) 50.5 -> 44.6; but 1,073 tiles 74 -> 85.
+// The line is at three tiles to four CUs, since the particles spread after the choice: a block on 216 tiles gains at
+// first (18.1 -> 16.5) and loses once it covers more than 256.
 static int choose_p2g(mpm_ctx* ctx) {
   if (ctx->p2g_tuned) return MPM_OK;
   int tiles = 0;
@@ -542,9 +546,12 @@ static int choose_p2g(mpm_ctx* ctx) {
   const bool layers = ctx->mesh.ne == 0 && tiles > ctx->n_cu && ctx->n <= 640LL * tiles;
   ctx->p2g_pass = layers ? P2G_LAYERS : P2G_ROWS;
   ctx->p2g_ranks = layers ? 4 : 8;
-  ctx->p2g_grid = std::max(128, ctx->n_cu * (layers ? 3 : tiles > 4 * ctx->n_cu ? 4 : 2));
+  ctx->p2g_wide = !layers && 4 * tiles <= 3 * ctx->n_cu;
+  ctx->p2g_grid = std::max(128, ctx->n_cu * (layers ? 3 : ctx->p2g_wide ? 1 : tiles > 4 * ctx->n_cu ? 4 : 2));
   return MPM_OK;
 }
+
+static int p2g_pass(const mpm_ctx* ctx) { return ctx->p2g_wide ? P2G_WIDE_ROWS : ctx->p2g_pass; }
 
 static int stage_p2g(mpm_ctx* ctx, float dt) {
   hipStream_t s = ctx->stream;
@@ -556,12 +563,12 @@ static int stage_p2g(mpm_ctx* ctx, float dt) {
       launch_stress_init(s, ctx->T, ctx->nblocks_p, ctx->state[ctx->cur], ctx->cap, ctx->n, ctx->fallbacks);
       ctx->stress_valid = true;
     }
-    launch_p2g(s, a, ctx->order, P2G_MOM_STRESS, ctx->p2g_grid, ctx->p2g_ranks, ctx->p2g_pass);
+    launch_p2g(s, a, ctx->order, P2G_MOM_STRESS, ctx->p2g_grid, ctx->p2g_ranks, p2g_pass(ctx));
   } else {
-    launch_p2g(s, a, ctx->order, P2G_MOM, ctx->p2g_grid, ctx->p2g_ranks, ctx->p2g_pass);
+    launch_p2g(s, a, ctx->order, P2G_MOM, ctx->p2g_grid, ctx->p2g_ranks, p2g_pass(ctx));
     launch_grid(s, grid_args(ctx, dt), GRID_NORMALIZE, ctx->grid_grid);
     launch_stress_predicted(s, a, ctx->order, ctx->nblocks_p);
-    launch_p2g(s, a, ctx->order, P2G_FORCE, ctx->p2g_grid, ctx->p2g_ranks, ctx->p2g_pass);
+    launch_p2g(s, a, ctx->order, P2G_FORCE, ctx->p2g_grid, ctx->p2g_ranks, p2g_pass(ctx));
   }
   return MPM_OK;
 }
@@ -1362,7 +1369,7 @@ int mpm_estimate_volumes(mpm_ctx* ctx) {
   rc = stage_sort(ctx);
   if (rc) return rc;
   P2GArgs a = p2g_args(ctx, 0.0f);
-  launch_p2g(ctx->stream, a, ctx->order, P2G_MOM, ctx->p2g_grid, ctx->p2g_ranks, ctx->p2g_pass);
+  launch_p2g(ctx->stream, a, ctx->order, P2G_MOM, ctx->p2g_grid, ctx->p2g_ranks, p2g_pass(ctx));
   launch_grid(ctx->stream, grid_args(ctx, 0.0f), GRID_NORMALIZE, ctx->grid_grid);
   launch_volumes(ctx->stream, ctx->T, ctx->order, ctx->nblocks_p, ctx->state[ctx->cur], ctx->cap, ctx->n, ctx->grid);
   ctx->stress_valid = false;
@@ -1488,7 +1495,7 @@ int mpm_solve(mpm_ctx* ctx, double cfl, double maxt, mpm_frame_callback cb, void
   // first Dt from the velocities p/m of a P2G without forces
   rc = stage_sort(ctx);
   if (rc) return rc;
-  launch_p2g(ctx->stream, p2g_args(ctx, 0.0f), ctx->order, P2G_MOM, ctx->p2g_grid, ctx->p2g_ranks, ctx->p2g_pass);
+  launch_p2g(ctx->stream, p2g_args(ctx, 0.0f), ctx->order, P2G_MOM, ctx->p2g_grid, ctx->p2g_ranks, p2g_pass(ctx));
   GridArgs g0 = grid_args(ctx, 0.0f);
   g0.vmax_out = &ctx->clock->vmax_bits;
   launch_grid(ctx->stream, g0, GRID_NORMALIZE, ctx->grid_grid);
@@ -1646,6 +1653,7 @@ int mpm_autotune(mpm_ctx* ctx, float dt, int32_t reps, mpm_tuning* chosen) {
   ctx->p2g_grid = best.p2g_blocks;
   ctx->p2g_pass = best.p2g_pass;
   ctx->p2g_tuned = true;
+  ctx->p2g_wide = false;
   ctx->grid_grid = best.grid_blocks;
   drop_graphs(ctx);
   if (chosen) *chosen = best;
@@ -1681,6 +1689,7 @@ int mpm_set_tuning(mpm_ctx* ctx, const mpm_tuning* t) {
   ctx->sort_mode = t->sort_mode;
   ctx->p2g_pass = t->p2g_pass;
   ctx->p2g_tuned = true;
+  ctx->p2g_wide = false;
   drop_graphs(ctx);
   return MPM_OK;
 }
