@@ -559,41 +559,42 @@ __device__ __forceinline__ void claim_block(const SortBufs& a, int b) {
   }
 }
 
-// The scan blocks' totals (workgroups below nscan) and the tile lists (the others): independent of each other,
-// so one launch hides one's latency behind the other's. With the counts made by G2P a substep sorts in four
-// launches (this one, scan, scatter, rank) where a separate count, totals and claim took six: sort 117 -> 83 us and
-// G2P 356 -> 328 at 2^22 particles (of which 55 us less by the cell_key changes), sort 30 -> 22 us at 2^15.
-__global__ __launch_bounds__(256) void k_sums_claim(SortBufs a, int nscan) {
-  if (clock_skip(a.clk)) return;
-  const int b = (int)blockIdx.x;
-  if (b < nscan) {
-    if (b == 0 && threadIdx.x < 2) a.counters_clear[threadIdx.x] = 0;
-    if (b == 0 && threadIdx.x == 2) *a.cand_count = 0;
-    sum_block(a, b);
-  } else {
-    claim_block(a, b - nscan);
-  }
-}
-
 // Exclusive scan of the cell counts into cell_start[0 .. ncells]: block b starts at the sum of the
-// totals of the blocks before it (read and summed by the block itself) and scans its SCAN_TILE cells; the blocks are independent. A block without particles writes nothing: its cells are
-// empty, which every reader learns from scan_flag (the getter of the bins fills them, k_fill_bins). A
+// totals of the blocks before it (read and summed by the block itself) and scans its SCAN_TILE cells;
+// the blocks are independent. A block without particles writes nothing: its cells are empty, which every reader learns from scan_flag (the getter of the bins fills them, k_fill_bins). A
 // block with particles also writes the start of the next block's first cell (its own end), which
 // the next block, if it has particles, writes with the same value. The last block writes
 // cell_start[ncells].
-__global__ __launch_bounds__(256) void k_cell_scan(const int* __restrict__ cnt, int64_t ncells, int* __restrict__ cell_start,
-                                                   const uint32_t* __restrict__ agg, const uint8_t* __restrict__ flag,
-                                                   const Clock* clk) {
-  if (clock_skip(clk)) return;
+// With few scan blocks (SMALL) a block adds up the cells of the occupied blocks before it, instead of reading
+// their totals.
+template <bool SMALL>
+__device__ __forceinline__ void scan_block(const SortBufs& a, int b) {
+  const int* cnt = a.bins.cell_count;
+  const int64_t ncells = a.ncells;
+  int* cell_start = a.cell_start;
   __shared__ uint32_t s_wsum[4];
   __shared__ uint32_t s_boff[4];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int b = blockIdx.x;
   const bool last = (int64_t)(b + 1) * SCAN_TILE >= ncells;
-  if (!flag[b] && !last) return;
+  if (SMALL && tid == 0) a.scan_flag_clear[b] = 0;
+  if (!a.bins.scan_flag[b] && !last) return;
   {
     uint32_t p = 0;
-    for (int q = tid; q < b; q += 256) p += agg[q];
+    if constexpr (SMALL) {
+      // every fourth of them a wave, with all of a block's loads in flight (every block before b is whole)
+      uint64_t todo = __ballot(lane < b && a.bins.scan_flag[lane < b ? lane : 0]);
+      for (int r = 0; todo; ++r, todo &= todo - 1) {
+        if ((r & 3) != w) continue;
+        const int4* p4 = reinterpret_cast<const int4*>(cnt + (int64_t)(__ffsll((long long)todo) - 1) * SCAN_TILE);
+#pragma unroll
+        for (int q = 0; q < SCAN_TILE / 256; ++q) {
+          const int4 v = p4[64 * q + lane];
+          p += (uint32_t)v.x + (uint32_t)v.y + (uint32_t)v.z + (uint32_t)v.w;
+        }
+      }
+    } else {
+      for (int q = tid; q < b; q += 256) p += a.scan_sum[q];
+    }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) p += __shfl_xor(p, off);
     if (lane == 0) s_boff[w] = p;
@@ -649,6 +650,32 @@ __global__ __launch_bounds__(256) void k_cell_scan(const int* __restrict__ cnt, 
   }
   if (base < ncells && base + SCAN_IPT >= ncells) cell_start[ncells] = (int)run;  // the total
   if (tid == 255 && !last) cell_start[(int64_t)(b + 1) * SCAN_TILE] = (int)run;  // the next block's first cell
+}
+
+// The scan blocks' totals (workgroups below nscan) and the tile lists (the others): independent of each other,
+// so one launch hides one's latency behind the other's. With the counts made by G2P a substep sorts in four
+// launches (this one, scan, scatter, rank) where a separate count, totals and claim took six: sort 117 -> 83 us and
+// G2P 356 -> 328 at 2^22 particles (of which 55 us less by the cell_key changes), sort 30 -> 22 us at 2^15.
+// Up to SMALL_SCAN scan blocks (a 64^3 grid's), the scan itself takes the totals' place and the sort has three launches:
+// 30 substeps of 2^15 particles on 64^3 1.50 -> 1.46 ms, 20 of a tiny scene on 24^3 1.59 -> 1.54.
+constexpr int SMALL_SCAN = 64;
+template <bool SMALL>
+__global__ __launch_bounds__(256) void k_sums_claim(SortBufs a, int nscan) {
+  if (clock_skip(a.clk)) return;
+  const int b = (int)blockIdx.x;
+  if (b < nscan) {
+    if (b == 0 && threadIdx.x < 2) a.counters_clear[threadIdx.x] = 0;
+    if (b == 0 && threadIdx.x == 2) *a.cand_count = 0;
+    if constexpr (SMALL) scan_block<true>(a, b);
+    else sum_block(a, b);
+  } else {
+    claim_block(a, b - nscan);
+  }
+}
+
+__global__ __launch_bounds__(256) void k_cell_scan(SortBufs a) {
+  if (clock_skip(a.clk)) return;
+  scan_block<false>(a, (int)blockIdx.x);
 }
 
 // The bins of the last sort for the host: cell_start[c] = the first sorted position whose key is at
@@ -2721,9 +2748,13 @@ void launch_count(hipStream_t s, const SceneTable& T, const BinCounts& b, const 
 void launch_sort(hipStream_t s, const SortBufs& b, const uint32_t* keys_in, int n, int nblocks, int passes, int mode) {
   if (n <= 0) return;
   const int nscan = blocks_for(b.ncells, SCAN_TILE);
-  hipLaunchKernelGGL(k_sums_claim, dim3(nscan + blocks_for(b.ntiles, 256)), dim3(256), 0, s, b, nscan);
-  hipLaunchKernelGGL(k_cell_scan, dim3(nscan), dim3(256), 0, s, b.bins.cell_count, b.ncells, b.cell_start, b.scan_sum,
-                     b.bins.scan_flag, b.clk);
+  const dim3 first(nscan + blocks_for(b.ntiles, 256));
+  if (nscan <= SMALL_SCAN) {
+    hipLaunchKernelGGL(k_sums_claim<true>, first, dim3(256), 0, s, b, nscan);
+  } else {
+    hipLaunchKernelGGL(k_sums_claim<false>, first, dim3(256), 0, s, b, nscan);
+    hipLaunchKernelGGL(k_cell_scan, dim3(nscan), dim3(256), 0, s, b);
+  }
   if (mode == SORT_COUNTING) {
     uint32_t* kf = (passes & 1) ? b.k1 : b.k2;  // the result goes where the digit passes put it
     int* vf = (passes & 1) ? b.v1 : b.v2;

@@ -144,3 +144,32 @@ def test_read_between_stages(kind):
             assert np.array_equal(some.view(np.uint32), outs[-1]["B"].view(np.uint32))
     for k in KEYS:
         assert np.array_equal(outs[0][k].view(np.uint32), outs[1][k].view(np.uint32)), k
+
+
+@pytest.mark.parametrize("res", [(16, 16, 16), (17, 16, 16), (15, 16, 17), (64, 64, 64), (64, 64, 65), (63, 65, 64)])
+@pytest.mark.parametrize("spread", ["everywhere", "ends"])
+def test_scan_of_sparse_grids(res, spread):
+    # scan blocks of 4096 cells: one, a last one of few cells, 64 (the most that one launch scans) and 65; particles
+    # in every block or only in the first and last cells
+    rng = np.random.default_rng(sum(res))
+    n, cells = 5000, int(np.prod(res))
+    key = rng.integers(0, cells, n) if spread == "everywhere" else np.where(rng.random(n) < 0.5, rng.integers(0, 40, n),
+                                                                            cells - 1 - rng.integers(0, 40, n))
+    c = np.stack([key % res[0], key // res[0] % res[1], key // (res[0] * res[1])])
+    x = ((c + rng.uniform(0.1, 0.9, (3, n))) / np.array(res)[:, None]).astype(np.float32)
+    with Solver(0) as s:
+        s.set_grid((0, 0, 0), (1, 1, 1), res)
+        s.set_params(scenes.sand_params())
+        s.set_particles(x, np.ones(n, np.float32))
+        for _ in range(2):
+            s.stage(_lib.STAGE_SORT, 0.0)
+            keys, ids, bins = s.get_sorted()
+            order = np.lexsort((np.arange(n), key))
+            assert np.array_equal(ids, order) and np.array_equal(keys, key[order])
+            assert np.array_equal(bins, np.concatenate([[0], np.cumsum(np.bincount(key, minlength=cells))]))
+            tiles = np.unique((c[2] // 4 * 100 + c[1] // 4) * 100 + c[0] // 4)
+            assert s.stats()["n_active_tiles"] == len(tiles)
+            for st in (_lib.STAGE_P2G, _lib.STAGE_GRID, _lib.STAGE_G2P):
+                s.stage(st, 0.0)
+            p = s.get_particles()
+            assert np.array_equal(p["x"], x)
