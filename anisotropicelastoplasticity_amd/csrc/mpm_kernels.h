@@ -265,7 +265,7 @@ struct ApexArgs {
   unsigned long long* fallback_apex;
   const Clock* clk;
 };
-constexpr int APEX_GROUP = 16;  // largest group
+constexpr int APEX_GROUP = 32;  // largest group
 void launch_apex_finish(hipStream_t s, ApexArgs a, int n_cu);
 
 // Planes of a deferred particle's trial SVD (surrogate candidates and FP64 apex projections). k_g2p

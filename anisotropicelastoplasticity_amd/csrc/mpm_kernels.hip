@@ -2167,9 +2167,11 @@ __global__ __launch_bounds__(256) void k_g2p(G2PArgs a) {
 // buffer. The result equals computing it inside k_g2p.
 //
 // A workgroup takes the masks of `gw` G2P waves at a time (4, a G2P workgroup's, where that gives few groups;
-// else 16, which gathers fuller waves), lists their flagged positions in LDS and works the list off. Bound by
-// the launch and one round trip of the masks where few particles are flagged. (With a list over all waves, made by
-// two launches before this one, G2P to here took 95 us instead of 92 at 2^20 particles, 177 instead of 171 for 16 scenes.)
+// else 32, which gathers fuller waves), lists their flagged positions in LDS and works the list off. Bound by
+// the launch and one round trip of the masks where few particles are flagged, and by scattered writes where many
+// are (410k of 2^22: 63 us; in groups of 16 and 64 waves 65-68 and 72, with two list launches before it and waves
+// filled over the whole state 53 + 11). With few flagged, G2P and what follows it took 95 us with the list launches
+// and 92 without at 2^20 particles, 177 and 171 for 16 scenes.
 __global__ __launch_bounds__(256) void k_apex_finish(ApexArgs a) {
   if (clock_skip(a.clk)) return;
   __shared__ int s_slot[64 * APEX_GROUP], s_idx[64 * APEX_GROUP];
@@ -2918,7 +2920,7 @@ void launch_surrogate(hipStream_t s, const SurrogateArgs& a, int n_cu, hipEvent_
 void launch_apex_finish(hipStream_t s, ApexArgs a, int n_cu) {
   const int small = blocks_for(a.nwaves, 4);
   a.gw = small <= 8 * n_cu ? 4 : APEX_GROUP;
-  hipLaunchKernelGGL(k_apex_finish, dim3(a.gw == 4 ? small : std::min(8 * n_cu, blocks_for(a.nwaves, APEX_GROUP))),
+  hipLaunchKernelGGL(k_apex_finish, dim3(a.gw == 4 ? small : std::min(4 * n_cu, blocks_for(a.nwaves, APEX_GROUP))),
                      dim3(256), 0, s, a);
 }
 
