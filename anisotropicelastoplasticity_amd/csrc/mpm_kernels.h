@@ -363,12 +363,14 @@ struct ClothArgs {
   const float* thr;
   int* status;
   unsigned long long* fallback;
+  unsigned long long* fallback_next;  // of element forces that the next P2G will use
   const Clock* clk;
 };
 void launch_cloth_rest(hipStream_t s, const ClothArgs& a, float* rest);  // rest in-plane R from the directions
-void launch_cloth_forces(hipStream_t s, const ClothArgs& a);   // element forces, then the per-vertex sums
+void launch_cloth_element_forces(hipStream_t s, const ClothArgs& a);
+void launch_cloth_vertex_forces(hipStream_t s, const ClothArgs& a);  // the per-vertex sums of the element forces
 void launch_cloth_fixed(hipStream_t s, const ClothArgs& a);    // after the grid update
-void launch_cloth_elements(hipStream_t s, const ClothArgs& a); // after G2P: positions, velocities, D, return map
+void launch_cloth_elements(hipStream_t s, const ClothArgs& a); // after G2P: positions, velocities, D, return map, forces
 void surrogate_set_smem_limit();
 // List of the sorted positions that G2P flagged (mask[w] of wave w, whose lane 0 sits at wpos[w]), in
 // ascending order and built without atomics; its length goes to *count.

@@ -2465,6 +2465,16 @@ __global__ __launch_bounds__(MLP_FWD_THREADS) void k_surrogate(SurrogateArgs a) 
 // ================================================================== cloth
 // Element forces from the current directions (per element), then each vertex sums the forces of
 // its incident elements in ascending element order (deterministic).
+__device__ __forceinline__ void element_forces(const ClothArgs& a, int e, const float* D, float vol, int& fb) {
+  float fv[9], M[9];
+  cloth_element_forces(a.P, D, a.rest + 9 * (size_t)e, vol, fv, M, fb);
+#pragma unroll
+  for (int i = 0; i < 9; ++i) {
+    a.elem_fv[9 * (size_t)e + i] = fv[i];
+    a.elem_stress[9 * (size_t)e + i] = M[i];
+  }
+}
+// The element forces of directions that no substep has advanced; else k_cloth_elements has formed them.
 __global__ __launch_bounds__(256) void k_cloth_element_forces(ClothArgs a) {
   if (clock_skip(a.clk)) return;
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2472,15 +2482,10 @@ __global__ __launch_bounds__(256) void k_cloth_element_forces(ClothArgs a) {
   if (e < a.ne) {
     const DevParams& P = a.P;
     const int pi = clamp_index(a.pos[P.mesh_e0 + e], a.n);
-    float D[9], fv[9], M[9];
+    float D[9];
 #pragma unroll
     for (int i = 0; i < 9; ++i) D[i] = a.st[(PF + i) * a.cap + pi];
-    cloth_element_forces(P, D, a.rest + 9 * (size_t)e, a.st[PVOL * a.cap + pi], fv, M, fb);
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-      a.elem_fv[9 * (size_t)e + i] = fv[i];
-      a.elem_stress[9 * (size_t)e + i] = M[i];
-    }
+    element_forces(a, e, D, a.st[PVOL * a.cap + pi], fb);
   }
   if (fb) atomicAdd(a.fallback, (unsigned long long)fb);
 }
@@ -2503,6 +2508,10 @@ __global__ __launch_bounds__(256) void k_cloth_rest(ClothArgs a, float* __restri
 __global__ __launch_bounds__(256) void k_cloth_vertex_forces(ClothArgs a) {
   if (clock_skip(a.clk)) return;
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v == 0 && *a.fallback_next) {  // the element forces are used now
+    *a.fallback += *a.fallback_next;
+    *a.fallback_next = 0;
+  }
   if (v >= a.nv) return;
   float f[3] = {0.0f, 0.0f, 0.0f};
   for (int k = a.vcsr_off[v]; k < a.vcsr_off[v + 1]; ++k) {
@@ -2567,7 +2576,7 @@ __global__ __launch_bounds__(64) void k_cloth_fixed(ClothArgs a) {
 __global__ __launch_bounds__(256) void k_cloth_elements(ClothArgs a) {
   if (clock_skip(a.clk)) return;
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  int fb = 0, oob = 0;
+  int fb = 0, fb_next = 0, oob = 0;
   const DevParams& P = a.P;
   const CellThr thr = cell_thr(a.thr, P.res);
   if (e < a.ne) {
@@ -2578,6 +2587,7 @@ __global__ __launch_bounds__(256) void k_cloth_elements(ClothArgs a) {
 #pragma unroll
     for (int c = 0; c < 3; ++c) pv[c] = clamp_index(a.pos[clamp_index(a.faces[3 * e + c], a.n)], a.n);
     float xv[3][3], vv[3][3], d3[3];
+    const float vol = a.st[PVOL * a.cap + pe];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       d3[d] = a.st[(PF + 3 * d + 2) * a.cap + pe];
@@ -2600,6 +2610,9 @@ __global__ __launch_bounds__(256) void k_cloth_elements(ClothArgs a) {
     cloth_return_map(P, D, fb);
 #pragma unroll
     for (int i = 0; i < 9; ++i) a.st[(PF + i) * a.cap + pe] = D[i];
+    // the forces that the next P2G scatters, from D while it is at hand (a lookup, ten scattered loads and a launch
+    // fewer: 30 substeps of 0.69 M entries with a 256 x 256-vertex cloth 8.27 -> 7.93 ms)
+    element_forces(a, e, D, vol, fb_next);
     int cell[3];
     const uint32_t key = cell_key(P, thr, xe[0], xe[1], xe[2], oob, cell);
     const CountTicket ticket = count_wave(a.bins, true, key, tile_of(P, cell[0], cell[1], cell[2]));
@@ -2607,6 +2620,7 @@ __global__ __launch_bounds__(256) void k_cloth_elements(ClothArgs a) {
     a.bins.rank[pe] = count_rank(ticket);
   }
   if (fb) atomicAdd(a.fallback, (unsigned long long)fb);
+  if (fb_next) atomicAdd(a.fallback_next, (unsigned long long)fb_next);
   if (oob) atomicOr(a.status, MPM_STATUS_OUT_OF_DOMAIN);
 }
 
@@ -2932,10 +2946,12 @@ void launch_cloth_rest(hipStream_t s, const ClothArgs& a, float* rest) {
   if (a.ne > 0) hipLaunchKernelGGL(k_cloth_rest, dim3(blocks_for(a.ne, 256)), dim3(256), 0, s, a, rest);
 }
 
-void launch_cloth_forces(hipStream_t s, const ClothArgs& a) {
-  if (a.ne <= 0) return;
-  hipLaunchKernelGGL(k_cloth_element_forces, dim3(blocks_for(a.ne, 256)), dim3(256), 0, s, a);
-  hipLaunchKernelGGL(k_cloth_vertex_forces, dim3(blocks_for(a.nv, 256)), dim3(256), 0, s, a);
+void launch_cloth_element_forces(hipStream_t s, const ClothArgs& a) {
+  if (a.ne > 0) hipLaunchKernelGGL(k_cloth_element_forces, dim3(blocks_for(a.ne, 256)), dim3(256), 0, s, a);
+}
+
+void launch_cloth_vertex_forces(hipStream_t s, const ClothArgs& a) {
+  if (a.nv > 0) hipLaunchKernelGGL(k_cloth_vertex_forces, dim3(blocks_for(a.nv, 256)), dim3(256), 0, s, a);
 }
 
 void launch_cloth_fixed(hipStream_t s, const ClothArgs& a) {

@@ -56,6 +56,7 @@ struct MeshHost {
   float* vert_force = nullptr; // device: [v][3]
   int* fixed = nullptr;        // device: fixed vertex caller ids
   int nfixed = 0;
+  bool forces_valid = false;   // elem_fv and elem_stress belong to the elements of state[cur]
 };
 
 struct mpm_ctx {
@@ -126,7 +127,7 @@ struct mpm_ctx {
   // counters and statistics
   int* counters = nullptr;
   int* status = nullptr;
-  unsigned long long* fallbacks = nullptr;  // [0] svd, [1] apex, [2] node count scratch
+  unsigned long long* fallbacks = nullptr;  // [0] svd, [1] apex, [2] node count scratch, [3] svd of the next cloth forces
   int64_t substeps = 0;
   int next_stage = MPM_STAGE_SORT;
 
@@ -331,6 +332,7 @@ static int upload_table(mpm_ctx* ctx) {
   }
   ctx->order = dp[0].order;
   ctx->predicted = dp[0].predicted;
+  ctx->mesh.forces_valid = false;
   ctx->nblocks_p = pblock_off[S];
   auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
   const size_t o_dp = 0, o_part = al(o_dp + sizeof(DevParams) * S), o_pb = al(o_part + sizeof(int) * (S + 1));
@@ -474,6 +476,7 @@ static ClothArgs cloth_args(mpm_ctx* ctx, int b) {
   c.thr = ctx->thr;
   c.status = ctx->status;
   c.fallback = ctx->fallbacks;
+  c.fallback_next = ctx->fallbacks + 3;
   c.clk = ctx->clk_active;
   return c;
 }
@@ -551,13 +554,26 @@ static int choose_p2g(mpm_ctx* ctx) {
   return MPM_OK;
 }
 
+// The cloth's element forces of state[cur]: k_cloth_elements leaves them for the next substep; a new mesh's or
+// changed parameters' are formed here.
+static void ensure_forces(mpm_ctx* ctx) {
+  if (ctx->mesh.ne <= 0 || ctx->mesh.forces_valid) return;
+  ensure_pos(ctx);
+  (void)hipMemsetAsync(ctx->fallbacks + 3, 0, sizeof(unsigned long long), ctx->stream);  // never while capturing
+  launch_cloth_element_forces(ctx->stream, cloth_args(ctx, ctx->cur));
+  ctx->mesh.forces_valid = true;
+}
+
 static int p2g_pass(const mpm_ctx* ctx) { return ctx->p2g_wide ? P2G_WIDE_ROWS : ctx->p2g_pass; }
 
 static int stage_p2g(mpm_ctx* ctx, float dt) {
   hipStream_t s = ctx->stream;
   P2GArgs a = p2g_args(ctx, dt);
   // cloth forces from the current directions (HybridSolver.cpp:370-455), read by the P2G staging
-  if (ctx->mesh.ne > 0) launch_cloth_forces(s, cloth_args(ctx, ctx->cur));
+  if (ctx->mesh.ne > 0) {
+    ensure_forces(ctx);
+    launch_cloth_vertex_forces(s, cloth_args(ctx, ctx->cur));
+  }
   if (!ctx->predicted) {
     if (!ctx->stress_valid) {
       launch_stress_init(s, ctx->T, ctx->nblocks_p, ctx->state[ctx->cur], ctx->cap, ctx->n, ctx->fallbacks);
@@ -668,6 +684,7 @@ static int stage_g2p(mpm_ctx* ctx, float dt) {
   }
   // cloth elements follow their vertices (positions, velocities, d1 d2) and are return-mapped
   if (ctx->mesh.ne > 0) launch_cloth_elements(ctx->stream, cloth_args(ctx, 1 - ctx->cur));
+  ctx->mesh.forces_valid = ctx->mesh.ne > 0;
   if (ctx->clk_active) launch_clock_end(ctx->stream, ctx->clk_active);
   ctx->cur = 1 - ctx->cur;
   ctx->keys_valid = true;
@@ -1420,6 +1437,7 @@ int mpm_run(mpm_ctx* ctx, float dt, int32_t nsteps) {
       rc = choose_p2g(ctx);
       if (rc) return rc;
       ensure_counts(ctx);  // a captured pair starts at the scan of what the G2P before it counted
+      ensure_forces(ctx);
       hipGraph_t g = nullptr;
       const int64_t steps0 = ctx->substeps;
       const int sort0 = ctx->sort_buf;
@@ -1444,6 +1462,7 @@ int mpm_run(mpm_ctx* ctx, float dt, int32_t nsteps) {
       ctx->cur = c0;  // capture did not execute anything
     }
     ensure_counts(ctx);
+    ensure_forces(ctx);
     for (int i = 0; i < pairs; ++i) CK(hipGraphLaunch(ctx->graph[c0], ctx->stream));
     ctx->substeps += 2 * pairs;
     ctx->sort_buf = 1 - c0;
@@ -1514,6 +1533,7 @@ int mpm_solve(mpm_ctx* ctx, double cfl, double maxt, mpm_frame_callback cb, void
         rc = choose_p2g(ctx);
         if (rc) return rc;
         ensure_counts(ctx);
+        ensure_forces(ctx);
         hipGraph_t gr = nullptr;
         const int64_t steps0 = ctx->substeps;
         const int sort0 = ctx->sort_buf;
@@ -1535,6 +1555,7 @@ int mpm_solve(mpm_ctx* ctx, double cfl, double maxt, mpm_frame_callback cb, void
         if (ei != hipSuccess) return fail(ctx, MPM_ERR_HIP, std::string("graph instantiate: ") + hipGetErrorString(ei));
       }
       ensure_counts(ctx);
+      ensure_forces(ctx);
       const double left = dt_last > 0.0 ? (1.0 / 60.0 - h.inner) / dt_last : 0.0;
       const int pairs = std::max(1, (int)std::min(left / 2.0, (double)SOLVE_PAIRS));
       for (int i = 0; i < pairs; ++i) CK(hipGraphLaunch(ctx->graph_adapt[c0], ctx->stream));
