@@ -42,9 +42,6 @@ __device__ __forceinline__ int clamp_index(int i, int n) { return i < 0 ? 0 : (i
 __device__ __forceinline__ float plane_load(const float* plane, uint32_t i) {
   return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(plane) + (size_t)(uint32_t)(4u * i));
 }
-__device__ __forceinline__ void plane_store(float* plane, uint32_t i, float v) {
-  *reinterpret_cast<float*>(reinterpret_cast<char*>(plane) + (size_t)(uint32_t)(4u * i)) = v;
-}
 
 // wave-uniform float held in a scalar register (the readfirstlane builtin works on 32-bit integers)
 __device__ __forceinline__ float uniform_f(float x) {
@@ -1280,7 +1277,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_p2g(P2GArgs a) {
     while (cr < 2) {
       const int cy = row0 + cr;
       const int g1 = 4 * t1 + cy;
-      const int cnt = rcnt_of(cr), rstart = rstart_of(cr);
+      const int cnt = rcnt_of(cr);
       // ---- stage ranks RANKS k .. RANKS k + RANKS - 1 of each cell of the row
       if (sr < P2G_RANKS) {
         const int rank = P2G_RANKS * k + sr;
