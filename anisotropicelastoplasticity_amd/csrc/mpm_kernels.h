@@ -315,7 +315,7 @@ void launch_fill_bins(hipStream_t s, const uint32_t* ks, int n, int64_t ncells, 
 enum SortMode : int { SORT_COUNTING = 0, SORT_RADIX = 1 };
 void launch_sort(hipStream_t s, const SortBufs& b, const uint32_t* keys_in, int n, int nblocks, int passes, int mode);
 // order: B-spline order of every scene (2 or 3); ranks: particles per cell staged per chunk (4 or 8)
-// pass P2G_ROWS (8-wave workgroups, ranks 4 or 8), P2G_WIDE_ROWS (16-wave workgroups, 8 ranks; not a tuning) or
+// pass P2G_ROWS (8-wave workgroups, ranks 4 or 8), P2G_WIDE_ROWS (16-wave workgroups, 8 ranks) or
 // P2G_LAYERS (4-wave workgroups, ranks 2 or 4): schedules of the same sums in the same order, so every choice
 // gives the same bits.
 enum P2GPass : int { P2G_ROWS = 0, P2G_LAYERS = 1, P2G_WIDE_ROWS = 2 };

@@ -138,7 +138,6 @@ struct mpm_ctx {
   int p2g_grid = 512;
   int p2g_ranks = 8;  // P2G staging chunk
   int p2g_pass = P2G_ROWS;  // P2G schedule
-  bool p2g_wide = false;    // rows by 16 waves (choose_p2g only)
   bool p2g_tuned = false;   // set by mpm_autotune or mpm_set_tuning (else choose_p2g does)
   // adaptive time step (mpm_solve): the device clock, and the pointer the kernels get (null for
   // fixed-step runs)
@@ -549,8 +548,9 @@ static int choose_p2g(mpm_ctx* ctx) {
   const bool layers = ctx->mesh.ne == 0 && tiles > ctx->n_cu && ctx->n <= 640LL * tiles;
   ctx->p2g_pass = layers ? P2G_LAYERS : P2G_ROWS;
   ctx->p2g_ranks = layers ? 4 : 8;
-  ctx->p2g_wide = !layers && 4 * tiles <= 3 * ctx->n_cu;
-  ctx->p2g_grid = std::max(128, ctx->n_cu * (layers ? 3 : ctx->p2g_wide ? 1 : tiles > 4 * ctx->n_cu ? 4 : 2));
+  ctx->p2g_grid = !layers && 4 * tiles <= 3 * ctx->n_cu
+                      ? ctx->n_cu  // by 16 waves (p2g_kernel)
+                      : std::max(128, ctx->n_cu * (layers ? 3 : tiles > 4 * ctx->n_cu ? 4 : 2));
   return MPM_OK;
 }
 
@@ -564,7 +564,14 @@ static void ensure_forces(mpm_ctx* ctx) {
   ctx->mesh.forces_valid = true;
 }
 
-static int p2g_pass(const mpm_ctx* ctx) { return ctx->p2g_wide ? P2G_WIDE_ROWS : ctx->p2g_pass; }
+// The P2G kernel of a launch shape. Rows of 8 ranks with no more workgroups than CUs leave a workgroup its CU to
+// itself, which then takes 16 waves instead of 8; the shape says so, so that a tuning names the kernel that runs.
+// With as many workgroups 16 waves are the faster at every size (P2G stage, us, 8 -> 16 waves on one workgroup per
+// CU): 8 tiles 15.9 -> 13.6, 125 17.2 -> 15.5, 392 29.2 -> 26.0, 1,728 85.8 -> 75.4, 9,632 454 -> 404.
+static int p2g_kernel(const mpm_ctx* ctx, int pass, int ranks, int blocks) {
+  return pass == P2G_ROWS && ranks == 8 && blocks <= ctx->n_cu ? P2G_WIDE_ROWS : pass;
+}
+static int p2g_pass(const mpm_ctx* ctx) { return p2g_kernel(ctx, ctx->p2g_pass, ctx->p2g_ranks, ctx->p2g_grid); }
 
 static int stage_p2g(mpm_ctx* ctx, float dt) {
   hipStream_t s = ctx->stream;
@@ -1642,11 +1649,13 @@ int mpm_autotune(mpm_ctx* ctx, float dt, int32_t reps, mpm_tuning* chosen) {
   const P2GArgs a = p2g_args(ctx, dt);
   best.p2g_ms = 1e30f;
   struct P2GCand { int pass, ranks, mult; };
-  const P2GCand cands[] = {{P2G_ROWS, 4, 2}, {P2G_ROWS, 8, 2}, {P2G_ROWS, 8, 4}, {P2G_LAYERS, 2, 6},
-                           {P2G_LAYERS, 4, 2}, {P2G_LAYERS, 4, 3}, {P2G_LAYERS, 4, 6}};
+  // rows of 8 ranks on one workgroup per CU: the 16-wave kernel (p2g_kernel)
+  const P2GCand cands[] = {{P2G_ROWS, 4, 1}, {P2G_ROWS, 4, 2}, {P2G_ROWS, 4, 4}, {P2G_ROWS, 8, 1}, {P2G_ROWS, 8, 2},
+                           {P2G_ROWS, 8, 4}, {P2G_LAYERS, 2, 2}, {P2G_LAYERS, 2, 3}, {P2G_LAYERS, 2, 6},
+                           {P2G_LAYERS, 4, 2}, {P2G_LAYERS, 4, 3}, {P2G_LAYERS, 4, 4}, {P2G_LAYERS, 4, 6}};
   for (const P2GCand& cd : cands) {
-    const int blocks = std::max(64, cd.mult * ctx->n_cu);
-    const float ms = time_launches(ctx, reps, [&] { launch_p2g(s, a, ctx->order, p2g_mode, blocks, cd.ranks, cd.pass); });
+    const int blocks = std::max(64, cd.mult * ctx->n_cu), kernel = p2g_kernel(ctx, cd.pass, cd.ranks, blocks);
+    const float ms = time_launches(ctx, reps, [&] { launch_p2g(s, a, ctx->order, p2g_mode, blocks, cd.ranks, kernel); });
     CK(hipGetLastError());
     if (ms >= 0.0f && ms < best.p2g_ms) {
       best.p2g_ms = ms;
@@ -1655,7 +1664,8 @@ int mpm_autotune(mpm_ctx* ctx, float dt, int32_t reps, mpm_tuning* chosen) {
       best.p2g_pass = cd.pass;
     }
   }
-  launch_p2g(s, a, ctx->order, p2g_mode, best.p2g_blocks, best.p2g_ranks, best.p2g_pass);
+  launch_p2g(s, a, ctx->order, p2g_mode, best.p2g_blocks, best.p2g_ranks,
+             p2g_kernel(ctx, best.p2g_pass, best.p2g_ranks, best.p2g_blocks));
   const GridArgs g = grid_args(ctx, dt);
   best.grid_ms = 1e30f;
   const int gmults[4] = {2, 4, 8, 16};
@@ -1674,7 +1684,6 @@ int mpm_autotune(mpm_ctx* ctx, float dt, int32_t reps, mpm_tuning* chosen) {
   ctx->p2g_grid = best.p2g_blocks;
   ctx->p2g_pass = best.p2g_pass;
   ctx->p2g_tuned = true;
-  ctx->p2g_wide = false;
   ctx->grid_grid = best.grid_blocks;
   drop_graphs(ctx);
   if (chosen) *chosen = best;
@@ -1710,7 +1719,6 @@ int mpm_set_tuning(mpm_ctx* ctx, const mpm_tuning* t) {
   ctx->sort_mode = t->sort_mode;
   ctx->p2g_pass = t->p2g_pass;
   ctx->p2g_tuned = true;
-  ctx->p2g_wide = false;
   drop_graphs(ctx);
   return MPM_OK;
 }

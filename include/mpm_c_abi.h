@@ -259,7 +259,8 @@ int mpm_solve(mpm_ctx* ctx, double cfl, double maxt, mpm_frame_callback cb, void
 #define MPM_P2G_LAYERS 1    /* P2G: a wave holds a whole cell layer, 4 lanes per cell */
 typedef struct mpm_tuning {
   int32_t p2g_ranks;   /* particles per cell staged per P2G chunk (the bin tile): 4 or 8 (rows), 2 or 4 (layers) */
-  int32_t p2g_blocks;  /* P2G workgroups, persistent over the active 4x4x4-cell tiles */
+  int32_t p2g_blocks;  /* P2G workgroups, persistent over the active 4x4x4-cell tiles; rows of 8 ranks run with
+                          16 waves a workgroup instead of 8 where there are no more workgroups than CUs */
   int32_t grid_blocks; /* grid-update workgroups, persistent over the active node blocks */
   float p2g_ms;        /* times of the chosen shapes measured by mpm_autotune (0 otherwise) */
   float grid_ms;
