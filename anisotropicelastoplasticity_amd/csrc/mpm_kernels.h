@@ -41,7 +41,8 @@ constexpr int PART_STRIDE = 7 * FOOT3 + 3;
 
 // The lengths of the active tile and node block lists of the last sort of state buffer b are counters
 // CNT_TILES + 2 b and CNT_BLOCKS + 2 b (the kernels get a pointer offset by 2 b).
-enum Counter : int { CNT_TILES = 0, CNT_BLOCKS = 1, CNT_CAND = 4, CNT_NUM = 5 };
+// CNT_START: the tiles of new particles (launch_count_tiles).
+enum Counter : int { CNT_TILES = 0, CNT_BLOCKS = 1, CNT_CAND = 4, CNT_START = 5, CNT_NUM = 6 };
 enum P2GMode : int { P2G_MOM_STRESS = 0, P2G_MOM = 1, P2G_FORCE = 2 };
 enum GridMode : int { GRID_FUSED = 0, GRID_NORMALIZE = 1, GRID_FORCE_UPDATE = 2 };
 
@@ -130,6 +131,7 @@ struct Clock {
   int done;          // t > maxt
   int skip;          // the rest of the replayed batch does nothing
   int executed;      // substeps completed in the current batch
+  int tiles;         // active tiles of the last substep
   long long substeps;  // substeps completed in total
 };
 
@@ -301,6 +303,9 @@ void launch_keys(hipStream_t s, const SceneTable& T, int nblocks, const float* s
                  const float* thr, uint32_t* keys, int* status);
 void launch_stress_init(hipStream_t s, const SceneTable& T, int nblocks, float* st, int64_t cap, int n,
                         unsigned long long* fallback);
+// The number of tiles that hold particles, added to *count; flag: one byte per tile, zero before and after.
+void launch_count_tiles(hipStream_t s, const SceneTable& T, int nblocks, const float* st, int64_t cap, const float* thr,
+                        uint8_t* flag, int64_t ntiles, int* count);
 // The counts of particles whose keys no G2P has counted (set by the caller, or sorted before): clears the
 // flags and counters (and, if dirty, cell_count), then counts.
 void launch_count(hipStream_t s, const SceneTable& T, const BinCounts& b, const uint32_t* keys, int n, int64_t ncells,
@@ -339,7 +344,7 @@ void launch_stress_predicted(hipStream_t s, const P2GArgs& a, int order, int nbl
 // The first Dt from the max node speed.
 void launch_clock_init(hipStream_t s, Clock* c);
 // End of a substep: the new Dt from the max node speed and the frame clamp; count it, close a completed frame, stop the batch after a frame or the run.
-void launch_clock_end(hipStream_t s, Clock* c);
+void launch_clock_end(hipStream_t s, Clock* c, const int* tiles);
 // Cloth (mesh vertices and elements among the particles of scene 0; caller ids from the DevParams).
 struct ClothArgs {
   DevParams P;

@@ -454,6 +454,29 @@ __global__ __launch_bounds__(256) void k_cell_count(SceneTable T, BinCounts b, c
   if (valid) b.rank[i] = r;
 }
 
+// The tiles that hold particles: their flags, then the number of flags, which are cleared (new particles or a new
+// grid; a substep's tiles are counted by claim_block).
+__global__ __launch_bounds__(256) void k_flag_tiles(SceneTable T, const float* __restrict__ st, int64_t cap,
+                                                    const float* __restrict__ thr, uint8_t* __restrict__ flag) {
+  const PBlock b = particle_block(T);
+  if (b.j >= b.end) return;
+  const DevParams& P = T.params[b.s];
+  const CellThr t = cell_thr(thr + T.thr_off[b.s], P.res);
+  int oob = 0, c[3];
+  (void)cell_key(P, t, st[PX * cap + b.j], st[(PX + 1) * cap + b.j], st[(PX + 2) * cap + b.j], oob, c);
+  flag[T.tile_off[b.s] + tile_of(P, c[0], c[1], c[2])] = 1;
+}
+__global__ __launch_bounds__(256) void k_sum_flags(uint8_t* __restrict__ flag, int64_t ntiles, int* __restrict__ count) {
+  int sum = 0;
+  for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < ntiles; q += (int64_t)gridDim.x * 256) {
+    sum += flag[q];
+    flag[q] = 0;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+  if (lane_id() == 0 && sum) atomicAdd(count, sum);
+}
+
 // Total of a scan block's SCAN_TILE cell counts (the blocks are independent).
 __device__ __forceinline__ void sum_block(const SortBufs& a, int b) {
   __shared__ uint32_t s_wsum[4];
@@ -1730,12 +1753,13 @@ __global__ void k_clock_init(Clock* c) {
 
 // End of a substep: the clock advances by the Dt that its G2P took; the reference closes a frame after the
 // substep that completed it (output at HybridSolver.cpp:990-1029) and leaves its loop when t > maxt (:867).
-__global__ void k_clock_end(Clock* c) {
+__global__ void k_clock_end(Clock* c, const int* tiles) {
   if (threadIdx.x != 0 || blockIdx.x != 0 || c->skip) return;
   const ClockStep s = clock_step(c, false);
   c->dt = s.dt;
   c->dt_f = (float)s.dt;
   c->vmax_bits = 0u;
+  c->tiles = *tiles;
   c->executed += 1;
   c->substeps += 1;
   if (s.frame) {
@@ -2750,6 +2774,13 @@ void launch_stress_init(hipStream_t s, const SceneTable& T, int nblocks, float* 
   if (n > 0) hipLaunchKernelGGL(k_stress_init, dim3(nblocks), dim3(256), 0, s, T, st, cap, n, fallback);
 }
 
+void launch_count_tiles(hipStream_t s, const SceneTable& T, int nblocks, const float* st, int64_t cap, const float* thr,
+                        uint8_t* flag, int64_t ntiles, int* count) {
+  if (nblocks <= 0) return;
+  hipLaunchKernelGGL(k_flag_tiles, dim3(nblocks), dim3(256), 0, s, T, st, cap, thr, flag);
+  hipLaunchKernelGGL(k_sum_flags, dim3(std::min(1024, blocks_for(ntiles, 256))), dim3(256), 0, s, flag, ntiles, count);
+}
+
 void launch_count(hipStream_t s, const SceneTable& T, const BinCounts& b, const uint32_t* keys, int n, int64_t ncells,
                   int64_t ntiles, int* counters, bool dirty) {
   const int64_t nscan = blocks_for(ncells, SCAN_TILE), work = dirty ? ncells : std::max(nscan, ntiles);
@@ -2852,7 +2883,9 @@ void launch_stress_predicted(hipStream_t s, const P2GArgs& a, int order, int nbl
 
 void launch_clock_init(hipStream_t s, Clock* c) { hipLaunchKernelGGL(k_clock_init, dim3(1), dim3(64), 0, s, c); }
 
-void launch_clock_end(hipStream_t s, Clock* c) { hipLaunchKernelGGL(k_clock_end, dim3(1), dim3(64), 0, s, c); }
+void launch_clock_end(hipStream_t s, Clock* c, const int* tiles) {
+  hipLaunchKernelGGL(k_clock_end, dim3(1), dim3(64), 0, s, c, tiles);
+}
 
 void launch_grid(hipStream_t s, const GridArgs& a, int mode, int grid) {
   if (mode == GRID_FUSED) hipLaunchKernelGGL(k_grid<GRID_FUSED>, dim3(grid), dim3(64), 0, s, a);

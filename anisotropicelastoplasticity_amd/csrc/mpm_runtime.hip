@@ -138,7 +138,13 @@ struct mpm_ctx {
   int p2g_grid = 512;
   int p2g_ranks = 8;  // P2G staging chunk
   int p2g_pass = P2G_ROWS;  // P2G schedule
-  bool p2g_tuned = false;   // set by mpm_autotune or mpm_set_tuning (else choose_p2g does)
+  bool p2g_tuned = false;   // set by mpm_autotune or mpm_set_tuning (else from the active tiles, p2g_rule)
+  // the active tiles of an earlier call's last sort on their way to the host (note_tiles, poll_tiles)
+  int* tiles_host = nullptr;  // pinned
+  hipEvent_t tiles_ev = nullptr;
+  bool tiles_pending = false;
+  int64_t tiles_steps = 0;  // substeps since the last such copy
+  std::vector<hipGraphExec_t> retired;  // graphs of a shape no longer taken that may still run
   // adaptive time step (mpm_solve): the device clock, and the pointer the kernels get (null for
   // fixed-step runs)
   Clock* clock = nullptr;
@@ -214,6 +220,19 @@ template <class T>
 static void dfree(T*& p) {
   if (p) (void)hipFree(p);
   p = nullptr;
+}
+
+static void drop_retired(mpm_ctx* ctx) {
+  for (hipGraphExec_t g : ctx->retired) (void)hipGraphExecDestroy(g);
+  ctx->retired.clear();
+}
+
+// Graphs that may still be running are kept until poll_tiles knows that they are done.
+static void retire_graphs(mpm_ctx* ctx) {
+  for (hipGraphExec_t* g : {&ctx->graph[0], &ctx->graph[1], &ctx->graph_adapt[0], &ctx->graph_adapt[1]}) {
+    if (*g) ctx->retired.push_back(*g);
+    *g = nullptr;
+  }
 }
 
 static void drop_graphs(mpm_ctx* ctx) {
@@ -521,9 +540,8 @@ static GridArgs grid_args(mpm_ctx* ctx, float dt) {
   return g;
 }
 
-// The P2G launch shape of a context that nothing has tuned, before its substeps are captured: from the active
-// tiles of the last sort. A layer's wave works through its 16 cells in lockstep and a row's 8 waves share a
-// tile, so layers pay when the tiles outnumber the CUs and are not crowded. Measured (MI355X, quadratic, P2G
+// The P2G launch shape of a context that nothing has tuned, from its active tiles. A layer's wave works through its 16
+// cells in lockstep and a row's 8 waves share a tile, so layers pay when the tiles outnumber the CUs and are not crowded. Measured (MI355X, quadratic, P2G
 // stage in us, rows of 8 ranks on 2 / 4 workgroups per CU against layers of 4 ranks on 3):
 //   particles  tiles  per tile     rows        layers
 //      64,000    216       296    19 /  19        20
@@ -538,20 +556,82 @@ static GridArgs grid_args(mpm_ctx* ctx, float dt) {
 // cells that it passes through, whatever the mean: 0.5 M sand particles on a 256 x 256-vertex cloth 89 / 89
 // against 99. Where every tile has a CU to itself, 16 waves take its rows one each instead of two: 145 tiles of 2^15
 // particles 18.1 -> 16.7 us, 8 tiles (cubic, predicted stress: both passes) 50.5 -> 44.6; but 1,073 tiles 74 -> 85.
-// The line is at three tiles to four CUs, since the particles spread after the choice: a block on 216 tiles gains at
+// The line is at three tiles to four CUs, since the particles may spread within one call: a block on 216 tiles gains at
 // first (18.1 -> 16.5) and loses once it covers more than 256.
-static int choose_p2g(mpm_ctx* ctx) {
-  if (ctx->p2g_tuned) return MPM_OK;
-  int tiles = 0;
-  CK(hipMemcpyAsync(&tiles, ctx->counters + CNT_TILES + 2 * ctx->sort_buf, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-  CK(hipStreamSynchronize(ctx->stream));
-  const bool layers = ctx->mesh.ne == 0 && tiles > ctx->n_cu && ctx->n <= 640LL * tiles;
-  ctx->p2g_pass = layers ? P2G_LAYERS : P2G_ROWS;
-  ctx->p2g_ranks = layers ? 4 : 8;
-  ctx->p2g_grid = !layers && 4 * tiles <= 3 * ctx->n_cu
-                      ? ctx->n_cu  // by 16 waves (p2g_kernel)
-                      : std::max(128, ctx->n_cu * (layers ? 3 : tiles > 4 * ctx->n_cu ? 4 : 2));
+struct P2GShape {
+  int pass, ranks, grid;
+  bool operator==(const P2GShape& o) const { return pass == o.pass && ranks == o.ranks && grid == o.grid; }
+};
+static P2GShape p2g_rule(const mpm_ctx* ctx, int64_t tiles) {
+  if (ctx->mesh.ne == 0 && tiles > ctx->n_cu && ctx->n <= 640 * tiles)
+    return {P2G_LAYERS, 4, std::max(128, 3 * ctx->n_cu)};
+  if (4 * tiles <= 3 * ctx->n_cu) return {P2G_ROWS, 8, ctx->n_cu};  // by 16 waves (p2g_kernel)
+  return {P2G_ROWS, 8, std::max(128, (tiles > 4 * ctx->n_cu ? 4 : 2) * ctx->n_cu)};
+}
+
+// When the rule is asked. New particles or a new grid: their tiles are counted while that call waits for the GPU anyhow
+// (count_tiles, take_tiles). Later, as the particles spread: a run copies the last sort's count to pinned memory behind
+// its substeps (note_tiles, once in TILE_STEPS substeps: the copy takes about as long as a small launch) and a later
+// run that finds it arrived asks again (poll_tiles); mpm_solve finds the count in the clock it reads. No run waits for
+// it. A shape is replaced, and the substeps captured anew, where the rule no longer gives it for an eighth more or fewer
+// tiles either.
+constexpr int TILE_STEPS = 64;
+
+static void set_shape(mpm_ctx* ctx, const P2GShape& c) {
+  ctx->p2g_pass = c.pass;
+  ctx->p2g_ranks = c.ranks;
+  ctx->p2g_grid = c.grid;
+}
+
+static int count_tiles(mpm_ctx* ctx, int buf) {
+  int64_t total = 0;
+  for (const SceneHost& sc : ctx->scenes) total += sc.n;
+  ctx->tiles_pending = false;  // a count of other particles
+  ctx->tiles_steps = 0;
+  *ctx->tiles_host = 0;
+  if (ctx->p2g_tuned || ctx->n <= 0 || total != ctx->n) return MPM_OK;
+  uint8_t* flag = ctx->tile_flag[1 - buf];  // no particles there: the next sort finds it cleared
+  int* count = ctx->counters + CNT_START;
+  CK(hipMemsetAsync(flag, 0, (size_t)ctx->ntiles, ctx->stream));
+  CK(hipMemsetAsync(count, 0, sizeof(int), ctx->stream));
+  launch_count_tiles(ctx->stream, ctx->T, ctx->nblocks_p, ctx->state[buf], ctx->cap, ctx->thr, flag, ctx->ntiles, count);
+  CK(hipMemcpyAsync(ctx->tiles_host, count, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   return MPM_OK;
+}
+// after the stream has been waited for
+static void take_tiles(mpm_ctx* ctx) {
+  if (!ctx->p2g_tuned && *ctx->tiles_host > 0) set_shape(ctx, p2g_rule(ctx, *ctx->tiles_host));
+}
+
+static bool renew_shape(mpm_ctx* ctx, int64_t tiles) {
+  if (ctx->p2g_tuned || tiles <= 0) return false;
+  const P2GShape now{ctx->p2g_pass, ctx->p2g_ranks, ctx->p2g_grid};
+  for (int64_t t : {tiles, tiles - tiles / 8, tiles + tiles / 8})
+    if (p2g_rule(ctx, t) == now) return false;
+  set_shape(ctx, p2g_rule(ctx, tiles));
+  return true;
+}
+
+static int note_tiles(mpm_ctx* ctx, int64_t steps) {
+  ctx->tiles_steps += steps;
+  if (ctx->p2g_tuned || ctx->tiles_pending || ctx->tiles_steps < TILE_STEPS) return MPM_OK;
+  CK(hipMemcpyAsync(ctx->tiles_host, ctx->counters + CNT_TILES + 2 * ctx->sort_buf, sizeof(int), hipMemcpyDeviceToHost,
+                    ctx->stream));
+  CK(hipEventRecord(ctx->tiles_ev, ctx->stream));
+  ctx->tiles_pending = true;
+  ctx->tiles_steps = 0;
+  return MPM_OK;
+}
+
+static void poll_tiles(mpm_ctx* ctx) {
+  if (!ctx->tiles_pending) return;
+  if (hipEventQuery(ctx->tiles_ev) != hipSuccess) {
+    (void)hipGetLastError();  // not ready is no failure
+    return;
+  }
+  ctx->tiles_pending = false;
+  drop_retired(ctx);  // they were launched before that copy
+  if (renew_shape(ctx, *ctx->tiles_host)) retire_graphs(ctx);
 }
 
 // The cloth's element forces of state[cur]: k_cloth_elements leaves them for the next substep; a new mesh's or
@@ -692,7 +772,7 @@ static int stage_g2p(mpm_ctx* ctx, float dt) {
   // cloth elements follow their vertices (positions, velocities, d1 d2) and are return-mapped
   if (ctx->mesh.ne > 0) launch_cloth_elements(ctx->stream, cloth_args(ctx, 1 - ctx->cur));
   ctx->mesh.forces_valid = ctx->mesh.ne > 0;
-  if (ctx->clk_active) launch_clock_end(ctx->stream, ctx->clk_active);
+  if (ctx->clk_active) launch_clock_end(ctx->stream, ctx->clk_active, ctx->counters + CNT_TILES + 2 * ctx->sort_buf);
   ctx->cur = 1 - ctx->cur;
   ctx->keys_valid = true;
   ctx->counted = true;
@@ -790,6 +870,14 @@ int mpm_create(mpm_ctx** out, int32_t device) {
     return MPM_ERR_HIP;
   }
   scene0(ctx);
+  e = hipHostMalloc(reinterpret_cast<void**>(&ctx->tiles_host), sizeof(int), hipHostMallocDefault);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->tiles_ev, hipEventDisableTiming);
+  if (e != hipSuccess) {
+    g_create_error = std::string("pinned count: ") + hipGetErrorString(e);
+    mpm_destroy(ctx);
+    return MPM_ERR_HIP;
+  }
+  *ctx->tiles_host = 0;
   int rc = dalloc(ctx, ctx->counters, CNT_NUM);
   if (!rc) rc = dalloc(ctx, ctx->status, 1);
   if (!rc) rc = dalloc(ctx, ctx->fallbacks, 4);
@@ -819,6 +907,9 @@ int mpm_destroy(mpm_ctx* ctx) {
   if (!ctx) return MPM_OK;
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   drop_graphs(ctx);
+  drop_retired(ctx);
+  if (ctx->tiles_ev) (void)hipEventDestroy(ctx->tiles_ev);
+  if (ctx->tiles_host) (void)hipHostFree(ctx->tiles_host);
   dfree(ctx->table_buf);
   drop_mesh(ctx);
   dfree(ctx->thr); dfree(ctx->grid); dfree(ctx->cell_start); dfree(ctx->cell_count); dfree(ctx->scan_sum); dfree(ctx->scan_flag[0]); dfree(ctx->scan_flag[1]); dfree(ctx->tile_flag[0]); dfree(ctx->tile_flag[1]);
@@ -967,6 +1058,15 @@ static int layout(mpm_ctx* ctx) {
   return rc;
 }
 
+// The tiles of the particles, if any, on a new grid.
+static int regrid_tiles(mpm_ctx* ctx) {
+  int rc = count_tiles(ctx, ctx->cur);
+  if (rc) return rc;
+  CK(hipStreamSynchronize(ctx->stream));
+  take_tiles(ctx);
+  return MPM_OK;
+}
+
 int mpm_set_grid(mpm_ctx* ctx, const double min_bound[3], const double max_bound[3], const int32_t res[3]) {
   if (!ctx || !min_bound || !max_bound || !res) return MPM_ERR_INVALID;
   if (ctx->batch) return fail(ctx, MPM_ERR_STATE, "the context holds several scenes (mpm_set_scenes)");
@@ -974,7 +1074,7 @@ int mpm_set_grid(mpm_ctx* ctx, const double min_bound[3], const double max_bound
   int rc = set_geometry(ctx, sc, min_bound, max_bound, res);
   if (!rc) rc = layout(ctx);
   if (!rc) rc = upload_table(ctx);
-  return rc;
+  return rc ? rc : regrid_tiles(ctx);
 }
 
 int mpm_set_params(mpm_ctx* ctx, const mpm_params* p) {
@@ -1014,7 +1114,7 @@ int mpm_set_scenes(mpm_ctx* ctx, int32_t nscenes, const mpm_scene_desc* descs) {
   ctx->batch = true;
   int rc = layout(ctx);
   if (!rc) rc = upload_table(ctx);
-  return rc;
+  return rc ? rc : regrid_tiles(ctx);
 }
 
 // Per-wave tables of G2P's deferred lanes (positions, masks, group sums) for the current particle
@@ -1072,7 +1172,10 @@ static int install_state(mpm_ctx* ctx, int n, const std::vector<float>& h) {
   CK(hipMemsetAsync(ctx->k2, 0, sizeof(uint32_t) * n, ctx->stream));
   launch_iota(ctx->stream, ctx->pos[0], n);
   ctx->pos_ok = true;
+  rc = count_tiles(ctx, 0);
+  if (rc) return rc;
   CK(hipStreamSynchronize(ctx->stream));
+  take_tiles(ctx);
   ctx->stress_valid = false;
   ctx->cur = 0;
   drop_keys(ctx);
@@ -1407,11 +1510,12 @@ int mpm_stage(mpm_ctx* ctx, int32_t stage, float dt) {
   if (rc) return rc;
   if (stage != ctx->next_stage) return fail(ctx, MPM_ERR_STATE, "stages must be issued in order SORT, P2G, GRID, G2P");
   CK(hipSetDevice(ctx->device));
+  if (stage == MPM_STAGE_SORT) poll_tiles(ctx);
   rc = run_stage(ctx, stage, dt);
   if (rc) return rc;
   CK(hipGetLastError());
   ctx->next_stage = (stage + 1) % MPM_NUM_STAGES;
-  return MPM_OK;
+  return stage == MPM_STAGE_G2P ? note_tiles(ctx, 1) : MPM_OK;
 }
 
 int mpm_substep(mpm_ctx* ctx, float dt) {
@@ -1419,7 +1523,9 @@ int mpm_substep(mpm_ctx* ctx, float dt) {
   if (rc) return rc;
   if (ctx->next_stage != MPM_STAGE_SORT) return fail(ctx, MPM_ERR_STATE, "a staged substep is in progress");
   CK(hipSetDevice(ctx->device));
-  return one_substep(ctx, dt);
+  poll_tiles(ctx);
+  rc = one_substep(ctx, dt);
+  return rc ? rc : note_tiles(ctx, 1);
 }
 
 int mpm_run(mpm_ctx* ctx, float dt, int32_t nsteps) {
@@ -1428,6 +1534,8 @@ int mpm_run(mpm_ctx* ctx, float dt, int32_t nsteps) {
   if (nsteps < 0) return fail(ctx, MPM_ERR_INVALID, "nsteps < 0");
   if (ctx->next_stage != MPM_STAGE_SORT) return fail(ctx, MPM_ERR_STATE, "a staged substep is in progress");
   CK(hipSetDevice(ctx->device));
+  poll_tiles(ctx);
+  const int asked = nsteps;
   if (nsteps > 0 && (!ctx->keys_valid || (!ctx->predicted && !ctx->stress_valid))) {
     rc = one_substep(ctx, dt);
     if (rc) return rc;
@@ -1441,8 +1549,6 @@ int mpm_run(mpm_ctx* ctx, float dt, int32_t nsteps) {
         (void)hipGraphExecDestroy(ctx->graph[c0]);
         ctx->graph[c0] = nullptr;
       }
-      rc = choose_p2g(ctx);
-      if (rc) return rc;
       ensure_counts(ctx);  // a captured pair starts at the scan of what the G2P before it counted
       ensure_forces(ctx);
       hipGraph_t g = nullptr;
@@ -1480,7 +1586,7 @@ int mpm_run(mpm_ctx* ctx, float dt, int32_t nsteps) {
     if (rc) return rc;
   }
   CK(hipGetLastError());
-  return MPM_OK;
+  return note_tiles(ctx, asked);
 }
 
 // ------------------------------------------------------------------ adaptive time step
@@ -1518,6 +1624,7 @@ int mpm_solve(mpm_ctx* ctx, double cfl, double maxt, mpm_frame_callback cb, void
     mpm_ctx* c;
     ~Off() { c->clk_active = nullptr; }
   } off{ctx};
+  poll_tiles(ctx);
   // first Dt from the velocities p/m of a P2G without forces
   rc = stage_sort(ctx);
   if (rc) return rc;
@@ -1537,8 +1644,6 @@ int mpm_solve(mpm_ctx* ctx, double cfl, double maxt, mpm_frame_callback cb, void
     } else {
       const int c0 = ctx->cur;
       if (!ctx->graph_adapt[c0]) {
-        rc = choose_p2g(ctx);
-        if (rc) return rc;
         ensure_counts(ctx);
         ensure_forces(ctx);
         hipGraph_t gr = nullptr;
@@ -1578,6 +1683,7 @@ int mpm_solve(mpm_ctx* ctx, double cfl, double maxt, mpm_frame_callback cb, void
       ctx->cur = (e % 2 == 0) ? c0 : 1 - c0;
       ctx->sort_buf = (e % 2 == 0) ? 1 - c0 : c0;
     }
+    if (renew_shape(ctx, h.tiles)) drop_graphs(ctx);  // the stream has been waited for
     if (!h.frame_done) dt_last = h.dt;
     const bool frame = h.frame_done != 0;
     const bool done = h.done != 0;
@@ -1864,6 +1970,7 @@ static int time_kernels(mpm_ctx* ctx, float dt, int32_t nsteps, float* total_ms,
       }
     }
   } clear{ctx};
+  poll_tiles(ctx);
   float acc[MPM_NUM_STAGES] = {0, 0, 0, 0}, g2p_main = 0.0f, sacc = 0.0f;
   CK(hipEventRecord(t0, ctx->stream));
   for (int i = 0; i < nsteps; ++i) {
@@ -1903,7 +2010,7 @@ static int time_kernels(mpm_ctx* ctx, float dt, int32_t nsteps, float* total_ms,
   (void)hipEventDestroy(t0);
   (void)hipEventDestroy(t1);
   CK(hipGetLastError());
-  return MPM_OK;
+  return note_tiles(ctx, nsteps);
 }
 
 int mpm_time_kernels(mpm_ctx* ctx, float dt, int32_t nsteps, float* total_ms, float* stage_ms, float* kernel_ms) {

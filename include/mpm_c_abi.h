@@ -240,7 +240,9 @@ int mpm_estimate_volumes(mpm_ctx* ctx);
 
 /* One explicit substep with fixed dt (HybridSolver.cpp:873-987). */
 int mpm_substep(mpm_ctx* ctx, float dt);
-/* nsteps substeps with fixed dt, replayed from one captured HIP graph. */
+/* nsteps substeps with fixed dt, replayed from one captured HIP graph. The call enqueues its work and does not wait for
+ * the GPU. A context that nothing has tuned takes its P2G shape from the occupied tiles: of new particles (or a new
+ * grid) at once, and again as they spread, at a later call once the count of an earlier one has arrived. */
 int mpm_run(mpm_ctx* ctx, float dt, int32_t nsteps);
 /* Called by mpm_solve on the calling thread after the substep that completes frame `frame`
  * (0-based) at simulated time t; the particle state may be read from inside the callback. */
