@@ -552,6 +552,10 @@ static GridArgs grid_args(mpm_ctx* ctx, float dt) {
 //   1,560,896  2,227       701   105 / 108       101
 //   1,560,896  1,579       989   118 / 114       139
 //   4,194,304  9,537       440   357 / 333       271
+// The lines: layers up to 768 particles per tile (0.96 of the rows' time at 770, 1.04 at 779, above). Where the tiles
+// exceed two per CU, rows need another round (576 tiles of 64 / 216 / 512 particles: layers 0.90 / 0.96 / 0.94 of the
+// rows' time); up to there every row tile has a workgroup, and layers pay from about 320 per tile (294 and 512 tiles of
+// 118-125 particles 1.02, 216: 1.03, 329-343: 0.97-1.00, 512: 0.98).
 // Cubic splines and predicted stress lie alike (681,472 particles, cubic: 77 / 80 against 60). A mesh crowds the
 // cells that it passes through, whatever the mean: 0.5 M sand particles on a 256 x 256-vertex cloth 89 / 89
 // against 99. Where every tile has a CU to itself, 16 waves take its rows one each instead of two: 145 tiles of 2^15
@@ -563,7 +567,7 @@ struct P2GShape {
   bool operator==(const P2GShape& o) const { return pass == o.pass && ranks == o.ranks && grid == o.grid; }
 };
 static P2GShape p2g_rule(const mpm_ctx* ctx, int64_t tiles) {
-  if (ctx->mesh.ne == 0 && tiles > ctx->n_cu && ctx->n <= 640 * tiles)
+  if (ctx->mesh.ne == 0 && tiles > ctx->n_cu && ctx->n <= 768 * tiles && (tiles > 2 * ctx->n_cu || ctx->n >= 320 * tiles))
     return {P2G_LAYERS, 4, std::max(128, 3 * ctx->n_cu)};
   if (4 * tiles <= 3 * ctx->n_cu) return {P2G_ROWS, 8, ctx->n_cu};  // by 16 waves (p2g_kernel)
   return {P2G_ROWS, 8, std::max(128, (tiles > 4 * ctx->n_cu ? 4 : 2) * ctx->n_cu)};
@@ -575,7 +579,7 @@ static P2GShape p2g_rule(const mpm_ctx* ctx, int64_t tiles) {
 // run that finds it arrived asks again (poll_tiles); mpm_solve finds the count in the clock it reads. No run waits for
 // it. A shape is replaced, and the substeps captured anew, where the rule no longer gives it for an eighth more or fewer
 // tiles either.
-constexpr int TILE_STEPS = 64;
+constexpr int TILE_STEPS = 32;
 
 static void set_shape(mpm_ctx* ctx, const P2GShape& c) {
   ctx->p2g_pass = c.pass;
