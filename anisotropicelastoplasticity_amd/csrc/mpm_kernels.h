@@ -42,7 +42,7 @@ constexpr int PART_STRIDE = 7 * FOOT3 + 3;
 // The lengths of the active tile and node block lists of the last sort of state buffer b are counters
 // CNT_TILES + 2 b and CNT_BLOCKS + 2 b (the kernels get a pointer offset by 2 b).
 // CNT_START: the tiles of new particles (launch_count_tiles).
-enum Counter : int { CNT_TILES = 0, CNT_BLOCKS = 1, CNT_CAND = 4, CNT_START = 5, CNT_NUM = 6 };
+enum Counter : int { CNT_TILES = 0, CNT_BLOCKS = 1, CNT_CAND = 4, CNT_START = 5, CNT_APEX = 6, CNT_NUM = 7 };
 enum P2GMode : int { P2G_MOM_STRESS = 0, P2G_MOM = 1, P2G_FORCE = 2 };
 enum GridMode : int { GRID_FUSED = 0, GRID_NORMALIZE = 1, GRID_FORCE_UPDATE = 2 };
 
@@ -257,6 +257,9 @@ struct ApexArgs {
   const int* wave_pos;    // ... and the sorted position of its lane 0
   int nwaves;
   int gw;                 // waves per group (set by the launcher)
+  const int* list;        // or the deferred particles' sorted positions (else null),
+  const int* idx;         // their record indices in apex_usv
+  const int* count;       // and their number
   const float* apex_usv;  // the deferred particles' trial SVDs
   int write_stress;
   int log_pairs;
@@ -273,7 +276,7 @@ void launch_apex_finish(hipStream_t s, ApexArgs a, int n_cu);
 // Planes of a deferred particle's trial SVD (surrogate candidates and FP64 apex projections). k_g2p
 // writes the records of a wave's deferred lanes next to each other: the record index of lane L is
 // the sorted position of the wave's lane 0 plus the number of deferred lanes below L (so it is at
-// most L's own position, below n), and the position list carries it with every entry.
+// most L's own position, below n), and the position lists carry it with every entry.
 constexpr int CAND_SIGMA = 0, CAND_U = 3, CAND_V = 12, CAND_SVD_PLANES = 21;
 
 struct SurrogateArgs {
@@ -377,18 +380,18 @@ void launch_cloth_vertex_forces(hipStream_t s, const ClothArgs& a);  // the per-
 void launch_cloth_fixed(hipStream_t s, const ClothArgs& a);    // after the grid update
 void launch_cloth_elements(hipStream_t s, const ClothArgs& a); // after G2P: positions, velocities, D, return map, forces
 void surrogate_set_smem_limit();
-// List of the sorted positions that G2P flagged (mask[w] of wave w, whose lane 0 sits at wpos[w]), in
-// ascending order and built without atomics; its length goes to *count.
+// Up to two lists of the sorted positions that G2P flagged (mask[l][w] of wave w, whose lane 0 sits at wpos[w]), in
+// ascending order and built without atomics; list l's length goes to *count[l].
 struct ListArgs {
-  const uint64_t* mask;
-  int* list;
-  int* idx;  // each entry's record index (see CAND_SIGMA)
-  int* count;
-  int* gsum;  // [(nwaves + 63) / 64]
+  const uint64_t* mask[2];
+  int* list[2];
+  int* idx[2];  // each entry's record index (see CAND_SIGMA)
+  int* count[2];
+  int* gsum;  // [2][(nwaves + 63) / 64]
   const int* wpos;
-  int nwaves;
+  int nwaves, nlists;
 };
-void launch_position_list(hipStream_t s, const ListArgs& a);
+void launch_position_lists(hipStream_t s, const ListArgs& a);
 // k_surrogate: MFMA network, gate and state update of the listed candidates (ev: optional start
 // and stop events of the dispatch)
 void launch_surrogate(hipStream_t s, const SurrogateArgs& a, int n_cu, hipEvent_t* ev);

@@ -2185,13 +2185,58 @@ __global__ __launch_bounds__(256) void k_g2p(G2PArgs a) {
 // The FP64 apex projections deferred by k_g2p, gathered into full waves: from the trial SVD that
 // k_g2p stored and the particle's q, phi and V, the FP64 projection and F_E and V tau (the same
 // function return_map calls, on the same operands), stored over the trial F^ left in the output
-// buffer. The result equals computing it inside k_g2p.
-//
-// A workgroup takes the masks of `gw` G2P waves at a time (4, a G2P workgroup's, where that gives few groups;
-// else 32, which gathers fuller waves), lists their flagged positions in LDS and works the list off. Bound by
-// the launch and one round trip of the masks where few particles are flagged, and by scattered writes where many
-// are (410k of 2^22: 63 us; in groups of 16 and 64 waves 65-68 and 72, with two list launches before it and waves
-// filled over the whole state 53 + 11). With few flagged, G2P and what follows it took 95 us with the list launches
+// buffer. The result equals computing it inside k_g2p. j: the particle's sorted position, r: its record.
+__device__ __forceinline__ void apex_particle(const ApexArgs& a, int j, int r, int& fb_apex) {
+  const int sc = scene_of(a.T.part_off, a.T.nscenes, j);
+  const DevParams& P = a.T.params[sc];
+  float* st = a.st;
+  const int64_t cap = a.cap, n = a.n;
+  float S[3], U[9], V[9];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) S[k] = a.apex_usv[(CAND_SIGMA + k) * n + r];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) {
+    U[k] = a.apex_usv[(CAND_U + k) * n + r];
+    V[k] = a.apex_usv[(CAND_V + k) * n + r];
+  }
+  float plastic = st[PPL * cap + j];
+  const float phi_p = st[PPHI * cap + j];
+  const float vol = st[PVOL * cap + j];
+  SurrogateIO io;
+  io.mode = a.log_pairs ? 1 : 0;
+  io.pair_log = a.pair_log;
+  io.pair_cap = a.pair_cap;
+  io.pair_count = a.pair_count;
+  // the FP32 trial strains, as the return map computed them (used by the pair log only)
+  float l[3] = {0.0f, 0.0f, 0.0f};
+  if (io.mode == 1) {
+    l[0] = logf(S[0]);
+    l[1] = logf(S[1]);
+    l[2] = logf(S[2]);
+  }
+  float Fe[9], K[6];
+  sand_apex_finish(P, U, S, V, l, P.per_particle_phi ? phi_p : P.h0, phi_p, plastic, vol, Fe, K, fb_apex, io);
+#pragma unroll
+  for (int i = 0; i < 9; ++i) st[(PF + i) * cap + j] = Fe[i];
+  st[PPL * cap + j] = plastic;
+  if (a.write_stress) {
+#pragma unroll
+    for (int e = 0; e < 6; ++e) st[(PK + e) * cap + j] = K[e];
+  }
+}
+// One atomic per wave.
+__device__ __forceinline__ void apex_fallbacks(const ApexArgs& a, int fb_apex) {
+  unsigned long long c = (unsigned long long)fb_apex;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off);
+  if ((threadIdx.x & 63) == 0 && c) atomicAdd(a.fallback_apex, c);
+}
+
+// Without the surrogate, from G2P's masks: a workgroup takes those of `gw` G2P waves at a time (4, a G2P workgroup's,
+// where that gives few groups; else 32, which gathers fuller waves), lists their flagged positions in LDS and works the
+// list off. Bound by the launch and one round trip of the masks where few particles are flagged, and by scattered writes
+// where many are (410k of 2^22: 63 us; in groups of 16 and 64 waves 65-68 and 72, with two list launches before it and
+// waves filled over the whole state 53 + 11). With few flagged, G2P and what follows it took 95 us with the list launches
 // and 92 without at 2^20 particles, 177 and 171 for 16 scenes.
 __global__ __launch_bounds__(256) void k_apex_finish(ApexArgs a) {
   if (clock_skip(a.clk)) return;
@@ -2223,90 +2268,64 @@ __global__ __launch_bounds__(256) void k_apex_finish(ApexArgs a) {
       }
     }
     __syncthreads();
-    for (int c = (int)threadIdx.x; c < count; c += 256) {
-      const int j = clamp_index(s_slot[c], a.n);
-      const int r = clamp_index(s_idx[c], a.n);
-      const int sc = scene_of(a.T.part_off, a.T.nscenes, j);
-      const DevParams& P = a.T.params[sc];
-      float* st = a.st;
-      const int64_t cap = a.cap, n = a.n;
-      float S[3], U[9], V[9];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) S[k] = a.apex_usv[(CAND_SIGMA + k) * n + r];
-#pragma unroll
-      for (int k = 0; k < 9; ++k) {
-        U[k] = a.apex_usv[(CAND_U + k) * n + r];
-        V[k] = a.apex_usv[(CAND_V + k) * n + r];
-      }
-      float plastic = st[PPL * cap + j];
-      const float phi_p = st[PPHI * cap + j];
-      const float vol = st[PVOL * cap + j];
-      SurrogateIO io;
-      io.mode = a.log_pairs ? 1 : 0;
-      io.pair_log = a.pair_log;
-      io.pair_cap = a.pair_cap;
-      io.pair_count = a.pair_count;
-      // the FP32 trial strains, as the return map computed them (used by the pair log only)
-      float l[3] = {0.0f, 0.0f, 0.0f};
-      if (io.mode == 1) {
-        l[0] = logf(S[0]);
-        l[1] = logf(S[1]);
-        l[2] = logf(S[2]);
-      }
-      float Fe[9], K[6];
-      sand_apex_finish(P, U, S, V, l, P.per_particle_phi ? phi_p : P.h0, phi_p, plastic, vol, Fe, K, fb_apex, io);
-#pragma unroll
-      for (int i = 0; i < 9; ++i) st[(PF + i) * cap + j] = Fe[i];
-      st[PPL * cap + j] = plastic;
-      if (a.write_stress) {
-#pragma unroll
-        for (int e = 0; e < 6; ++e) st[(PK + e) * cap + j] = K[e];
-      }
-    }
+    for (int c = (int)threadIdx.x; c < count; c += 256)
+      apex_particle(a, clamp_index(s_slot[c], a.n), clamp_index(s_idx[c], a.n), fb_apex);
     __syncthreads();
   }
-  // one atomic per wave
-  unsigned long long c = (unsigned long long)fb_apex;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off);
-  if ((threadIdx.x & 63) == 0 && c) atomicAdd(a.fallback_apex, c);
+  apex_fallbacks(a, fb_apex);
 }
 
-// ================================================================== position list
-// List of the sorted positions that G2P flagged as the surrogate's candidates, in ascending order and without
-// atomics. Every G2P wave w stores the ballot of its flagged lanes (mask[w]) and the position of its
+// Beside the surrogate, whose candidates are listed by launches of their own, from the list that these make as well:
+// waves full over the whole state. Both with the lists, 2^22 particles: 75.3 us from the masks, 71.6 so (MI355X).
+__global__ __launch_bounds__(256) void k_apex_list(ApexArgs a) {
+  if (clock_skip(a.clk)) return;
+  const int count = min(*a.count, a.n);
+  int fb_apex = 0;
+  for (int c = (int)blockIdx.x * 256 + (int)threadIdx.x; c < count; c += (int)gridDim.x * 256)
+    apex_particle(a, clamp_index(a.list[c], a.n), clamp_index(a.idx[c], a.n), fb_apex);
+  apex_fallbacks(a, fb_apex);
+}
+
+// ================================================================== position lists
+// Lists of the sorted positions that G2P flagged, in ascending order and without atomics: the surrogate's candidates
+// and, beside them, the deferred FP64 apex projections (two lists, one set of launches).
+// Every G2P wave w stores the ballots of its flagged lanes (mask[l][w]) and the position of its
 // lane 0 (wpos[w]). Waves form groups of 64: k_list_sums totals each group; k_list_write (one
 // workgroup per group) adds up the totals of the groups before its own, places each wave's
 // positions after that offset and the waves before it in the group, and the last group's
-// workgroup writes the list's length.
+// workgroup writes the list lengths.
 __global__ __launch_bounds__(256) void k_list_sums(ListArgs a) {
   const int ng = (a.nwaves + 63) / 64;
   const int g = blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (g >= ng) return;
   const int w = g * 64 + lane;
-  int c = w < a.nwaves ? __popcll(a.mask[w]) : 0;
+  for (int l = 0; l < a.nlists; ++l) {
+    int c = w < a.nwaves ? __popcll(a.mask[l][w]) : 0;
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off);
-  if (lane == 0) a.gsum[g] = c;
+    for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off);
+    if (lane == 0) a.gsum[l * ng + g] = c;
+  }
 }
 
 __global__ __launch_bounds__(256) void k_list_write(ListArgs a) {
-  __shared__ uint64_t s_m[64];
-  __shared__ int s_off[64], s_p[64], s_red[4];
+  __shared__ uint64_t s_m[2][64];
+  __shared__ int s_off[2][64], s_p[64], s_red[2][4];
   const int ng = (a.nwaves + 63) / 64;
   const int g = blockIdx.x, t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int w = g * 64 + lane;
-  // the offset of this group: the totals of the groups before it, summed by the workgroup
+  // each list's offset of this group: the totals of the groups before it, summed by the workgroup
   // itself (integer sums, so the order does not matter)
-  int sum = 0;
-  for (int i = t; i < g; i += 256) sum += a.gsum[i];
+  for (int l = 0; l < a.nlists; ++l) {
+    int sum = 0;
+    for (int i = t; i < g; i += 256) sum += a.gsum[l * ng + i];
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-  if (lane == 0) s_red[wv] = sum;
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+    if (lane == 0) s_red[l][wv] = sum;
+  }
   __syncthreads();
-  if (wv == 0) {  // the offsets of the group's 64 masks
-    const int pre = s_red[0] + s_red[1] + s_red[2] + s_red[3];
-    const uint64_t m = w < a.nwaves ? a.mask[w] : 0ull;
+  if (wv < a.nlists) {  // wave l: the offsets of list l's 64 masks of the group
+    const int pre = s_red[wv][0] + s_red[wv][1] + s_red[wv][2] + s_red[wv][3];
+    const uint64_t m = w < a.nwaves ? a.mask[wv][w] : 0ull;
     const int c = __popcll(m);
     int x = c;
 #pragma unroll
@@ -2314,23 +2333,24 @@ __global__ __launch_bounds__(256) void k_list_write(ListArgs a) {
       const int y = __shfl_up(x, off);
       if (lane >= off) x += y;
     }
-    s_m[lane] = m;
-    s_off[lane] = pre + x - c;
+    s_m[wv][lane] = m;
+    s_off[wv][lane] = pre + x - c;
     // the last group's workgroup writes the list's length
-    if (g == ng - 1 && lane == 63) *a.count = pre + x;
+    if (g == ng - 1 && lane == 63) *a.count[wv] = pre + x;
   } else if (wv == 3) {
     s_p[lane] = w < a.nwaves ? a.wpos[w] : 0;
   }
   __syncthreads();
-  // wave wv writes the positions of masks 16 wv .. 16 wv + 15, one mask at a time
-  for (int i = 16 * wv; i < 16 * wv + 16; ++i) {
-    const uint64_t mi = s_m[i];
-    if ((mi >> lane) & 1ull) {
-      const int rank = __popcll(mi & ((1ull << lane) - 1ull));
-      a.list[s_off[i] + rank] = s_p[i] + lane;
-      a.idx[s_off[i] + rank] = s_p[i] + rank;
+  // wave wv writes the positions of masks 16 wv .. 16 wv + 15 of each list, one mask at a time
+  for (int l = 0; l < a.nlists; ++l)
+    for (int i = 16 * wv; i < 16 * wv + 16; ++i) {
+      const uint64_t mi = s_m[l][i];
+      if ((mi >> lane) & 1ull) {
+        const int rank = __popcll(mi & ((1ull << lane) - 1ull));
+        a.list[l][s_off[l][i] + rank] = s_p[i] + lane;
+        a.idx[l][s_off[l][i] + rank] = s_p[i] + rank;
+      }
     }
-  }
 }
 
 // ================================================================== surrogate return map
@@ -2946,8 +2966,8 @@ void surrogate_set_smem_limit() {
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)surrogate_smem());
 }
 
-void launch_position_list(hipStream_t s, const ListArgs& a) {
-  if (a.nwaves <= 0) return;
+void launch_position_lists(hipStream_t s, const ListArgs& a) {
+  if (a.nwaves <= 0 || a.nlists <= 0) return;
   const int ng = (a.nwaves + 63) / 64;
   hipLaunchKernelGGL(k_list_sums, dim3((ng + 3) / 4), dim3(256), 0, s, a);
   hipLaunchKernelGGL(k_list_write, dim3(ng), dim3(256), 0, s, a);
@@ -2962,6 +2982,10 @@ void launch_surrogate(hipStream_t s, const SurrogateArgs& a, int n_cu, hipEvent_
 }
 
 void launch_apex_finish(hipStream_t s, ApexArgs a, int n_cu) {
+  if (a.list) {
+    hipLaunchKernelGGL(k_apex_list, dim3(2 * n_cu), dim3(256), 0, s, a);
+    return;
+  }
   const int small = blocks_for(a.nwaves, 4);
   a.gw = small <= 8 * n_cu ? 4 : APEX_GROUP;
   hipLaunchKernelGGL(k_apex_finish, dim3(a.gw == 4 ? small : std::min(4 * n_cu, blocks_for(a.nwaves, APEX_GROUP))),

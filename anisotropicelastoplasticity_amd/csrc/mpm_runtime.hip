@@ -170,7 +170,7 @@ struct mpm_ctx {
   int* wave_pos = nullptr;
   uint64_t* cand_mask = nullptr;
   uint64_t* apex_mask = nullptr;
-  int* list_gsum = nullptr;  // candidates per group of 64 waves
+  int* list_gsum = nullptr;  // per list and group of 64 waves: listed particles
   int64_t wave_cap = 0;
   float* dec_log = nullptr;  // per-candidate gate records of the last surrogate substep
   int64_t dec_cap = 0;
@@ -723,8 +723,36 @@ static int stage_g2p(mpm_ctx* ctx, float dt) {
   a.apex_usv = ctx->apex_usv;
   a.clk = ctx->clk_active;
   launch_g2p(ctx->stream, a, ctx->order, ctx->nblocks_p, ctx->ev_main[0], ctx->ev_main[1]);
+  // the surrogate's candidates are listed, and then the apex particles with them, into scratch of the sort, which is
+  // done with it
+  int* const apex_list = ctx->tslot;
+  int* const apex_idx = (ctx->sort_passes & 1) ? ctx->v2 : ctx->v1;
+  if (surrogate) {
+    ListArgs la{};
+    la.wpos = ctx->wave_pos;
+    la.gsum = ctx->list_gsum;
+    la.nwaves = 4 * ctx->nblocks_p;
+    la.mask[0] = ctx->cand_mask;
+    la.list[0] = ctx->cand_slot;
+    la.idx[0] = ctx->cand_idx;
+    la.count[0] = ctx->counters + CNT_CAND;
+    la.nlists = 1;
+    if (a.apex_mask) {
+      la.mask[1] = ctx->apex_mask;
+      la.list[1] = apex_list;
+      la.idx[1] = apex_idx;
+      la.count[1] = ctx->counters + CNT_APEX;
+      la.nlists = 2;
+    }
+    launch_position_lists(ctx->stream, la);
+  }
   if (a.apex_mask) {
-    ApexArgs x;
+    ApexArgs x{};
+    if (surrogate) {
+      x.list = apex_list;
+      x.idx = apex_idx;
+      x.count = ctx->counters + CNT_APEX;
+    }
     x.T = ctx->T;
     x.st = ctx->state[1 - ctx->cur];
     x.cap = ctx->cap;
@@ -744,15 +772,6 @@ static int stage_g2p(mpm_ctx* ctx, float dt) {
     launch_apex_finish(ctx->stream, x, ctx->n_cu);
   }
   if (surrogate) {
-    ListArgs la;
-    la.mask = ctx->cand_mask;
-    la.list = ctx->cand_slot;
-    la.idx = ctx->cand_idx;
-    la.count = ctx->counters + CNT_CAND;
-    la.gsum = ctx->list_gsum;
-    la.wpos = ctx->wave_pos;
-    la.nwaves = 4 * ctx->nblocks_p;
-    launch_position_list(ctx->stream, la);
     SurrogateArgs sa;
     sa.T = ctx->T;
     sa.wbf = ctx->mlp_wbf;
@@ -1128,7 +1147,7 @@ static int alloc_wave_tables(mpm_ctx* ctx) {
   int rc = dalloc(ctx, ctx->wave_pos, (size_t)nw);
   if (!rc) rc = dalloc(ctx, ctx->cand_mask, (size_t)nw);
   if (!rc) rc = dalloc(ctx, ctx->apex_mask, (size_t)nw);
-  if (!rc) rc = dalloc(ctx, ctx->list_gsum, (size_t)((nw + 63) / 64));
+  if (!rc) rc = dalloc(ctx, ctx->list_gsum, (size_t)(2 * ((nw + 63) / 64)));
   ctx->wave_cap = rc ? 0 : nw;
   return rc;
 }
