@@ -1441,7 +1441,9 @@ __device__ __forceinline__ TileCell tile_cell(const P2GArgs& a, const TileScene&
 // before this tile's chunks, its first slots after them, and its first particles before the slab sums are
 // stored; and a wave's slabs take the place of its payloads, which are done with by then: 52 KB a workgroup
 // instead of 71, three on a CU instead of two. P2G at 2^22 particles (7.5 per cell) 302 -> 272 us; 16 scenes
-// of 1.8 M in all 157 -> 148 us.
+// of 1.8 M in all 157 -> 148 us. Three on a CU leave a wave 168 registers; with momentum and stress in one pass that is
+// two too few, and the compiler stores one pair before the loop over the tiles and loads it once per tile (12 bytes of
+// scratch a lane, nothing in the particle loops).
 template <int ORDER, int MODE, int RANKS>
 __global__ __launch_bounds__(256, 3) void k_p2g_layer(P2GArgs a) {
   if (clock_skip(a.clk)) return;

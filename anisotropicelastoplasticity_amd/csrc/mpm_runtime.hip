@@ -140,8 +140,7 @@ struct mpm_ctx {
   int p2g_pass = P2G_ROWS;  // P2G schedule
   bool p2g_tuned = false;   // set by mpm_autotune or mpm_set_tuning (else from the active tiles, p2g_rule)
   // the active tiles of an earlier call's last sort on their way to the host (note_tiles, poll_tiles)
-  int* tiles_host = nullptr;  // pinned
-  hipEvent_t tiles_ev = nullptr;
+  int* tiles_host = nullptr;  // pinned; negative until the copy arrives
   bool tiles_pending = false;
   int64_t tiles_steps = 0;  // substeps since the last such copy
   std::vector<hipGraphExec_t> retired;  // graphs of a shape no longer taken that may still run
@@ -575,11 +574,12 @@ static P2GShape p2g_rule(const mpm_ctx* ctx, int64_t tiles) {
 
 // When the rule is asked. New particles or a new grid: their tiles are counted while that call waits for the GPU anyhow
 // (count_tiles, take_tiles). Later, as the particles spread: a run copies the last sort's count to pinned memory behind
-// its substeps (note_tiles, once in TILE_STEPS substeps: the copy takes about as long as a small launch) and a later
-// run that finds it arrived asks again (poll_tiles); mpm_solve finds the count in the clock it reads. No run waits for
-// it. A shape is replaced, and the substeps captured anew, where the rule no longer gives it for an eighth more or fewer
+// its substeps (note_tiles) and a later run that finds it arrived asks again (poll_tiles); mpm_solve finds the count in
+// the clock it reads. No run waits for it. The copy holds up the substeps behind it by some 30 us, so it is made once in
+// TILE_STEPS substeps: every 32, a tiny scene took 1,519 us instead of 1,501 for 20. (Left in pinned memory by each G2P,
+// it cost 1,540: the kernel waits for the bus.) A shape is replaced, and the substeps captured anew, where the rule no longer gives it for an eighth more or fewer
 // tiles either.
-constexpr int TILE_STEPS = 32;
+constexpr int TILE_STEPS = 256;
 
 static void set_shape(mpm_ctx* ctx, const P2GShape& c) {
   ctx->p2g_pass = c.pass;
@@ -619,9 +619,9 @@ static bool renew_shape(mpm_ctx* ctx, int64_t tiles) {
 static int note_tiles(mpm_ctx* ctx, int64_t steps) {
   ctx->tiles_steps += steps;
   if (ctx->p2g_tuned || ctx->tiles_pending || ctx->tiles_steps < TILE_STEPS) return MPM_OK;
+  *ctx->tiles_host = -1;
   CK(hipMemcpyAsync(ctx->tiles_host, ctx->counters + CNT_TILES + 2 * ctx->sort_buf, sizeof(int), hipMemcpyDeviceToHost,
                     ctx->stream));
-  CK(hipEventRecord(ctx->tiles_ev, ctx->stream));
   ctx->tiles_pending = true;
   ctx->tiles_steps = 0;
   return MPM_OK;
@@ -629,13 +629,12 @@ static int note_tiles(mpm_ctx* ctx, int64_t steps) {
 
 static void poll_tiles(mpm_ctx* ctx) {
   if (!ctx->tiles_pending) return;
-  if (hipEventQuery(ctx->tiles_ev) != hipSuccess) {
-    (void)hipGetLastError();  // not ready is no failure
-    return;
-  }
+  // read as the copy leaves it: an event query would be refused while another thread captures a graph
+  const int tiles = __atomic_load_n(ctx->tiles_host, __ATOMIC_ACQUIRE);
+  if (tiles < 0) return;
   ctx->tiles_pending = false;
   drop_retired(ctx);  // they were launched before that copy
-  if (renew_shape(ctx, *ctx->tiles_host)) retire_graphs(ctx);
+  if (renew_shape(ctx, tiles)) retire_graphs(ctx);
 }
 
 // The cloth's element forces of state[cur]: k_cloth_elements leaves them for the next substep; a new mesh's or
@@ -894,7 +893,6 @@ int mpm_create(mpm_ctx** out, int32_t device) {
   }
   scene0(ctx);
   e = hipHostMalloc(reinterpret_cast<void**>(&ctx->tiles_host), sizeof(int), hipHostMallocDefault);
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->tiles_ev, hipEventDisableTiming);
   if (e != hipSuccess) {
     g_create_error = std::string("pinned count: ") + hipGetErrorString(e);
     mpm_destroy(ctx);
@@ -931,7 +929,6 @@ int mpm_destroy(mpm_ctx* ctx) {
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   drop_graphs(ctx);
   drop_retired(ctx);
-  if (ctx->tiles_ev) (void)hipEventDestroy(ctx->tiles_ev);
   if (ctx->tiles_host) (void)hipHostFree(ctx->tiles_host);
   dfree(ctx->table_buf);
   drop_mesh(ctx);

@@ -57,8 +57,9 @@ def test_shape_follows_runs(how):
             if fixed:
                 s.set_tuning(*FIXED)
             first = s.tuning()
-            for n in (80, 80, 8):
-                _advance(s, sc.dt, how, n)
+            # the count that a call finds is that of an earlier one, up to some hundred substeps old
+            for n in (200, 200, 200, 1):
+                _advance(s, 0.4 * sc.dt, how, n)
                 s.synchronize()
             print(how, fixed, first, s.tuning(), s.stats()["n_active_tiles"], flush=True)
             if not fixed:
