@@ -6,20 +6,21 @@
 //               the planes are kept physically sorted by cell key, so every particle pass streams
 //               them. A cloth's vertices and elements are particles of the same buffers.
 //   keys        uint32 cell key per particle in the current physical order (written by G2P).
-//   sort        counting sort: per-cell counts (zero between substeps), cell_start over all cells
-//               plus one, scan status words and tickets; LSD radix: K1/K2 keys and V1/V2 index
-//               ping-pong buffers and per-pass look-back status words.
+//   sort        per-cell counts of the next sort (made by G2P, zero from a sort to the next G2P), by state
+//               buffer a flag per tile and per scan block of cells, cell_start over all cells plus one, scan
+//               block totals; LSD radix besides: K1/K2 keys and V1/V2 index ping-pong buffers, tickets and
+//               per-pass look-back status words.
 //   grid        dense planes m, mom(3) and interleaved float4 pairs (v, v_BF) over the nodes; only
 //               the 4x4x4 node blocks around active tiles are written each substep.
 //   tiles       4x4x4-cell tiles: slot per tile (-1 = inactive), active list, per-slot P2G partials
 //               over the tile's 7x7x7 node footprint.
 //
-// Substep (stress at F^n): reset -> cell count -> cell scan -> cell scatter -> cell rank (bins,
-// tile flags) -> claim tiles -> claim node blocks -> p2g -> grid -> g2p -> apex finish.
-// Reference-compatible substep (stress at predicted F^): p2g(momentum) -> grid(normalise) ->
-// p2g(force, gathers grad v) -> grid(force update) replace the p2g -> grid pair. A cloth adds its
-// element and vertex forces before P2G, the fixed-vertex node stops after the grid update, and the
-// element update (directions, QR return map) after G2P.
+// Substep (stress at F^n): scan block totals and tile lists -> cell scan (small grids: in the first launch) ->
+// cell scatter -> cell rank (bins) -> p2g -> grid -> g2p (counts the next sort's cells) -> apex finish.
+// Reference-compatible substep (stress at predicted F^): p2g(momentum) -> grid(normalise) -> stress at F^ ->
+// p2g(force) -> grid(force update) replace the p2g -> grid pair. A cloth adds its vertex forces before P2G, the
+// fixed-vertex node stops after the grid update, and the element update (directions, QR return map, the next
+// substep's element forces) after G2P. The surrogate adds the position lists and its kernel after G2P.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 

@@ -170,7 +170,8 @@ __global__ __launch_bounds__(SMALL_THREADS) void k_mlp_forward_small(const uint1
 // tile w: it reads its column tile of Z_{L-1} once (the next layer's while this one is computed) for
 // both SiLU (the operand A_{L-1}^T) and SiLU', and its 16 rows of W_L^T straight into registers. The
 // kernel is bound by the chain of layers (few workgroups: 64 for a 4096-row batch), so its steps hold
-// no global read-modify-write and no strided gather.
+// no strided gather and, for a workgroup's first group, no global read-modify-write (later groups, in batches of
+// more than 1024 x 64 rows, add to its gradients in memory).
 // Measured on MI355X at 4096 rows: 30 us; with 4 waves, gradients accumulated in global memory and each
 // Z element gathered by row (64 cache lines per load) it took 152 us.
 constexpr int BWD_THREADS = 512;

@@ -389,8 +389,7 @@ static float threshold(double gmin, double h, int c) {
   return f;
 }
 
-// Sort workspace words: 4 x 256 digit histograms, 4 digit-pass tickets and 4 cell-scan tickets, the
-// cell-scan look-back words (64-bit, one per scan block), then the digit passes' look-back words.
+// Workspace words of the digit passes: 4 x 256 histograms, 4 tickets (and 4 spare words), look-back words.
 static constexpr int64_t SORTWS_TICKETS = 1024, SORTWS_STATUS = 1032;
 
 // ------------------------------------------------------------------ substep stages

@@ -47,15 +47,15 @@ COMPARE_SUBSTEPS = 1020
 #   GRID reads m, momentum (16 B), writes v and v_BF (24 B) per active node
 #   G2P  reads x, F, plastic (13 floats), writes x, v, B, F, plastic (25 floats) per particle,
 #        reads v and v_BF (24 B) per active node; a per-particle friction angle adds 4 B per particle
-#   SORT (counting sort) reads the key twice and the rank once, writes rank, scattered id, sorted key,
-#        id and slot index: 36 B per particle, plus the cell counts scanned into the bins
+#   SORT (counting sort) reads key, rank and id and writes id, slot and key into the cells, then reads those
+#        and writes the ordered id and the slot index: 44 B per particle, plus the cell counts scanned into the bins
 STAGES = ["sort", "p2g", "grid", "g2p"]
-ALG_PER_PARTICLE = {"sort": 36, "p2g": 104, "grid": 0, "g2p": 152}
+ALG_PER_PARTICLE = {"sort": 44, "p2g": 104, "grid": 0, "g2p": 152}
 ALG_PER_NODE = {"sort": 0, "p2g": 16, "grid": 40, "g2p": 24}
 SUBSTEP_PER_PARTICLE, SUBSTEP_PER_NODE = 208, 56
 P2G_LAYER_NAME = "k_p2g_layer<2, P2G_MOM_STRESS>"  # the autotuner's other P2G schedule
 KERNEL_NAMES = {"p2g": "k_p2g<2, P2G_MOM_STRESS>", "g2p": "k_g2p<2>", "grid": "k_grid<GRID_FUSED>",
-                "sort": "k_cell_count + k_cell_scan + k_cell_scatter + k_cell_rank + k_claim",
+                "sort": "k_sums_claim + k_cell_scan + k_cell_scatter + k_cell_rank",
                 "surrogate": "k_surrogate"}
 # flops of one network evaluation: 2 x (5x128 + 3 x 128x128 + 128x3) multiply-adds
 MLP_FLOPS = 2 * (5 * 128 + 3 * 128 * 128 + 128 * 3)

@@ -334,7 +334,7 @@ int mpm_surrogate_gradient(mpm_ctx* ctx, const float* in, const float* H, int32_
  * (mpm_surrogate_nparam() floats) and loss (1 float, the mean loss) are DEVICE pointers. The call
  * only enqueues kernels on the context's stream (results are ready after mpm_synchronize) and
  * allocates nothing: its intermediates live in one fixed library-owned device array of about
- * 9.3 MB per GPU, which keeps the last call's contents. n must be in [1, 2048] (MPM_ERR_INVALID
+ * 11.4 MB per GPU, which keeps the last call's contents. n must be in [1, 2048] (MPM_ERR_INVALID
  * otherwise). Calls that overlap on one GPU (from different contexts or threads) race on that
  * array. Results equal mpm_surrogate_gradient's bit for bit. */
 int mpm_surrogate_gradient_noalloc(mpm_ctx* ctx, const float* in, const float* H, int32_t n, float* grad, float* loss);
